@@ -944,7 +944,7 @@ int launch_spectrum_t(gctf_ctx* c, const TileGrid& g, const TileTables& tt, cons
 		c->rt.as<float2>(), rts));
 	constexpr int CPW = 4;
 	const float fac = 1.0f / (float)ntiles;                   // CGenAvgSpectrum.cpp:90
-	PROF(c, "k_tile_cols", k_tile_cols<T, CPW><<<dim3((CX + CPW - 1) / CPW, nsplit, n), CPW * (T / 8), 0, s>>>(
+	PROF(c, "k_tile_cols", k_tile_cols<T, CPW><<<dim3(tile_col_groups(CX, CPW), nsplit, n), CPW * (T / 8), 0, s>>>(
 		c->rt.as<float2>(), rts, ntiles, nsplit, fac, tt.tw.as<float2>(), c->tpart.as<float>()));
 	const int npix = T * CX;
 	PROF(c, "k_tile_reduce", k_tile_reduce<<<dim3((npix + 255) / 256, n), 256, 0, s>>>(c->tpart.as<float>(), nsplit, npix,
@@ -2676,7 +2676,7 @@ int launch_tile_list_t(gctf_ctx* c, const TileTables& tt, const TileJob* d_jobs,
 {
 	hipStream_t s = c->stream;
 	constexpr int CX = T / 2 + 1, ROWS = 16, RG = 2, CPW = 4;
-	constexpr int NCG = (CX + CPW - 1) / CPW;
+	constexpr int NCG = tile_col_groups(CX, CPW);
 	const TileJob* jobs = d_jobs + G.j0;
 	if (G.max_nr > 0)
 		PROF(c, "k_row_sums", k_row_sums_list<Tin><<<dim3(G.max_nr, G.nj), 256, 0, s>>>(jobs, c->rowsum.as<float>()));

@@ -167,14 +167,15 @@ __device__ __forceinline__ void twiddle_powers(float2* u, float2 w)
 }
 
 // Synchronisation of the NT threads that share one transform.  A transform
-// of 64 threads belongs to a single wavefront: its LDS accesses execute in
-// issue order, so a wavefront-scope fence (which keeps the compiler from
-// moving LDS accesses across it and waits for the outstanding ones) replaces
-// the workgroup barrier, and the other transforms of the workgroup run on.
+// of at most 64 threads belongs to a single wavefront: its LDS accesses
+// execute in issue order, so a wavefront-scope fence (which keeps the
+// compiler from moving LDS accesses across it and waits for the outstanding
+// ones) replaces the workgroup barrier, and the other transforms of the
+// workgroup run on.
 template <int NT>
 __device__ __forceinline__ void fft_sync()
 {
-	if constexpr (NT == 64) {
+	if constexpr (NT <= 64) {
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -293,6 +294,52 @@ __device__ __forceinline__ void fft_run(float2* buf, const TW& twf, int tid)
 		fft_pass<N, R, L, P, NT, INV>(buf, twf, tid);
 		fft_run<N, L * R, P + 1, NT, INV>(buf, twf, tid);
 	}
+}
+
+// The transform of N = 8 NT elements from registers to registers: thread tid
+// holds elements x[i] = input tid + i NT and gets x[i] = output tid + i NT.
+// Those are exactly the inputs of its first (radix-8) butterfly and the
+// outputs of its last ones, so a transform makes one LDS round trip per pass
+// boundary (two for 512 points) instead of one more at either end.  Same
+// arithmetic as fft_lds.  buf may still be read by the NT threads' previous
+// transform; its contents afterwards are not defined, and it may be reused
+// after an fft_sync.
+template <int N, int L, int P, int NT, bool INV, class TW>
+__device__ __forceinline__ void fft_regs_run(float2* buf, const TW& twf, int tid, float2 (&x)[N / NT])
+{
+	constexpr int rem = N / L;
+	constexpr int R = rem >= 8 ? 8 : rem;
+	if constexpr (L * R < N) {
+		fft_pass<N, R, L, P, NT, INV>(buf, twf, tid);
+		fft_regs_run<N, L * R, P + 1, NT, INV>(buf, twf, tid, x);
+	} else {
+		constexpr int T = N / R, BPT = T / NT;
+#pragma unroll
+		for (int b = 0; b < BPT; ++b) {
+			const int j = tid + b * NT;
+			float2 u[R];
+#pragma unroll
+			for (int r = 0; r < R; ++r) u[r] = buf[pidx(j + r * T)];
+			float2 w = twf.template get<N, R, L, P>(b, j);
+			if (INV) w.y = -w.y;
+			twiddle_powers<R>(u, w);
+			dft_small<R, INV>(u);
+#pragma unroll
+			for (int r = 0; r < R; ++r) x[b + BPT * r] = u[r];
+		}
+	}
+}
+
+template <int N, int NT, bool INV, class TW>
+__device__ __forceinline__ void fft_regs(float2* buf, const TW& twf, int tid, float2 (&x)[N / NT])
+{
+	static_assert(N == 8 * NT && N > 64, "one radix-8 butterfly per thread, and a pass after it");
+	dft_small<8, INV>(x);
+	fft_sync<NT>();
+#pragma unroll
+	for (int r = 0; r < 8; ++r) buf[pidx(8 * tid + r)] = x[r];
+	fft_sync<NT>();
+	fft_regs_run<N, 8, 1, NT, INV>(buf, twf, tid, x);
 }
 
 // In-place power-of-two FFT of the N logical elements of buf (padded

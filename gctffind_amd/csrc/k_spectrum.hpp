@@ -659,12 +659,11 @@ __device__ __forceinline__ void tile_rows_body(const Tin* __restrict__ im, int p
 	constexpr int CX = T / 2 + 1;
 	constexpr int FL = fft_lds_len(T);
 	constexpr int PX = T / FT;             // pixels per thread and row
-	constexpr int KP = (CX + FT - 1) / FT; // half-spectrum entries per thread
-	constexpr int SP = ROWS + 1;           // stage pitch: lanes of a wave write
+	constexpr int SP = NG + 1;             // stage pitch: lanes of a wave write
 	                                       // k-consecutive entries, an odd pitch
 	                                       // keeps them off one LDS bank
 	constexpr int NRB = T / ROWS;          // row blocks per tile
-	static_assert(CX * SP <= NG * FL, "stage must fit in the transform buffers");
+	static_assert(T * SP <= NG * FL, "stage must fit in the transform buffers");
 	__shared__ float2 buf[NG * FL];
 	float2* stage = buf;
 	const int nblk = g.ntx * g.nty * NRB;
@@ -713,41 +712,26 @@ __device__ __forceinline__ void tile_rows_body(const Tin* __restrict__ im, int p
 			tsum = block_sum(bs, ty * g.nbx + tx);
 		}
 		const float mean = tsum / ((float)T * (float)T);
+		float2 z[PX];
 #pragma unroll
-		for (int i = 0; i < PX; ++i) {
-			const int x = lane + i * FT;
-			fb[pidx(x)] = make_float2((va[i] - mean) * ma[i], (vb[i] - mean) * mb[i]);
-		}
-		fft_sync<FT>();
+		for (int i = 0; i < PX; ++i) z[i] = make_float2((va[i] - mean) * ma[i], (vb[i] - mean) * mb[i]);
 		TwRegs<T, FT> twr;
 		fft_tw_load(twr, tw, lane);
 		if (it + 1 < G) load_rows(nb);
-		fft_lds<T, FT, false>(fb, twr, lane);
-		float2 sa[KP], sb[KP];
-#pragma unroll
-		for (int i = 0; i < KP; ++i) {
-			const int k = lane + i * FT;
-			if (k < CX) {
-				float2 z = fb[pidx(k)];
-				float2 zc = fb[pidx((T - k) & (T - 1))];
-				sa[i] = make_float2(0.5f * (z.x + zc.x), 0.5f * (z.y - zc.y));
-				sb[i] = make_float2(0.5f * (z.y + zc.y), -0.5f * (z.x - zc.x));
-			}
-		}
+		fft_regs<T, FT, false>(fb, twr, lane, z);
 		__syncthreads();
 #pragma unroll
-		for (int i = 0; i < KP; ++i) {
-			const int k = lane + i * FT;
-			if (k < CX) {
-				stage[k * SP + 2 * grp] = sa[i];
-				stage[k * SP + 2 * grp + 1] = sb[i];
-			}
-		}
+		for (int i = 0; i < PX; ++i) stage[(lane + i * FT) * SP + grp] = z[i];
 		__syncthreads();
+		// Rows 2q and 2q + 1 of the block are (Z[k] + conj Z[T-k]) / 2 and
+		// -i (Z[k] - conj Z[T-k]) / 2 of transform q: neighbours in the
+		// transposed output, one 16-byte store
 		float2* dst = rt + (long long)t * CX * T + rb * ROWS;
-		for (int i = threadIdx.x; i < CX * ROWS; i += NT) {
-			int k = i / ROWS, yy = i % ROWS;
-			dst[(long long)k * T + yy] = stage[k * SP + yy];
+		for (int i = threadIdx.x; i < CX * NG; i += NT) {
+			const int k = i / NG, q = i % NG;
+			const float2 zk = stage[k * SP + q], zc = stage[((T - k) & (T - 1)) * SP + q];
+			*reinterpret_cast<float4*>(dst + (long long)k * T + 2 * q) =
+				make_float4(0.5f * (zk.x + zc.x), 0.5f * (zk.y - zc.y), 0.5f * (zk.y + zc.y), -0.5f * (zk.x - zc.x));
 		}
 		if (it + 1 < G) load_mask(nb);
 		// the stage is the transforms' buffer: read out before it is refilled
@@ -812,7 +796,7 @@ __device__ __forceinline__ void tile_cols_body(const float2* __restrict__ src, i
 {
 	constexpr int FT = T / 8;
 	constexpr int CX = T / 2 + 1;
-	constexpr int PER = T / FT;            // 8 outputs per thread
+	constexpr int PER = T / FT;            // 8 inputs and outputs per thread
 	constexpr int FL = fft_lds_len(T);
 	__shared__ float2 buf[CPW * FL];
 	const int grp = threadIdx.x / FT, lane = threadIdx.x % FT;
@@ -826,19 +810,16 @@ __device__ __forceinline__ void tile_cols_body(const float2* __restrict__ src, i
 	float2* fb = buf + grp * FL;
 	TwRegs<T, FT> twr;
 	fft_tw_load(twr, tw, lane);
-	for (int t = t0; t < t1; ++t) {
-		if (live) {
-			const float2* col = src + ((long long)t * CX + kx) * T;
-			for (int y = lane; y < T; y += FT) fb[pidx(y)] = col[y];
-		}
-		fft_sync<FT>();
-		fft_lds<T, FT, false>(fb, twr, lane);
+	// columns past the last (live false) run on the last one's data
+	const float2* col = src + ((long long)t0 * CX + min(kx, CX - 1)) * T + lane;
+	for (int t = t0; t < t1; ++t, col += (long long)CX * T) {
+		float2 z[PER];
 #pragma unroll
-		for (int i = 0; i < PER; ++i) {
-			float2 c = fb[pidx(lane + i * FT)];
-			acc[i] = fmaf(sqrtf(fmaf(c.x, c.x, c.y * c.y)), fac, acc[i]);
-		}
-		fft_sync<FT>();
+		for (int i = 0; i < PER; ++i) z[i] = col[i * FT];
+		fft_regs<T, FT, false>(fb, twr, lane, z);
+#pragma unroll
+		for (int i = 0; i < PER; ++i)
+			acc[i] = fmaf(__builtin_amdgcn_sqrtf(fmaf(z[i].x, z[i].x, z[i].y * z[i].y)), fac, acc[i]);
 	}
 	if (!live) return;
 	float* dst = part + (long long)s * T * CX;
@@ -850,26 +831,33 @@ __device__ __forceinline__ void tile_cols_body(const float2* __restrict__ src, i
 	}
 }
 
+// Column group of workgroup bx of a padded grid of tile_col_groups(CX, CPW).
+__host__ __device__ constexpr int tile_col_groups(int cx, int cpw) { return ((cx + cpw - 1) / cpw + 7) / 8 * 8; }
+
 template <int T, int CPW>
 __global__ __launch_bounds__(CPW * (T / 8)) void k_tile_cols(const float2* __restrict__ rt,
 	long long rt_stride, int ntiles, int nsplit, float fac, const float2* __restrict__ tw,
 	float* __restrict__ part)
 {
 	constexpr int CX = T / 2 + 1;
+	const int cg = xcd_group(blockIdx.x, (CX + CPW - 1) / CPW);
+	if (cg < 0) return;
 	tile_cols_body<T, CPW>(rt + blockIdx.z * rt_stride, ntiles, nsplit, fac, tw,
-		part + (long long)blockIdx.z * nsplit * T * CX, blockIdx.x, blockIdx.y);
+		part + (long long)blockIdx.z * nsplit * T * CX, cg, blockIdx.y);
 }
 
-// The same over a tile work list: grid (ceil(CX/CPW), largest nsplit, jobs).
+// The same over a tile work list: grid (tile_col_groups, largest nsplit, jobs).
 template <int T, int CPW>
 __global__ __launch_bounds__(CPW * (T / 8)) void k_tile_cols_list(const TileJob* __restrict__ jobs,
 	const float2* __restrict__ rt, const float2* __restrict__ tw, float* __restrict__ part)
 {
+	constexpr int CX = T / 2 + 1;
 	const TileJob& J = jobs[blockIdx.z];
-	if ((int)blockIdx.y >= J.nsplit) return;
+	const int cg = xcd_group(blockIdx.x, (CX + CPW - 1) / CPW);
+	if (cg < 0 || (int)blockIdx.y >= J.nsplit) return;
 	const int ntiles = J.g.ntx * J.g.nty;
-	tile_cols_body<T, CPW>(rt + J.rt_off, ntiles, J.nsplit, 1.0f / (float)ntiles, tw, part + J.part_off,
-		blockIdx.x, blockIdx.y);
+	tile_cols_body<T, CPW>(rt + J.rt_off, ntiles, J.nsplit, 1.0f / (float)ntiles, tw, part + J.part_off, cg,
+		blockIdx.y);
 }
 
 // Zero the work-queue counters of a list's persistent launches.
