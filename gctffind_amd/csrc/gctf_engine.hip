@@ -10,7 +10,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <complex>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -68,47 +67,77 @@ int next_pow2(int n)
 	return m;
 }
 
-void host_fft(std::vector<std::complex<double>>& a, bool inv)
-{
-	const int n = (int)a.size();
-	for (int i = 1, j = 0; i < n; i++) {
-		int bit = n >> 1;
-		for (; j & bit; bit >>= 1) j ^= bit;
-		j ^= bit;
-		if (i < j) std::swap(a[i], a[j]);
+// The interpolation kernel of a length-n transform on m fine points: the
+// Kaiser-Bessel window of 8 points, I0(beta sqrt(1 - (d/4)^2)) / I0(beta) at
+// distance d, and its Fourier transform.  beta is 0.985 of Kaiser's
+// pi w (1 - n/(2 m)): least aliasing over n/m in [1/4, 1/2].
+struct ItpKernel {
+	double beta, top;
+	int m;
+	ItpKernel(int n, int m_) : m(m_)
+	{
+		beta = 0.985 * M_PI * 8.0 * (1.0 - 0.5 * (double)n / (double)m_);
+		top = 1.0;
+		double t = 0.0;
+		at(&t, 1);
+		top = t;
 	}
-	for (int len = 2; len <= n; len <<= 1) {
-		for (int k = 0; k < len / 2; k++) {
-			double ang = (inv ? 2.0 : -2.0) * M_PI * k / len;
-			std::complex<double> w(cos(ang), sin(ang));
-			for (int i = k; i < n; i += len) {
-				std::complex<double> u = a[i], v = a[i + len / 2] * w;
-				a[i] = u + v;
-				a[i + len / 2] = u - v;
+	// d[0..cnt) -> the window at those distances.  I0(x) by its power series
+	// in q = (x/2)^2, 40 terms (x <= 24.8, where they reach 1e-15 of the sum):
+	// a fixed count over many distances, which the compiler vectorises; plans
+	// are made on a shape's first call, tens of thousands of values each
+	void at(double* d, int cnt) const
+	{
+		static const struct Coef {
+			double c[40];
+			Coef()
+			{
+				c[0] = 1.0;
+				for (int k = 1; k < 40; ++k) c[k] = c[k - 1] / ((double)k * k);
 			}
+		} co;
+		for (int i = 0; i < cnt; i += 8) {
+			const int e = std::min(8, cnt - i);
+			double q[8] = {0, 0, 0, 0, 0, 0, 0, 0}, s[8];
+			bool in[8] = {false, false, false, false, false, false, false, false};
+			for (int j = 0; j < e; ++j) {
+				const double u = 1.0 - d[i + j] * d[i + j] / 16.0;
+				in[j] = u > 0.0;
+				q[j] = in[j] ? 0.25 * beta * beta * u : 0.0;
+			}
+			for (int j = 0; j < 8; ++j) s[j] = co.c[39];
+			for (int k = 38; k >= 0; --k)
+				for (int j = 0; j < 8; ++j) s[j] = s[j] * q[j] + co.c[k];
+			for (int j = 0; j < e; ++j) d[i + j] = in[j] ? s[j] / top : 0.0;
 		}
 	}
-}
+	double hat(int k) const
+	{
+		const double w = M_PI * 8.0 * (double)k / (double)m, q = beta * beta - w * w;
+		if (q > 0.0) return 8.0 * sinh(sqrt(q)) / sqrt(q) / top;
+		return q == 0.0 ? 8.0 / top : 8.0 * sin(sqrt(-q)) / sqrt(-q) / top;
+	}
+};
 
 // Device tables of one transform length.
 struct FftDev {
 	int n = 0, m = 0;
-	std::vector<unsigned char> rad;   // mixed-radix passes (empty: power of two or Bluestein)
-	DevBuf tw, chirp, bhat;
-	DevBuf sub_chirp, sub_bhat, sub_tw, ct_tw;   // radix-4 step over quarter-length Bluestein transforms
+	std::vector<unsigned char> rad;   // mixed-radix passes (empty: power of two or fine grid)
+	DevBuf tab;                       // all tables, each at its byte offset (0: none but tw)
+	size_t mode = 0, w8 = 0, p0 = 0, w4 = 0, q0 = 0;
 	Fft1dPlan plan() const
 	{
 		Fft1dPlan p{};
 		p.n = n; p.m = m;
-		p.tw = tw.as<float2>();
-		p.chirp = chirp.p ? chirp.as<float2>() : nullptr;
-		p.bhat = bhat.p ? bhat.as<float2>() : nullptr;
+		char* t = tab.as<char>();
+		p.tw = (const float2*)t;
 		p.nrad = (int)rad.size();
 		for (size_t i = 0; i < rad.size(); ++i) p.rad[i] = rad[i];
-		p.sub_chirp = sub_chirp.p ? sub_chirp.as<float2>() : nullptr;
-		p.sub_bhat = sub_bhat.p ? sub_bhat.as<float2>() : nullptr;
-		p.sub_tw = sub_tw.p ? sub_tw.as<float2>() : nullptr;
-		p.ct_tw = ct_tw.p ? ct_tw.as<float2>() : nullptr;
+		p.mode = mode ? (const float2*)(t + mode) : nullptr;
+		p.w8 = w8 ? (const float4*)(t + w8) : nullptr;
+		p.p0 = p0 ? (const int*)(t + p0) : nullptr;
+		p.w4 = w4 ? (const float4*)(t + w4) : nullptr;
+		p.q0 = q0 ? (const int*)(t + q0) : nullptr;
 		return p;
 	}
 };
@@ -123,8 +152,8 @@ bool smooth235(int n)
 	return n == 1;
 }
 
-// The length a transform of length n works on in LDS: n itself for powers
-// of two and 2^a 3^b 5^c (Stockham passes), else the Bluestein length.
+// The length a transform of length n needs in LDS: n itself for powers of two
+// and 2^a 3^b 5^c (Stockham passes), else the fine grid's, at least 2 n - 1.
 int work_len(int n) { return is_pow2(n) || smooth235(n) ? n : next_pow2(2 * n - 1); }
 
 // Pass radices of a 2^a 3^b 5^c length: radix 8 while 8 divides what is
@@ -169,13 +198,12 @@ struct RescalePlan {
 	bool active = false;
 	// rows_half / c2r_half: the R2C / C2R row transforms run at half length
 	// (even/odd samples packed into one complex row); rows / c2r are then the
-	// half-length plans and rows_maxn / c2r_maxn the kernels' transform
-	// lengths (8192 or 16384)
+	// half-length plans.  rows_maxn / c2r_maxn: the kernels' LDS points
 	bool rows_half = false, c2r_half = false;
 	int rows_maxn = 16384, c2r_maxn = 16384;
 	// cols_split: the column pass's forward transform runs as the transforms
-	// of the even and odd samples; cf is then the half-length plan and
-	// cols_maxn the kernel's transform length (8192 or 16384)
+	// of the even and odd samples; cf is then the half-length plan.
+	// cols_maxn: the kernel's LDS points
 	bool cols_split = false;
 	int cols_maxn = 16384;
 	FftDev *rows = nullptr, *cf = nullptr, *ci = nullptr, *c2r = nullptr;
@@ -271,7 +299,7 @@ struct gctf_ctx {
 	float scan_lo = 0, scan_hi = 0, scan_step = 0;  // Do1D scan (gctf_set_search1d; 0: reference)
 	int gen = 0;  // bumped whenever a device buffer moves
 
-	std::map<int, std::unique_ptr<FftDev>> ffts;
+	std::map<std::pair<int, int>, std::unique_ptr<FftDev>> ffts;   // by length and fine-grid points (< 0: inverse)
 	std::map<int, std::unique_ptr<TileTables>> tiles;
 	std::map<std::string, std::unique_ptr<SearchPlan>> splans;
 	std::map<std::string, GraphEntry> graphs;
@@ -394,71 +422,98 @@ int ensure_buf(gctf_ctx* c, DevBuf& b, size_t bytes)
 	return GCTF_OK;
 }
 
-int get_fft(gctf_ctx* c, int n, FftDev** out)
+// LDS points of the kernel class a working length falls in.
+int pow2_class(int m) { return m <= 2048 ? 2048 : m <= 4096 ? 4096 : m <= 8192 ? 8192 : 16384; }
+
+// The plan of length n in kernels of maxn LDS points (the fine grid of a
+// length without Stockham passes is the kernel's maxn points), with the
+// tables of the inverse or the forward transform.
+int get_fft(gctf_ctx* c, int n, int maxn, bool inv, FftDev** out)
 {
-	auto it = c->ffts.find(n);
+	const bool grid = !is_pow2(n) && !smooth235(n);
+	const std::pair<int, int> key(n, grid ? (inv ? -maxn : maxn) : 0);
+	auto it = c->ffts.find(key);
 	if (it != c->ffts.end()) { *out = it->second.get(); return GCTF_OK; }
+	if (work_len(n) > 16384)
+		return fail(c, GCTF_ERR_UNSUPPORTED, "transform length " + std::to_string(n)
+			+ " needs a working length above 16384");
+	if (work_len(n) > maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "transform length " + std::to_string(n));
 	auto f = std::make_unique<FftDev>();
 	f->n = n;
-	f->m = work_len(n);
-	if (!is_pow2(n) && smooth235(n)) {
+	f->m = grid ? maxn : n;
+	if (!grid && !is_pow2(n)) {
 		f->rad = mixed_radices(n);
 		if (f->rad.size() > sizeof(Fft1dPlan{}.rad)) return fail(c, GCTF_ERR_UNSUPPORTED, "transform length");
 	}
-	const int m = f->m;
-	if (m > 16384)
-		return fail(c, GCTF_ERR_UNSUPPORTED, "transform length " + std::to_string(n)
-			+ " needs a working length above 16384");
-	std::vector<float2> tw(m);
-	for (int e = 0; e < m; ++e) {
-		double a = -2.0 * M_PI * (double)e / (double)m;
+	const int m = f->m, P = m / 2, nt = grid ? P : m;
+	const int S = n % 2 == 0 ? 2 : 1, kmax = n / 2;
+	// one buffer, every table on a 256-byte boundary
+	size_t bytes = 0;
+	auto place = [&](size_t b) { const size_t o = bytes; bytes = (bytes + b + 255) / 256 * 256; return o; };
+	place(sizeof(float2) * nt);
+	if (grid) {
+		f->mode = place(sizeof(float2) * 2 * (kmax + 1));
+		if (inv) {
+			f->w8 = place(sizeof(float4) * 2 * (n / S));
+			f->p0 = place(sizeof(int) * (n / S));
+		} else {
+			f->w4 = place(sizeof(float4) * 2 * (P / S));
+			f->q0 = place(sizeof(int) * 2 * (P / S));
+		}
+	}
+	std::vector<char> host(bytes);
+	float2* tw = (float2*)host.data();
+	for (int e = 0; e < nt; ++e) {
+		double a = -2.0 * M_PI * (double)e / (double)nt;
 		tw[e] = make_float2((float)cos(a), (float)sin(a));
 	}
-	CHK(ensure_buf(c, f->tw, sizeof(float2) * m));
-	HIPCHK(c, hipMemcpy(f->tw.p, tw.data(), sizeof(float2) * m, hipMemcpyHostToDevice));
-	// Bluestein tables of length n on m points: chirp[k] = exp(-pi i (k^2 mod
-	// 2n) / n) and bhat = FFT_m of the wrapped conj(chirp)
-	auto bluestein_tables = [&](int len, int work, DevBuf& dchirp, DevBuf& dbhat) -> int {
-		std::vector<std::complex<double>> w(len), b(work, 0.0);
-		std::vector<float2> chirp(len), bhat(work);
-		for (int k = 0; k < len; ++k) {
-			long long k2 = ((long long)k * k) % (2LL * len);
-			double a = -M_PI * (double)k2 / (double)len;
-			w[k] = std::complex<double>(cos(a), sin(a));
-			chirp[k] = make_float2((float)w[k].real(), (float)w[k].imag());
+	if (grid) {
+		const ItpKernel ker(n, m);
+		float2* mode = (float2*)(host.data() + f->mode);
+		for (int k = 0; k <= kmax; ++k) {
+			const double d = 1.0 / ker.hat(k), a = M_PI * (double)k / (double)P;
+			mode[k] = make_float2((float)d, 0.0f);
+			mode[kmax + 1 + k] = make_float2((float)(d * cos(a)), (float)(d * sin(a)));
 		}
-		b[0] = std::conj(w[0]);
-		for (int k = 1; k < len; ++k) { b[k] = std::conj(w[k]); b[work - k] = b[k]; }
-		host_fft(b, false);
-		for (int k = 0; k < work; ++k) bhat[k] = make_float2((float)b[k].real(), (float)b[k].imag());
-		CHK(ensure_buf(c, dchirp, sizeof(float2) * len));
-		CHK(ensure_buf(c, dbhat, sizeof(float2) * work));
-		HIPCHK(c, hipMemcpy(dchirp.p, chirp.data(), sizeof(float2) * len, hipMemcpyHostToDevice));
-		HIPCHK(c, hipMemcpy(dbhat.p, bhat.data(), sizeof(float2) * work, hipMemcpyHostToDevice));
-		return GCTF_OK;
-	};
-	auto twiddles = [&](int len, DevBuf& d) -> int {
-		std::vector<float2> t(len);
-		for (int e = 0; e < len; ++e) {
-			double a = -2.0 * M_PI * (double)e / (double)len;
-			t[e] = make_float2((float)cos(a), (float)sin(a));
-		}
-		CHK(ensure_buf(c, d, sizeof(float2) * len));
-		HIPCHK(c, hipMemcpy(d.p, t.data(), sizeof(float2) * len, hipMemcpyHostToDevice));
-		return GCTF_OK;
-	};
-	if (!is_pow2(n) && f->rad.empty()) {
-		CHK(bluestein_tables(n, m, f->chirp, f->bhat));
-		// n = 4 q whose quarter has Bluestein length m / 4: also the tables
-		// of one radix-4 step over four q-point Bluestein transforms
-		if (n % 4 == 0 && next_pow2(2 * (n / 4) - 1) == m / 4) {
-			CHK(bluestein_tables(n / 4, m / 4, f->sub_chirp, f->sub_bhat));
-			CHK(twiddles(m / 4, f->sub_tw));
-			CHK(twiddles(n, f->ct_tw));
+		if (inv) {
+			// output t lies at t m / n; its points are the 4 at or below it and
+			// the 4 above
+			float4* w8 = (float4*)(host.data() + f->w8);
+			int* p0 = (int*)(host.data() + f->p0);
+			for (int t = 0; t < n / S; ++t) {
+				const long long fl = (long long)t * m / n;
+				const double x = (double)((long long)t * m - fl * n) / (double)n;   // in [0, 1)
+				p0[t] = (int)fl - 3;
+				double w[8];
+				for (int j = 0; j < 8; ++j) w[j] = x + 3.0 - j;
+				ker.at(w, 8);
+				w8[2 * t] = make_float4((float)w[0], (float)w[1], (float)w[2], (float)w[3]);
+				w8[2 * t + 1] = make_float4((float)w[4], (float)w[5], (float)w[6], (float)w[7]);
+			}
+		} else {
+			// fine point l = 2 i + b takes the inputs j with |l - j m / n| < 4:
+			// at most 4 as m >= 2 n
+			float4* w4 = (float4*)(host.data() + f->w4);
+			int* q0 = (int*)(host.data() + f->q0);
+			for (int e = 0; e < 2 * (P / S); e += 2) {
+				double w[8];
+				for (int h = 0; h < 2; ++h) {
+					const int b = (e + h) / (P / S), l = 2 * ((e + h) % (P / S)) + b;
+					const long long num = (long long)(l - 4) * n;
+					const int q = (int)(num >= 0 ? num / m : -((-num + m - 1) / m)) + 1;   // floor + 1
+					q0[e + h] = q;
+					for (int j = 0; j < 4; ++j) w[4 * h + j] = (double)((long long)l * n - (long long)(q + j) * m) / n;
+				}
+				ker.at(w, 8);
+				for (int h = 0; h < 2; ++h)
+					w4[e + h] = make_float4((float)w[4 * h], (float)w[4 * h + 1], (float)w[4 * h + 2], (float)w[4 * h + 3]);
+			}
 		}
 	}
+	CHK(ensure_buf(c, f->tab, bytes));
+	HIPCHK(c, hipMemcpy(f->tab.p, host.data(), bytes, hipMemcpyHostToDevice));
 	*out = f.get();
-	c->ffts[n] = std::move(f);
+	c->ffts[key] = std::move(f);
 	return GCTF_OK;
 }
 
@@ -708,10 +763,13 @@ int make_rescale_plan(gctf_ctx* c, int nx, int ny, float pix, RescalePlan& rp)
 			rp.cols_split = true;
 			rp.cols_maxn = 8192;
 		}
-		CHK(get_fft(c, rp.rows_half ? nx / 2 : nx, &rp.rows));
-		CHK(get_fft(c, rp.cols_split ? ny / 2 : ny, &rp.cf));
-		CHK(get_fft(c, rp.nny, &rp.ci));
-		CHK(get_fft(c, rp.c2r_half ? rp.nnx / 2 : rp.nnx, &rp.c2r));
+		if (!rp.rows_half) rp.rows_maxn = pow2_class(work_len(nx));
+		if (!rp.cols_split) rp.cols_maxn = pow2_class(std::max(work_len(ny), work_len(rp.nny)));
+		if (!rp.c2r_half) rp.c2r_maxn = pow2_class(work_len(rp.nnx));
+		CHK(get_fft(c, rp.rows_half ? nx / 2 : nx, rp.rows_maxn, false, &rp.rows));
+		CHK(get_fft(c, rp.cols_split ? ny / 2 : ny, rp.cols_maxn, false, &rp.cf));
+		CHK(get_fft(c, rp.nny, rp.cols_maxn, true, &rp.ci));
+		CHK(get_fft(c, rp.c2r_half ? rp.nnx / 2 : rp.nnx, rp.c2r_maxn, true, &rp.c2r));
 	}
 	return GCTF_OK;
 }
@@ -821,12 +879,11 @@ int launch_rescale_t(gctf_ctx* c, const RescalePlan& rp, const Tin* in, long lon
 	const long long stA = (long long)cbuf_elems(rp), stB = stA;
 	// 1. rows R2C with x crop into A: A[y][kx], rows spec_ld(ncx) apart
 	{
-		const int m = rp.rows->m;
+		const int m = rp.rows_maxn;
 		dim3 grid((rp.ny + 1) / 2, n);
 		Fft1dPlan p = rp.rows->plan();
 		if (rp.rows_half) {
-			if (m > rp.rows_maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "row length");
-			if (rp.rows_maxn == 8192)
+			if (m == 8192)
 				PROF(c, "k_rescale_rows_r2c_half", k_rescale_rows_r2c_half<Tin, 1024, 8192><<<dim3(rp.ny, n), 1024,
 					0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA));
 			else
@@ -845,12 +902,11 @@ int launch_rescale_t(gctf_ctx* c, const RescalePlan& rp, const Tin* in, long lon
 	}
 	// 2. columns: forward ny, crop, inverse nny, written row-major into A: A[y'][kx]
 	{
-		const int m = std::max(rp.cf->m, rp.ci->m);
+		const int m = rp.cols_maxn;
 		dim3 grid(8 * ((ncx + 7) / 8), n);
 		Fft1dPlan pf = rp.cf->plan(), pi = rp.ci->plan();
 		if (rp.cols_split) {
-			if (m > rp.cols_maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "column length");
-			if (rp.cols_maxn == 8192)
+			if (m == 8192)
 				PROF(c, "k_rescale_cols_split", k_rescale_cols_split<1024, 8192><<<grid, 1024, 0, s>>>(B, stB, rp.ny,
 					rp.nny, ncx, pf, pi, A, stA));
 			else
@@ -864,14 +920,13 @@ int launch_rescale_t(gctf_ctx* c, const RescalePlan& rp, const Tin* in, long lon
 	}
 	// 3. rows C2R into the padded image
 	{
-		const int m = rp.c2r->m;
+		const int m = rp.c2r_maxn;
 		dim3 grid((rp.nny + 1) / 2, n);
 		Fft1dPlan p = rp.c2r->plan();
 		const TileGrid g = tg ? *tg : TileGrid{};
 		float* rs = tg ? (rowsum_out ? rowsum_out : c->rowsum.as<float>()) : nullptr;
 		if (rp.c2r_half) {
-			if (m > rp.c2r_maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "row length");
-			if (rp.c2r_maxn == 8192)
+			if (m == 8192)
 				PROF(c, "k_rescale_rows_c2r_half", k_rescale_rows_c2r_half<1024, 8192><<<dim3(rp.nny, n), 1024, 0,
 					s>>>(A, stA, rp.nny, rp.nnx, p, out, out_stride, rp.pitch, g, rs));
 			else
@@ -2579,26 +2634,20 @@ struct RsClass {
 	size_t first_off = 0, job_off = 0;               // offsets into the uploaded int table
 };
 
-int pow2_class(int m) { return m <= 2048 ? 2048 : m <= 4096 ? 4096 : m <= 8192 ? 8192 : 16384; }
-
 // Class keys and workgroup items of the four stages of one micrograph.
 int rescale_classes(gctf_ctx* c, const RescalePlan& rp, int f16, int key[4][3], int items[4])
 {
 	const int ncx = rp.nnx / 2 + 1;
-	if (rp.rows_half && rp.rows->m > rp.rows_maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "row length");
-	if (rp.cols_split && std::max(rp.cf->m, rp.ci->m) > rp.cols_maxn)
-		return fail(c, GCTF_ERR_UNSUPPORTED, "column length");
-	if (rp.c2r_half && rp.c2r->m > rp.c2r_maxn) return fail(c, GCTF_ERR_UNSUPPORTED, "row length");
-	key[RS_R2C][0] = rp.rows_half; key[RS_R2C][1] = rp.rows_half ? rp.rows_maxn : pow2_class(rp.rows->m);
+	key[RS_R2C][0] = rp.rows_half; key[RS_R2C][1] = rp.rows_maxn;
 	key[RS_R2C][2] = f16;
 	items[RS_R2C] = rp.rows_half ? rp.ny : (rp.ny + 1) / 2;
 	key[RS_TRANSPOSE][0] = 0; key[RS_TRANSPOSE][1] = 0; key[RS_TRANSPOSE][2] = 0;
 	items[RS_TRANSPOSE] = ((ncx + 31) / 32) * ((rp.ny + 31) / 32);
 	key[RS_COLS][0] = rp.cols_split;
-	key[RS_COLS][1] = rp.cols_split ? rp.cols_maxn : pow2_class(std::max(rp.cf->m, rp.ci->m));
+	key[RS_COLS][1] = rp.cols_maxn;
 	key[RS_COLS][2] = 0;
 	items[RS_COLS] = 8 * ((ncx + 7) / 8);                // a multiple of 8: xcd_group sees the XCD
-	key[RS_C2R][0] = rp.c2r_half; key[RS_C2R][1] = rp.c2r_half ? rp.c2r_maxn : pow2_class(rp.c2r->m);
+	key[RS_C2R][0] = rp.c2r_half; key[RS_C2R][1] = rp.c2r_maxn;
 	key[RS_C2R][2] = 0;
 	items[RS_C2R] = rp.c2r_half ? rp.nny : (rp.nny + 1) / 2;
 	return GCTF_OK;

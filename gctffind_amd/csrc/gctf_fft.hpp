@@ -5,8 +5,9 @@
 // separates the LDS reads of a pass from its writes, so one LDS buffer of N
 // complex values suffices.  Lengths 2^a 3^b 5^c run the same Stockham passes
 // with radix-3 and radix-5 butterflies added (fft_lds_mixed).  Other lengths
-// use Bluestein's chirp-z algorithm on a power-of-two length M >= 2n-1.  All
-// are unnormalised; the forward transform uses exp(-2 pi i k n / N).
+// run on a power-of-two grid at least twice as fine, reached by an eight-point
+// interpolation (itp_fwd, itp_inv).  All are unnormalised; the forward
+// transform uses exp(-2 pi i k n / N).
 //
 // LDS layout: logical element i lives at physical index pidx(i) = i + i/8.
 // The Stockham writes of the early passes stride by the radix (8 complex);
@@ -364,28 +365,23 @@ __device__ __forceinline__ void fft_lds(float2* buf, const TwRegs<N, NT>& w, int
 // ---- compile-time transform with input and output hooks -----------------
 // fft_lds_io runs the same passes as fft_lds, but the first pass takes its
 // inputs from ld(i) (logical input index i) instead of buf, and the last
-// pass stores st(i, v) at logical output index i.  ld may read buf: every
-// read of a pass precedes its writes.  Pointwise work before and after a
-// transform (chirps, filters, crops) then costs no LDS round trip and no
-// barrier of its own.
-//
-// ZIN: the inputs at i >= N/2 are zero (ld is not called for them).  DROP:
-// the outputs at i >= N/2 are not needed (not stored).  In the first pass
-// element r of a butterfly has index j + r N/R with j < N/R, and in the
-// last pass j + r L with j < L = N/R, so both halves are r >= R/2: known
-// at compile time.
+// pass hands its outputs to st(i, v) instead of storing v at buf[pidx(i)].
+// ld may read buf: every read of a pass precedes its writes.  st may write
+// anywhere in buf: the last pass's reads are over when it is called, and an
+// fft_sync follows.  Loading and pointwise work before and after a transform
+// then cost no LDS round trip and no barrier of their own.
 
-// The plain input: buf itself.
+// The plain input and output: buf itself.
 struct LdsIn {
 	const float2* buf;
 	__device__ __forceinline__ float2 operator()(int i) const { return buf[pidx(i)]; }
 };
-// The plain output: v unchanged.
-struct SameOut {
-	__device__ __forceinline__ float2 operator()(int, float2 v) const { return v; }
+struct LdsOut {
+	float2* buf;
+	__device__ __forceinline__ void operator()(int i, float2 v) const { buf[pidx(i)] = v; }
 };
 
-template <int N, int R, int L, int NT, bool INV, bool ZIN, bool DROP, class Ld, class St>
+template <int N, int R, int L, int NT, bool INV, class Ld, class St>
 __device__ __forceinline__ void fft_pass_io(float2* buf, const float2* __restrict__ tw, int tid,
 	const Ld& ld, const St& st)
 {
@@ -398,12 +394,8 @@ __device__ __forceinline__ void fft_pass_io(float2* buf, const float2* __restric
 		if (T % NT == 0 || j < T) {
 #pragma unroll
 			for (int r = 0; r < R; ++r) {
-				if constexpr (L == 1) {
-					if (ZIN && 2 * r >= R) u[b][r] = make_float2(0.f, 0.f);
-					else u[b][r] = ld(j + r * T);
-				} else {
-					u[b][r] = buf[pidx(j + r * T)];
-				}
+				if constexpr (L == 1) u[b][r] = ld(j + r * T);
+				else u[b][r] = buf[pidx(j + r * T)];
 			}
 			if constexpr (L > 1) {
 				const int k = j & (L - 1);
@@ -424,92 +416,34 @@ __device__ __forceinline__ void fft_pass_io(float2* buf, const float2* __restric
 			const int base = (j - k) * R + k;
 #pragma unroll
 			for (int r = 0; r < R; ++r) {
-				if constexpr (L * R == N) {
-					if (!(DROP && 2 * r >= R)) buf[pidx(base + r * L)] = st(base + r * L, u[b][r]);
-				} else {
-					buf[pidx(base + r * L)] = u[b][r];
-				}
+				if constexpr (L * R == N) st(base + r * L, u[b][r]);
+				else buf[pidx(base + r * L)] = u[b][r];
 			}
 		}
 	}
 	fft_sync<NT>();
 }
 
-template <int N, int L, int NT, bool INV, bool ZIN, bool DROP, class Ld, class St>
+template <int N, int L, int NT, bool INV, class Ld, class St>
 __device__ __forceinline__ void fft_run_io(float2* buf, const float2* __restrict__ tw, int tid,
 	const Ld& ld, const St& st)
 {
 	if constexpr (L < N) {
 		constexpr int rem = N / L;
 		constexpr int R = rem >= 8 ? 8 : rem;
-		fft_pass_io<N, R, L, NT, INV, ZIN, DROP>(buf, tw, tid, ld, st);
-		fft_run_io<N, L * R, NT, INV, ZIN, DROP>(buf, tw, tid, ld, st);
+		fft_pass_io<N, R, L, NT, INV>(buf, tw, tid, ld, st);
+		fft_run_io<N, L * R, NT, INV>(buf, tw, tid, ld, st);
 	}
 }
 
-// Same contract as fft_lds, except that the input need not be in buf: the
-// first pass reads ld(i).  N >= 16 (the first pass is not the last).
-template <int N, int NT, bool INV, bool ZIN = false, bool DROP = false, class Ld, class St>
+// Same contract as fft_lds, except that the first pass reads ld(i) and the
+// last pass writes through st.  N >= 16 (the first pass is not the last).
+template <int N, int NT, bool INV, class Ld, class St>
 __device__ __forceinline__ void fft_lds_io(float2* buf, const float2* __restrict__ tw, int tid,
 	const Ld& ld, const St& st)
 {
 	static_assert(N >= 16, "the first and last passes must differ");
-	fft_run_io<N, 1, NT, INV, ZIN, DROP>(buf, tw, tid, ld, st);
-}
-
-// Bluestein DFT of length n on the compile-time working length M
-// (M >= 2n-1), input element i < n given by src(i) (which may read buf),
-// result in logical buf[0..n).  The chirp multiply and zero padding run in
-// the forward transform's first pass, the filter multiply in its last pass
-// and the final chirp multiply and 1/M scale in the inverse's last pass;
-// the arithmetic is that of bluestein_lds.
-// opaque(i) is i, but the compiler may not reuse an address or comparison
-// computed from the same index passes earlier: keeping those live across a
-// whole transform costs more registers than recomputing them.
-__device__ __forceinline__ int opaque(int i)
-{
-	asm volatile("" : "+v"(i));
-	return i;
-}
-
-template <int NT, int M, bool INV, class Src>
-__device__ __forceinline__ void bluestein_io(float2* buf, int n, const float2* __restrict__ chirp,
-	const float2* __restrict__ bhat, const float2* __restrict__ twm, int tid, const Src& src)
-{
-	// The hooks are branch-free (clamped index, then a select): branches
-	// inside a pass split the live ranges of the addresses the passes share.
-	auto ld = [&](int i) -> float2 {
-		const int ic = min(i, n - 1);
-		float2 w = chirp[ic];
-		if (INV) w.y = -w.y;
-		const float2 v = cmul(src(ic), w);
-		return i < n ? v : make_float2(0.f, 0.f);
-	};
-	auto filt = [&](int k, float2 v) -> float2 {
-		k = opaque(k);
-		float2 b;
-		if (INV) {
-			b = bhat[(M - k) & (M - 1)];
-			b.y = -b.y;
-		} else {
-			b = bhat[k];
-		}
-		return cmul(v, b);
-	};
-	// n <= M/2: the chirped input is zero from M/2 on, and only the first n
-	// outputs of the inverse are kept
-	fft_lds_io<M, NT, false, true, false>(buf, twm, tid, ld, filt);
-	const float inv_m = 1.0f / (float)M;
-	auto fin = [&](int k, float2 v) -> float2 {
-		k = opaque(k);
-		const int kc = min(k, n - 1);
-		float2 w = chirp[kc];
-		if (INV) w.y = -w.y;
-		const float2 t = cmul(v, w);
-		return k < n ? make_float2(t.x * inv_m, t.y * inv_m) : v;
-	};
-	// the inverse recomputes its addresses rather than keeping the forward's
-	fft_lds_io<M, NT, true, false, true>(buf, twm, opaque(tid), LdsIn{buf}, fin);
+	fft_run_io<N, 1, NT, INV>(buf, tw, tid, ld, st);
 }
 
 // ---- runtime-length power-of-two FFT (lengths up to MAXN) ----------------
@@ -579,65 +513,20 @@ __device__ __forceinline__ void fft_lds_rt(float2* buf, int n, const float2* __r
 	}
 }
 
-// Bluestein DFT of length n held in logical buf[0..n); buf holds m logical
-// entries (m a power of two >= 2n-1).  chirp[k] = exp(-pi i (k^2 mod 2n) / n);
-// bhat = FFT_m of b[j] = conj(chirp[|j|]) (wrapped).  twm: the m-point
-// twiddle table.  The inverse uses conj(chirp) and
-// bhat_inv[j] = conj(bhat[(m-j) mod m]).
-template <int NT, int MAXN, bool INV>
-__device__ __forceinline__ void bluestein_lds(float2* buf, int n, int m, const float2* __restrict__ chirp,
-	const float2* __restrict__ bhat, const float2* __restrict__ twm, int tid)
-{
-	for (int k = tid; k < m; k += NT) {
-		if (k < n) {
-			float2 w = chirp[k];
-			if (INV) w.y = -w.y;
-			buf[pidx(k)] = cmul(buf[pidx(k)], w);
-		} else {
-			buf[pidx(k)] = make_float2(0.f, 0.f);
-		}
-	}
-	__syncthreads();
-	fft_lds_rt<NT, MAXN, false>(buf, m, twm, tid);
-	for (int k = tid; k < m; k += NT) {
-		float2 b;
-		if (INV) {
-			b = bhat[(m - k) & (m - 1)];
-			b.y = -b.y;
-		} else {
-			b = bhat[k];
-		}
-		buf[pidx(k)] = cmul(buf[pidx(k)], b);
-	}
-	__syncthreads();
-	fft_lds_rt<NT, MAXN, true>(buf, m, twm, tid);
-	const float inv_m = 1.0f / (float)m;
-	for (int k = tid; k < n; k += NT) {
-		float2 w = chirp[k];
-		if (INV) w.y = -w.y;
-		float2 v = cmul(buf[pidx(k)], w);
-		buf[pidx(k)] = make_float2(v.x * inv_m, v.y * inv_m);
-	}
-	__syncthreads();
-}
-
 // A 1D transform of arbitrary length n in LDS, as planned on the host.
 struct Fft1dPlan {
 	int n;                   // transform length
 	int m;                   // working length: n for powers of two and for lengths 2^a 3^b 5^c,
-	                         // else the Bluestein length, a power of two >= 2n-1
-	const float2* tw;        // m-point twiddles
-	const float2* chirp;     // n entries (Bluestein only, else null)
-	const float2* bhat;      // m entries (Bluestein only, else null)
+	                         // else the points of the fine grid, the kernel's MAXN
+	const float2* tw;        // twiddles of the passes: n points, or m / 2 points on the fine grid
 	int nrad;                // mixed-radix passes (lengths 2^a 3^b 5^c that are not powers of two), else 0
 	unsigned char rad[20];   // their radices, in pass order: 8s, then a 4 or 2, then 3s, then 5s
-	// Bluestein lengths n = 4 q whose quarter q has Bluestein length m / 4:
-	// the transform may run as one radix-4 Cooley-Tukey step over four
-	// q-point Bluestein transforms (ct4_bluestein); else sub_chirp is null
-	const float2* sub_chirp; // q entries: the q-point chirp
-	const float2* sub_bhat;  // m / 4 entries
-	const float2* sub_tw;    // m / 4-point twiddles
-	const float2* ct_tw;     // n entries: exp(-2 pi i e / n)
+	// lengths on the fine grid (else null); S = 2 when n is even, else 1
+	const float2* mode;      // [2][n/2 + 1]: the modes' factors on the grid's even and odd points
+	const float4* w8;        // [n/S][2]: the 8 weights of output t around point p0[t] (inverse)
+	const int* p0;           // [n/S]
+	const float4* w4;        // [2][m/2/S]: the 4 weights of fine point 2 i + b from input q0[b][i] on (forward)
+	const int* q0;           // [2][m/2/S]
 };
 
 // ---- mixed-radix FFT (lengths 2^a 3^b 5^c) --------------------------------
@@ -700,107 +589,269 @@ __device__ __forceinline__ void fft_lds_mixed(float2* buf, const Fft1dPlan& p, i
 	}
 }
 
-// ---- one radix-4 step over Bluestein transforms ---------------------------
-// For n = 4 q: X[k1 + q k2] = sum_g W^(g k1) Y_g[k1] exp(-+2 pi i g k2 / 4),
-// W = exp(-+2 pi i / n), with Y_g the q-point DFT of x[4 m + g].  Thread
-// group g (NT/4 threads) runs Y_g as a Bluestein transform on M/4 points in
-// its quarter of buf; the four read their inputs (src, which may read buf)
-// in the first pass, before its barrier, so no quarter is written before
-// every input is read.  The combine reads all Y into registers before the
-// barrier that precedes its writes.  Needs NT/4 > 64 (barriers span the
-// workgroup) and MAXN/4 = the plan's m/4.  Result in logical buf[0..n).
-template <int NT, int MAXN, bool INV, class Src>
-__device__ __forceinline__ void ct4_bluestein(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
+// ---- other lengths: a transform on a finer power-of-two grid ---------------
+// The DFT of any length n on a grid of m = 2 P points, P >= n a power of two,
+// by a band-limited interpolation kernel phi (Kaiser-Bessel, 8 fine points
+// wide, Fourier transform phi^):
+//   inverse:  y[t] = sum_k Y[k] exp(2 pi i k t / n), |k| <= n/2, is the
+//     trigonometric polynomial of the modes at t m / n on the fine grid.  With
+//     g[l] = sum_k (Y[k] / phi^(k/m)) exp(2 pi i k l / m),
+//     y[t] = sum over 8 points l of phi(t m/n - l) g[l].  The even and the odd
+//     points of g are one P-point inverse transform each, the odd one of the
+//     modes turned by exp(pi i k / P): no zero padding is transformed.
+//   forward: the adjoint.  f[l] = sum of phi(l - j m/n) x[j], at most 4 inputs
+//     per fine point; X[k] = (E[k] + exp(-pi i k / P) O[k]) / phi^(k/m) with
+//     E, O the P-point transforms of f's even and odd points.
+// At oversampling m/n >= 2 the kernel's aliasing is below 6e-8 of the result
+// (2e-8 at m/n = 2.4), under the FP32 rounding of the transforms.
+//
+// Why: Bluestein's convolution needs two m-point transforms of which half is
+// padding; this needs two P-point ones and 8 (4) multiply-adds per point.
+// Each half of the workgroup runs one of the two, in its half of buf; every
+// sync spans the workgroup (NT/2 > 64).
+constexpr int kItpHalo = 4;   // entries kept on either side of a periodic LDS array
+
+// For n even the outputs t and t + n/2 of the inverse have the same weights,
+// half the grid apart.  TOBUF: out may write buf (it is called after every
+// read of the grid).
+template <int NT, int MAXN, bool TOBUF, class Src, class Out>
+__device__ __forceinline__ void itp_inv(float2* buf, const Fft1dPlan& p, int tid, const Src& src, const Out& out)
 {
-	constexpr int SNT = NT / 4, SM = MAXN / 4;
-	static_assert(SNT > 64, "the sub-transforms' barriers must span the workgroup");
-	const int g = tid / SNT, lt = tid - g * SNT;
-	const int q = p.n / 4;
-	float2* sb = buf + g * fft_lds_len(SM);           // = buf + pidx(g SM): SM is a multiple of 8
-	auto ld = [&](int i) -> float2 { return src(4 * i + g); };
-	bluestein_io<SNT, SM, INV>(sb, q, p.sub_chirp, p.sub_bhat, p.sub_tw, lt, ld);
-	constexpr int PER = (MAXN / 4 + NT - 1) / NT;
-	float2 y[PER][4];
+	constexpr int P = MAXN / 2, HT = NT / 2, RL = fft_lds_len(P), H = kItpHalo;
+	static_assert(HT > 64, "the halves' barriers must span the workgroup");
+	static_assert(P + 2 * H <= RL, "the halo fits a half of the buffer");
+	const int g = tid / HT, lt = tid - g * HT;
+	float2* hb = buf + g * RL;
+	const int n = p.n, kmax = n / 2, kmin = -((n - 1) / 2);
+	const float2* mode = p.mode + g * (kmax + 1);
+	auto ld = [&](int i) -> float2 {
+		const int k = i < P / 2 ? i : i - P;
+		const bool in = k >= kmin && k <= kmax;
+		const int kc = min(max(k, kmin), kmax);
+		const float2 f = mode[kc < 0 ? -kc : kc];
+		const float2 v = src(kc);
+		const float2 r = kc < 0 ? cmulc(v, f) : cmul(v, f);
+		return in ? r : make_float2(0.f, 0.f);
+	};
+	// the grid's half, linear with its periodic halo
+	auto st = [&](int i, float2 v) {
+		hb[i + H] = v;
+		if (i < H) hb[i + H + P] = v;
+		if (i >= P - H) hb[i + H - P] = v;
+	};
+	fft_lds_io<P, HT, true>(hb, p.tw, lt, ld, st);
+	auto at = [&](const float4& wa, const float4& wb, int l0, int shift) -> float2 {
+		// points l0 .. l0 + 7: the halves alternate, starting with l0's
+		const int e = l0 >> 1, odd = l0 & 1;
+		const float2* ga = buf + (odd ? RL : 0) + e + H + shift;
+		const float2* gb = buf + (odd ? 0 : RL) + e + odd + H + shift;
+		float2 s = make_float2(wa.x * ga[0].x, wa.x * ga[0].y);
+		s.x = fmaf(wa.y, gb[0].x, s.x); s.y = fmaf(wa.y, gb[0].y, s.y);
+		s.x = fmaf(wa.z, ga[1].x, s.x); s.y = fmaf(wa.z, ga[1].y, s.y);
+		s.x = fmaf(wa.w, gb[1].x, s.x); s.y = fmaf(wa.w, gb[1].y, s.y);
+		s.x = fmaf(wb.x, ga[2].x, s.x); s.y = fmaf(wb.x, ga[2].y, s.y);
+		s.x = fmaf(wb.y, gb[2].x, s.x); s.y = fmaf(wb.y, gb[2].y, s.y);
+		s.x = fmaf(wb.z, ga[3].x, s.x); s.y = fmaf(wb.z, ga[3].y, s.y);
+		s.x = fmaf(wb.w, gb[3].x, s.x); s.y = fmaf(wb.w, gb[3].y, s.y);
+		return s;
+	};
+	// PER outputs per thread at most; with n even two of them per weight set
+	constexpr int PER = (P + NT - 1) / NT;
+	static_assert(PER % 2 == 0, "outputs t and t + n/2 in pairs");
+	float2 v[PER];
+	if (n % 2 == 0) {
 #pragma unroll
-	for (int b = 0; b < PER; ++b) {
-		const int t = tid + b * NT;
-		if (t < q) {
-#pragma unroll
-			for (int h = 0; h < 4; ++h) {
-				const float2 v = buf[h * fft_lds_len(SM) + pidx(t)];
-				if (h == 0) {
-					y[b][h] = v;
-				} else {
-					const float2 w = p.ct_tw[h * t];
-					y[b][h] = INV ? cmulc(v, w) : cmul(v, w);
+		for (int b = 0; b < PER / 2; ++b) {
+			const int t = tid + b * NT;
+			if (t < n / 2) {
+				const float4 wa = p.w8[2 * t], wb = p.w8[2 * t + 1];
+				const int l0 = p.p0[t];
+				v[2 * b] = at(wa, wb, l0, 0);
+				v[2 * b + 1] = at(wa, wb, l0, P / 2);
+				if constexpr (!TOBUF) {
+					out(t, v[2 * b]);
+					out(t + n / 2, v[2 * b + 1]);
 				}
 			}
-			dft4<INV>(y[b][0], y[b][1], y[b][2], y[b][3]);
+		}
+		if constexpr (TOBUF) {
+			__syncthreads();
+#pragma unroll
+			for (int b = 0; b < PER / 2; ++b) {
+				const int t = tid + b * NT;
+				if (t < n / 2) {
+					out(t, v[2 * b]);
+					out(t + n / 2, v[2 * b + 1]);
+				}
+			}
+		}
+	} else {
+#pragma unroll
+		for (int b = 0; b < PER; ++b) {
+			const int t = tid + b * NT;
+			if (t < n) {
+				v[b] = at(p.w8[2 * t], p.w8[2 * t + 1], p.p0[t], 0);
+				if constexpr (!TOBUF) out(t, v[b]);
+			}
+		}
+		if constexpr (TOBUF) {
+			__syncthreads();
+#pragma unroll
+			for (int b = 0; b < PER; ++b) {
+				const int t = tid + b * NT;
+				if (t < n) out(t, v[b]);
+			}
+		}
+	}
+}
+
+// The forward transform; result in logical buf[0..n) (visible to the
+// workgroup).
+template <int NT, int MAXN, class Src>
+__device__ __forceinline__ void itp_fwd(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
+{
+	constexpr int P = MAXN / 2, HT = NT / 2, RL = fft_lds_len(P), H = kItpHalo;
+	static_assert(HT > 64, "the halves' barriers must span the workgroup");
+	const int g = tid / HT, lt = tid - g * HT;
+	float2* hb = buf + g * RL;
+	const int n = p.n;
+	constexpr int PER = (P + NT - 1) / NT;
+	{
+		float2 v[PER];
+#pragma unroll
+		for (int b = 0; b < PER; ++b) {
+			const int i = tid + b * NT;
+			if (i < n) v[b] = src(i);
+		}
+		__syncthreads();
+#pragma unroll
+		for (int b = 0; b < PER; ++b) {
+			const int i = tid + b * NT;
+			if (i < n) {
+				buf[i + H] = v[b];
+				if (i < H) buf[i + H + n] = v[b];
+				if (i >= n - H) buf[i + H - n] = v[b];
+			}
+		}
+		__syncthreads();
+	}
+	const bool even = n % 2 == 0;
+	const int sp = even ? P / 2 : P;              // fine points per half with weights of their own
+	const float4* w4 = p.w4 + g * sp;
+	const int* q0 = p.q0 + g * sp;
+	auto ld = [&](int i) -> float2 {
+		const bool up = even && i >= P / 2;
+		const int e = up ? i - P / 2 : i;
+		const float4 w = w4[e];
+		const float2* x = buf + q0[e] + (up ? n / 2 : 0) + H;
+		float2 s = make_float2(w.x * x[0].x, w.x * x[0].y);
+		s.x = fmaf(w.y, x[1].x, s.x); s.y = fmaf(w.y, x[1].y, s.y);
+		s.x = fmaf(w.z, x[2].x, s.x); s.y = fmaf(w.z, x[2].y, s.y);
+		s.x = fmaf(w.w, x[3].x, s.x); s.y = fmaf(w.w, x[3].y, s.y);
+		return s;
+	};
+	auto st = [&](int i, float2 v) { hb[i] = v; };
+	fft_lds_io<P, HT, false>(hb, p.tw, lt, ld, st);
+	const int kmax = n / 2;
+	float2 v[PER];
+#pragma unroll
+	for (int b = 0; b < PER; ++b) {
+		const int i = tid + b * NT;
+		if (i < n) {
+			const int k = i <= kmax ? i : i - n;
+			const int a = k < 0 ? -k : k, l = k & (P - 1);
+			const float2 e = buf[l], o = buf[RL + l];
+			const float d = p.mode[a].x;
+			const float2 f = p.mode[kmax + 1 + a];
+			const float2 t = k < 0 ? cmul(o, f) : cmulc(o, f);
+			v[b] = make_float2(fmaf(e.x, d, t.x), fmaf(e.y, d, t.y));
 		}
 	}
 	__syncthreads();
 #pragma unroll
 	for (int b = 0; b < PER; ++b) {
-		const int t = tid + b * NT;
-		if (t < q) {
-#pragma unroll
-			for (int h = 0; h < 4; ++h) buf[pidx(t + h * q)] = y[b][h];
-		}
+		const int i = tid + b * NT;
+		if (i < n) buf[pidx(i)] = v[b];
 	}
 	__syncthreads();
 }
 
-template <int NT, int MAXN, bool INV>
-__device__ __forceinline__ void fft_any_lds(float2* buf, const Fft1dPlan& p, int tid)
+// ---- any length ------------------------------------------------------------
+// Forward transform of src(i), i in [0, n), result in logical buf[0..n).
+// src may read buf.
+template <int NT, int MAXN, class Src>
+__device__ __forceinline__ void fft_any_fwd(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
 {
-	if (p.nrad > 0) {
-		fft_lds_mixed<NT, MAXN, INV>(buf, p, tid);
-	} else if (p.chirp == nullptr) {
-		fft_lds_rt<NT, MAXN, INV>(buf, p.n, p.tw, tid);
-	} else if (p.m == MAXN) {
-		if constexpr (NT / 4 > 64) {
-			if (p.sub_chirp != nullptr) {
-				ct4_bluestein<NT, MAXN, INV>(buf, p, tid, LdsIn{buf});
-				return;
-			}
-		}
-		bluestein_io<NT, MAXN, INV>(buf, p.n, p.chirp, p.bhat, p.tw, tid, LdsIn{buf});
+	if (p.mode != nullptr) {
+		itp_fwd<NT, MAXN>(buf, p, tid, src);
+	} else if (p.nrad == 0 && p.n == MAXN) {
+		fft_lds_io<MAXN, NT, false>(buf, p.tw, tid, src, LdsOut{buf});
+	} else if (p.nrad == 0 && p.n == MAXN / 2) {
+		fft_lds_io<MAXN / 2, NT, false>(buf, p.tw, tid, src, LdsOut{buf});
 	} else {
-		bluestein_lds<NT, MAXN, INV>(buf, p.n, p.m, p.chirp, p.bhat, p.tw, tid);
+		constexpr int PER = (MAXN + NT - 1) / NT;
+		float2 v[PER];
+#pragma unroll
+		for (int b = 0; b < PER; ++b) {
+			const int i = tid + b * NT;
+			if (i < p.n) v[b] = src(i);
+		}
+		__syncthreads();
+#pragma unroll
+		for (int b = 0; b < PER; ++b) {
+			const int i = tid + b * NT;
+			if (i < p.n) buf[pidx(i)] = v[b];
+		}
+		__syncthreads();
+		if (p.nrad > 0) fft_lds_mixed<NT, MAXN, false>(buf, p, tid);
+		else fft_lds_rt<NT, MAXN, false>(buf, p.n, p.tw, tid);
 	}
 }
 
-// The same transform with the input element i < p.n given by src(i) instead
-// of buf (src may read buf).  Bluestein plans of working length MAXN read src
-// inside the first pass; other plans first gather src into buf.
-template <int NT, int MAXN, bool INV, class Src>
-__device__ __forceinline__ void fft_any_lds_src(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
+// Inverse transform of the modes src(k), k in (-n/2, n/2].  src may read buf.
+template <int NT, int MAXN, class Src>
+__device__ __forceinline__ void fft_inv_passes(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
 {
-	if (p.chirp != nullptr && p.m == MAXN) {
-		if constexpr (NT / 4 > 64) {
-			if (p.sub_chirp != nullptr) {
-				ct4_bluestein<NT, MAXN, INV>(buf, p, tid, src);
-				return;
-			}
-		}
-		bluestein_io<NT, MAXN, INV>(buf, p.n, p.chirp, p.bhat, p.tw, tid, src);
-		return;
-	}
 	constexpr int PER = (MAXN + NT - 1) / NT;
 	float2 v[PER];
 #pragma unroll
-	for (int i = 0; i < PER; ++i) {
-		const int y = tid + i * NT;
-		if (y < p.n) v[i] = src(y);
+	for (int b = 0; b < PER; ++b) {
+		const int i = tid + b * NT;
+		if (i < p.n) v[b] = src(i > p.n / 2 ? i - p.n : i);
 	}
 	__syncthreads();
 #pragma unroll
-	for (int i = 0; i < PER; ++i) {
-		const int y = tid + i * NT;
-		if (y < p.n) buf[pidx(y)] = v[i];
+	for (int b = 0; b < PER; ++b) {
+		const int i = tid + b * NT;
+		if (i < p.n) buf[pidx(i)] = v[b];
 	}
 	__syncthreads();
-	fft_any_lds<NT, MAXN, INV>(buf, p, tid);
+	if (p.nrad > 0) fft_lds_mixed<NT, MAXN, true>(buf, p, tid);
+	else fft_lds_rt<NT, MAXN, true>(buf, p.n, p.tw, tid);
+}
+
+// Every output t handed to out(t, v) once; out may not write buf.
+template <int NT, int MAXN, class Src, class Out>
+__device__ __forceinline__ void fft_any_inv(float2* buf, const Fft1dPlan& p, int tid, const Src& src, const Out& out)
+{
+	if (p.mode != nullptr) {
+		itp_inv<NT, MAXN, false>(buf, p, tid, src, out);
+		return;
+	}
+	fft_inv_passes<NT, MAXN>(buf, p, tid, src);
+	for (int i = tid; i < p.n; i += NT) out(i, buf[pidx(i)]);
+}
+
+// Result in logical buf[0..n), visible to the workgroup.
+template <int NT, int MAXN, class Src>
+__device__ __forceinline__ void fft_any_inv_lds(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
+{
+	if (p.mode != nullptr) {
+		itp_inv<NT, MAXN, true>(buf, p, tid, src, LdsOut{buf});
+		__syncthreads();
+		return;
+	}
+	fft_inv_passes<NT, MAXN>(buf, p, tid, src);
 }
 
 }  // namespace gctf

@@ -91,13 +91,10 @@ __device__ __forceinline__ void rows_r2c_body(const Tin* __restrict__ img, int n
 	const int y0 = 2 * bx;
 	const bool two = (y0 + 1) < ny;
 	const Tin* src = img + (long long)y0 * nx;
-	for (int x = tid; x < nx; x += NT) {
-		float a = load_px(src, x);
-		float b = two ? load_px(src, (long long)nx + x) : 0.f;
-		buf[pidx(x)] = make_float2(a, b);
-	}
-	__syncthreads();
-	fft_any_lds<NT, MAXN, false>(buf, plan, tid);
+	auto px = [&](int x) -> float2 {
+		return make_float2(load_px(src, x), two ? load_px(src, (long long)nx + x) : 0.f);
+	};
+	fft_any_fwd<NT, MAXN>(buf, plan, tid, px);
 	const int ld = spec_ld(ncx_out);
 	float2* dst = out + (long long)y0 * ld;
 	for (int k = tid; k < ncx_out; k += NT) {
@@ -122,7 +119,7 @@ __global__ __launch_bounds__(NT, rescale_waves(MAXN)) void k_rescale_rows_r2c(co
 }
 
 // Rows too long for one LDS transform of length nx (nx even, not a power of
-// two, Bluestein length above MAXN): one row per workgroup as a complex
+// two, working length above MAXN): one row per workgroup as a complex
 // transform of length h = nx/2 of z[m] = x[2m] + i x[2m+1].  With
 // E = (Z[k] + conj Z[h-k]) / 2 and O = -i (Z[k] - conj Z[h-k]) / 2 the
 // transforms of the even and odd samples, X[k] = E[k] + exp(-2 pi i k/nx) O[k]
@@ -136,9 +133,8 @@ __device__ __forceinline__ void rows_r2c_half_body(const Tin* __restrict__ img, 
 	const int tid = threadIdx.x;
 	const int h = nx / 2;
 	const Tin* src = img + (long long)y * nx;
-	for (int m = tid; m < h; m += NT) buf[pidx(m)] = make_float2(load_px(src, 2 * m), load_px(src, 2 * m + 1));
-	__syncthreads();
-	fft_any_lds<NT, MAXN, false>(buf, plan, tid);
+	auto px = [&](int m) -> float2 { return make_float2(load_px(src, 2 * m), load_px(src, 2 * m + 1)); };
+	fft_any_fwd<NT, MAXN>(buf, plan, tid, px);
 	float2* dst = out + (long long)y * spec_ld(ncx_out);
 	for (int k = tid; k < ncx_out; k += NT) {
 		const float2 z = buf[pidx(k)];
@@ -200,17 +196,11 @@ __device__ __forceinline__ void cols_body(const float2* __restrict__ in, int ny,
 	__shared__ float2 buf[fft_lds_len(MAXN)];
 	const int tid = threadIdx.x;
 	const float2* src = in + (long long)kx * ny;
-	for (int y = tid; y < ny; y += NT) buf[pidx(y)] = src[y];
-	__syncthreads();
-	fft_any_lds<NT, MAXN, false>(buf, pf, tid);
-	// the crop is the inverse transform's input
-	auto crop = [&](int y) -> float2 {
-		const int ys = y > nny / 2 ? y - nny + ny : y;
-		return buf[pidx(ys)];
-	};
-	fft_any_lds_src<NT, MAXN, true>(buf, pi, tid, crop);
+	fft_any_fwd<NT, MAXN>(buf, pf, tid, [&](int y) -> float2 { return src[y]; });
+	// the crop: the inverse transform's modes are the forward's
+	auto crop = [&](int k) -> float2 { return buf[pidx(k < 0 ? k + ny : k)]; };
 	float2* dst = out + kx;
-	for (int y = tid; y < nny; y += NT) dst[(long long)y * ncx] = buf[pidx(y)];
+	fft_any_inv<NT, MAXN>(buf, pi, tid, crop, [&](int y, float2 v) { dst[(long long)y * ncx] = v; });
 }
 
 // Grid (8 ceil(ncx / 8), images).
@@ -241,9 +231,7 @@ __device__ __forceinline__ void cols_split_body(const float2* __restrict__ in, i
 	const int h = ny / 2;
 	const float2* src = in + (long long)kx * ny;
 	float2* dst = out + kx;
-	for (int m = tid; m < h; m += NT) buf[pidx(m)] = src[2 * m];
-	__syncthreads();
-	fft_any_lds<NT, MAXN, false>(buf, pf, tid);
+	fft_any_fwd<NT, MAXN>(buf, pf, tid, [&](int m) -> float2 { return src[2 * m]; });
 #pragma unroll
 	for (int j = 0; j < JN; ++j) {
 		const int y = tid + j * NT;
@@ -253,10 +241,7 @@ __device__ __forceinline__ void cols_split_body(const float2* __restrict__ in, i
 			dst[(long long)y * ncx] = buf[pidx(k)];
 		}
 	}
-	__syncthreads();
-	for (int m = tid; m < h; m += NT) buf[pidx(m)] = src[2 * m + 1];
-	__syncthreads();
-	fft_any_lds<NT, MAXN, false>(buf, pf, tid);
+	fft_any_fwd<NT, MAXN>(buf, pf, tid, [&](int m) -> float2 { return src[2 * m + 1]; });
 	float2 x[JN];
 #pragma unroll
 	for (int j = 0; j < JN; ++j) {
@@ -277,8 +262,8 @@ __device__ __forceinline__ void cols_split_body(const float2* __restrict__ in, i
 		if (y < nny) buf[pidx(y)] = x[j];
 	}
 	__syncthreads();
-	fft_any_lds<NT, MAXN, true>(buf, pi, tid);
-	for (int y = tid; y < nny; y += NT) dst[(long long)y * ncx] = buf[pidx(y)];
+	fft_any_inv<NT, MAXN>(buf, pi, tid, [&](int k) -> float2 { return buf[pidx(k < 0 ? k + nny : k)]; },
+		[&](int y, float2 v) { dst[(long long)y * ncx] = v; });
 }
 
 // Grid (8 ceil(ncx / 8), images).
@@ -315,19 +300,14 @@ __device__ __forceinline__ void rows_c2r_body(const float2* __restrict__ in, int
 	// Z = A + i B of the Hermitian extensions, read straight into the
 	// transform's first pass
 	auto herm = [&](int k) -> float2 {
-		float2 a, b;
-		if (k < ncx) {
-			a = ga[k];
-			b = two ? gb[k] : make_float2(0.f, 0.f);
-			if (k == 0 || k == nnx / 2) { a.y = 0.f; b.y = 0.f; }
-		} else {
-			a = ga[nnx - k]; a.y = -a.y;
-			b = two ? gb[nnx - k] : make_float2(0.f, 0.f);
-			b.y = -b.y;
-		}
+		const int c = k < 0 ? -k : k;
+		float2 a = ga[c];
+		float2 b = two ? gb[c] : make_float2(0.f, 0.f);
+		if (c == 0 || c == nnx / 2) { a.y = 0.f; b.y = 0.f; }
+		if (k < 0) { a.y = -a.y; b.y = -b.y; }
 		return make_float2(a.x - b.y, a.y + b.x);
 	};
-	fft_any_lds_src<NT, MAXN, true>(buf, plan, tid, herm);
+	fft_any_inv_lds<NT, MAXN>(buf, plan, tid, herm);
 	float* da = out + (long long)y0 * pitch;
 	for (int x = tid; x < pitch; x += NT) {
 		float2 z = x < nnx ? buf[pidx(x)] : make_float2(0.f, 0.f);
@@ -382,7 +362,8 @@ __device__ __forceinline__ void rows_c2r_half_body(const float2* __restrict__ in
 	const int tid = threadIdx.x;
 	const int ncx = nnx / 2 + 1, h = nnx / 2;
 	const float2* ga = in + (long long)y * ncx;
-	auto fold = [&](int k) -> float2 {
+	auto fold = [&](int ks) -> float2 {
+		const int k = ks < 0 ? ks + h : ks;            // F has period h
 		float2 a = ga[k];                              // X[k], k < h
 		float2 b = ga[h - k];                          // X[k+h] = conj X[h-k]
 		b.y = -b.y;
@@ -394,7 +375,7 @@ __device__ __forceinline__ void rows_c2r_half_body(const float2* __restrict__ in
 		const float2 t = make_float2(cs * di.x - sn * di.y, cs * di.y + sn * di.x);
 		return make_float2(su.x - t.y, su.y + t.x);    // su + i t
 	};
-	fft_any_lds_src<NT, MAXN, true>(buf, plan, tid, fold);
+	fft_any_inv_lds<NT, MAXN>(buf, plan, tid, fold);
 	float* da = out + (long long)y * pitch;
 	for (int x = tid; x < pitch; x += NT) {
 		float v = 0.f;
