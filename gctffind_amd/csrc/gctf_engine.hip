@@ -216,7 +216,7 @@ struct SearchPlan {
 	float lo1d = 0, hi1d = 0, flo2d = 0, fhi2d = 0;
 	float res[2] = {0, 0};
 	RingTables ring{};
-	DevBuf idx, a, b, c2, s2, w;
+	DevBuf idx, abcs, w;
 };
 
 struct GraphEntry {
@@ -228,7 +228,7 @@ struct GraphEntry {
 // Search buffers for at most kStaticMaxImages half spectra of the 512 tile,
 // in one file-scope device array: every GPU the library runs on holds its own
 // copy until the process ends, at its own address (kStaticScratchBytes, about
-// 18 MB).  Host code never passes `scratch` itself to a kernel (on the host
+// 15 MB).  Host code never passes `scratch` itself to a kernel (on the host
 // it names a stand-in, not device memory); it uses the address that
 // hipGetSymbolAddress returned for the device.
 constexpr int kStaticMaxImages = 16;
@@ -238,19 +238,18 @@ constexpr int kStaticMaxRing = 65536;   // ring pixels (zero-padded to 16) per s
 constexpr int kStaticMaxBins = 368;     // integer radius bins of the 512 half spectrum (363 used)
 constexpr size_t st_align(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t kStStates = 0;
-constexpr size_t kStPlans = kStStates + st_align(sizeof(SearchState) * kStaticMaxImages);
+constexpr size_t kStStates2 = kStStates + st_align(sizeof(SearchState) * kStaticMaxImages);
+constexpr size_t kStPlans = kStStates2 + st_align(sizeof(SearchState) * kStaticMaxImages);
 constexpr size_t kStRefine = kStPlans + st_align(sizeof(ImgPlan) * kStaticMaxImages);
 constexpr size_t kStRingSs = kStRefine + st_align(sizeof(RefineArgs) * kStaticMaxImages);
-constexpr size_t kStRadial = kStRingSs + st_align(sizeof(double) * kStaticMaxImages);
-constexpr size_t kStShellCc = kStRadial + st_align(sizeof(float) * kStaticCx * kStaticMaxImages);
-constexpr size_t kStBins = kStShellCc + st_align(sizeof(float) * kStaticCx * kStaticMaxImages);
+constexpr size_t kStRadial = kStRingSs + st_align(sizeof(double) * kRingParts * kStaticMaxImages);
+constexpr size_t kStBins = kStRadial + st_align(sizeof(float) * kStaticCx * kStaticMaxImages);
 constexpr size_t kStPart = kStBins + st_align(sizeof(double) * 6 * kStaticMaxBins * kStaticMaxImages);
 constexpr size_t kStRing = kStPart
-	+ st_align(sizeof(double2) * (size_t)kMaxCands * kPixChunks * kStaticMaxImages);
-constexpr size_t kStCtfMap = kStRing + st_align(sizeof(float) * (size_t)kStaticMaxRing * kStaticMaxImages);
+	+ st_align(sizeof(double2) * (size_t)kPartStride * kStaticMaxImages);
 // 1D search: the workgroup maxima of the reference's 501-point scan x 37 phases
 constexpr int kStaticS1dLd = (501 * 37 + kS1dPerWg - 1) / kS1dPerWg;
-constexpr size_t kStS1d = kStCtfMap + st_align(sizeof(float) * (size_t)kStaticTile * kStaticCx * kStaticMaxImages);
+constexpr size_t kStS1d = kStRing + st_align(sizeof(float) * (size_t)kStaticMaxRing * kStaticMaxImages);
 constexpr size_t kStaticScratchBytes = kStS1d + st_align(sizeof(float2) * (size_t)kStaticS1dLd * kStaticMaxImages);
 
 }  // namespace
@@ -327,7 +326,7 @@ struct gctf_ctx {
 	DevBuf s1part; // 1D search: workgroup maxima of a brute-force stage
 	DevBuf jobs;   // tile work lists of gctf_estimate_list
 	DevBuf rjobs, rtab, list_plans, qnext;   // its rescale jobs, class tables, plans, work-queue counters
-	DevBuf raw, hsum, spect, mom, q, radial, ring_spec, ring_ss, states, part2d, refine, shell_cc, fullsp,
+	DevBuf raw, hsum, spect, mom, q, radial, ring_spec, ring_ss, states, part2d, refine, states2, fullsp,
 		moments1, plans, shell_bins;
 	int kstride = 0;  // ring pixels reserved per image in ring_spec
 	DevBuf g_bt, g_fn, g_gt, g_cc, g_part, g_top, g_rs, g_rescored;
@@ -672,7 +671,8 @@ int get_search_plan(gctf_ctx* c, float kv, float cs, float ac, float pix, int T,
 	if (h > 0.75f) h = 0.75f;
 	float lo2 = l * l, hi2 = h * h;
 	std::vector<int> idx;
-	std::vector<float> a, b, c2, s2, w;
+	std::vector<float4> abcs;
+	std::vector<float> w;
 	const double pir = (double)3.1415926f / M_PI;
 	const double wl = sp->cc.wl, csp = sp->cc.cs;
 	for (int y = 0; y < cy; ++y)
@@ -686,36 +686,24 @@ int get_search_plan(gctf_ctx* c, float kv, float cs, float ac, float pix, int T,
 			double ss = dfx * dfx + dfy * dfy;
 			double th = atan(dfy / (dfx + (double)1e-30f));
 			idx.push_back(y * cx + x);
-			a.push_back((float)(pir * wl * ss));
-			b.push_back((float)(pir * 0.5 * wl * wl * wl * ss * ss * csp));
-			c2.push_back((float)cos(2.0 * th));
-			s2.push_back((float)sin(2.0 * th));
+			abcs.push_back(make_float4((float)(pir * wl * ss), (float)(pir * 0.5 * wl * wl * wl * ss * ss * csp),
+				(float)cos(2.0 * th), (float)sin(2.0 * th)));
 			w.push_back((float)exp(-16.0 * (double)s2f));
 		}
 	const int n = (int)idx.size();
 	if (n == 0) return fail(c, GCTF_ERR_ARG, "empty correlation ring");
 	// zero-padded to a multiple of 16 (w = 0 there) for the grid GEMM's vector loads
 	const int n16 = (n + 15) / 16 * 16;
-	idx.resize(n16, 0); a.resize(n16, 0.f); b.resize(n16, 0.f); c2.resize(n16, 0.f); s2.resize(n16, 0.f);
-	w.resize(n16, 0.f);
+	idx.resize(n16, 0); abcs.resize(n16, make_float4(0.f, 0.f, 0.f, 0.f)); w.resize(n16, 0.f);
 	CHK(ensure_buf(c, sp->idx, sizeof(int) * n16));
-	CHK(ensure_buf(c, sp->a, sizeof(float) * n16));
-	CHK(ensure_buf(c, sp->b, sizeof(float) * n16));
-	CHK(ensure_buf(c, sp->c2, sizeof(float) * n16));
-	CHK(ensure_buf(c, sp->s2, sizeof(float) * n16));
+	CHK(ensure_buf(c, sp->abcs, sizeof(float4) * n16));
 	CHK(ensure_buf(c, sp->w, sizeof(float) * n16));
 	HIPCHK(c, hipMemcpy(sp->idx.p, idx.data(), sizeof(int) * n16, hipMemcpyHostToDevice));
-	HIPCHK(c, hipMemcpy(sp->a.p, a.data(), sizeof(float) * n16, hipMemcpyHostToDevice));
-	HIPCHK(c, hipMemcpy(sp->b.p, b.data(), sizeof(float) * n16, hipMemcpyHostToDevice));
-	HIPCHK(c, hipMemcpy(sp->c2.p, c2.data(), sizeof(float) * n16, hipMemcpyHostToDevice));
-	HIPCHK(c, hipMemcpy(sp->s2.p, s2.data(), sizeof(float) * n16, hipMemcpyHostToDevice));
+	HIPCHK(c, hipMemcpy(sp->abcs.p, abcs.data(), sizeof(float4) * n16, hipMemcpyHostToDevice));
 	HIPCHK(c, hipMemcpy(sp->w.p, w.data(), sizeof(float) * n16, hipMemcpyHostToDevice));
 	sp->ring.n = n;
 	sp->ring.idx = sp->idx.as<int>();
-	sp->ring.a = sp->a.as<float>();
-	sp->ring.b = sp->b.as<float>();
-	sp->ring.c2 = sp->c2.as<float>();
-	sp->ring.s2 = sp->s2.as<float>();
+	sp->ring.abcs = sp->abcs.as<float4>();
 	sp->ring.w = sp->w.as<float>();
 	*out = sp.get();
 	c->splans[key] = std::move(sp);
@@ -826,11 +814,11 @@ int ensure_image_buffers(gctf_ctx* c, int n, int T, int ring_n)
 	CHK(ensure_buf(c, c->mom, sizeof(double) * 2 * nparts * n));
 	CHK(ensure_buf(c, c->radial, sizeof(float) * cx * n));
 	CHK(ensure_buf(c, c->ring_spec, sizeof(float) * (size_t)ring_n * n));
-	CHK(ensure_buf(c, c->ring_ss, sizeof(double) * n));
-	CHK(ensure_buf(c, c->part2d, sizeof(double2) * (size_t)kMaxCands * kPixChunks * n));
+	CHK(ensure_buf(c, c->ring_ss, sizeof(double) * kRingParts * n));
+	CHK(ensure_buf(c, c->part2d, sizeof(double2) * (size_t)kPartStride * n));
+	CHK(ensure_buf(c, c->states2, sizeof(SearchState) * n));
 	CHK(ensure_buf(c, c->refine, sizeof(RefineArgs) * n));
 	CHK(ensure_buf(c, c->plans, sizeof(ImgPlan) * n));
-	CHK(ensure_buf(c, c->shell_cc, sizeof(float) * cx * n));
 	// integer radius bins of the half spectrum: floor(sqrt(cx^2 + (T/2)^2)) + 1 at most
 	const size_t nb = (size_t)std::sqrt((double)cx * cx + (double)(T / 2) * (T / 2)) + 2;
 	CHK(ensure_buf(c, c->shell_bins, sizeof(double) * 6 * nb * n));
@@ -1093,13 +1081,12 @@ int launch_1d_at(gctf_ctx* c, const TileTables& tt, const float* spect, float* r
 {
 	hipStream_t s = c->stream;
 	const int T = tt.T, cx = T / 2 + 1;
-	PROF(c, "k_radial", k_radial<<<dim3((cx + 63) / 64, m), 64, 0, s>>>(spect, cx, T, tt.roff.as<int>(),
-		tt.rcnt.as<int>(), tt.ridx.as<int>(), radial, cx));
 	Search1DParams p{};
 	p.cmpx = cx;
 	p.mode = mode; p.init_df = init_df; p.range = range;
 	p.scan_lo = c->scan_lo; p.scan_hi = c->scan_hi; p.scan_step = c->scan_step;
-	PROF(c, "k_s1d_begin", k_s1d_begin<<<(m + 63) / 64, 64, 0, s>>>(p, plans, st, m));
+	PROF(c, "k_radial", k_radial_s1d<<<dim3((cx + kRadialBins - 1) / kRadialBins, m), 256, 0, s>>>(spect, cx, T,
+		tt.roff.as<int>(), tt.rcnt.as<int>(), tt.ridx.as<int>(), radial, p, plans, st));
 	// Do1D: the scan, then mRefineDefocus around its best; Refine1D: the latter only
 	for (int round = 0; round < (mode == 0 ? 2 : 1); ++round) {
 		PROF(c, "k_s1d_eval", k_s1d_eval<<<dim3(groups, m), 256, 0, s>>>(cx, plans, radial, tt.w1d.as<double>(), st,
@@ -1133,8 +1120,7 @@ struct Search2DView {
 	SearchState* st;
 	double2* part;
 	RefineArgs* refine;
-	float* shell_cc;
-	float* ctfmap;   // final-parameter CTF per half-spectrum pixel (the low-pass scratch)
+	SearchState* st2;   // the other copy of the states: transitions go from one to the other
 	double* bins;    // spectral-CC sums per integer radius bin
 	const int *boff, *bcnt, *bidx;
 	int nbins;
@@ -1150,12 +1136,11 @@ Search2DView view_2d(gctf_ctx* c, int T, int i0)
 	v.spect = c->spect.as<float>() + (size_t)i0 * T * v.cx;
 	v.plans = c->plans.as<ImgPlan>() + i0;
 	v.ring_spec = c->ring_spec.as<float>() + (size_t)i0 * c->kstride;
-	v.ring_ss = c->ring_ss.as<double>() + i0;
+	v.ring_ss = c->ring_ss.as<double>() + (size_t)i0 * kRingParts;
 	v.st = c->states.as<SearchState>() + i0;
-	v.part = c->part2d.as<double2>() + (size_t)i0 * kMaxCands * kPixChunks;
+	v.st2 = c->states2.as<SearchState>() + i0;
+	v.part = c->part2d.as<double2>() + (size_t)i0 * kPartStride;
 	v.refine = c->refine.as<RefineArgs>() + i0;
-	v.shell_cc = c->shell_cc.as<float>() + (size_t)i0 * v.cx;
-	v.ctfmap = c->q.as<float>() + (size_t)i0 * T * v.cx;
 	const TileTables& tt = *c->tiles.at(T);
 	v.nbins = tt.nbins;
 	v.boff = tt.boff.as<int>();
@@ -1165,6 +1150,9 @@ Search2DView view_2d(gctf_ctx* c, int T, int i0)
 	return v;
 }
 
+// Workgroups of a search stage that are resident at once (4 per CU).
+constexpr int kSearchWgs = 1024;
+
 // A 2D search program: `begin`, INIT, the astigmatism grid, `iters` - 1
 // rounds of (ASTMAG, ASTANG, DFMEAN, PHASE), the optional fine defocus
 // stage, then mCalcCtfRes.  The plain program is CFindDefocus2D::mIterate
@@ -1173,59 +1161,85 @@ int run_2d_program(gctf_ctx* c, const Search2DView& v, int m, int begin, const S
 	float phase_range)
 {
 	hipStream_t s = c->stream;
-	PROF(c, "k_ring_gather", k_ring_gather<<<m, 1024, 0, s>>>(v.spect, v.T * v.cx, v.plans, v.kstride,
+	PROF(c, "k_ring_gather", k_ring_gather<<<dim3(kRingParts, m), 256, 0, s>>>(v.spect, v.T * v.cx, v.plans, v.kstride,
 		v.ring_spec, v.ring_ss));
-	// search blocking: candidates per workgroup (each candidate's sums do not
-	// depend on its neighbours, so the choice leaves the results unchanged)
-	auto eval = [&](int maxc) {
-		const int cpb = c->cpb;
-		dim3 grid((maxc + cpb - 1) / cpb, kPixChunks, m);
-		if (cpb == 2)
-			PROF(c, "k_cc2d_eval", k_cc2d_eval<2><<<grid, 256, 0, s>>>(v.plans, v.ring_spec, v.kstride, v.st, v.part));
-		else if (cpb == 4)
-			PROF(c, "k_cc2d_eval", k_cc2d_eval<4><<<grid, 256, 0, s>>>(v.plans, v.ring_spec, v.kstride, v.st, v.part));
-		else if (cpb == 16)
-			PROF(c, "k_cc2d_eval", k_cc2d_eval<16><<<grid, 256, 0, s>>>(v.plans, v.ring_spec, v.kstride, v.st, v.part));
-		else
-			PROF(c, "k_cc2d_eval", k_cc2d_eval<8><<<grid, 256, 0, s>>>(v.plans, v.ring_spec, v.kstride, v.st, v.part));
+	// Transitions go from one copy of the states to the other, stages from one
+	// half of the sums to the other.
+	SearchState* cur = v.st;
+	SearchState* alt = v.st2;
+	double2* sums = v.part;                  // of the stage just evaluated
+	double2* other = v.part + kPartStage;
+	auto args = [&](int next, int next2) {
+		return StepArgs{cur, alt, sums, v.ring_ss, next, next2, v.refine, pg};
 	};
+	// The transition alone.
 	auto step = [&](int next, int next2 = -1) {
-		PROF(c, "k_s2d_step", k_s2d_step<<<m, 256, 0, s>>>(v.st, v.part, v.ring_ss, next, next2, v.refine, pg));
+		PROF(c, "k_s2d_step", k_s2d_step<<<m, 256, 0, s>>>(args(next, next2)));
+		std::swap(cur, alt);
 	};
+	// Candidates per workgroup (each candidate's sums do not depend on its
+	// neighbours, so the choice leaves the results unchanged).  Larger blocks
+	// share more of a pixel's loads and angle and make the transition fewer
+	// times, smaller ones put more workgroups on the chip: the smallest, up to
+	// the context's search blocking, whose workgroups all run at once.  A
+	// search of 16 spectra takes 1800 us so, and 2050 us with the largest
+	// block that still has 1024 workgroups (a second, mostly empty round); of
+	// one spectrum 585 us with blocks of 1 and 620 us with blocks of 2.
+	auto block = [&](int maxc) {
+		int b = 1;
+		while (b < c->cpb && (long long)((maxc + b - 1) / b) * kPixChunks * m > kSearchWgs) b *= 2;
+		return b;
+	};
+#define GCTF_EVAL(CPB, U)                                                                                        \
+	PROF(c, "k_cc2d_eval", k_cc2d_eval<CPB, U, TR><<<dim3((maxc + CPB - 1) / CPB, kPixChunks, m), 256, 0, s>>>( \
+		v.plans, v.ring_spec, v.kstride, cur, other, sa))
+	// One stage of at most maxc candidates, with transition TR into it
+	// (next, next2: the transition's stages, of TR_BEGIN and TR_FINE).
+	auto eval_tr = [&](auto tr, int maxc, int next = -1, int next2 = -1) {
+		constexpr int TR = decltype(tr)::value;
+		const StepArgs sa = args(next, next2);
+		const int b = block(maxc);
+		if (b == 1) GCTF_EVAL(1, 8);
+		else if (b == 2) GCTF_EVAL(2, 8);
+		else if (b == 4) GCTF_EVAL(4, 4);
+		else if (b == 8) GCTF_EVAL(8, 2);
+		else GCTF_EVAL(16, 2);
+		if (TR != TR_NONE) std::swap(cur, alt);
+		std::swap(sums, other);
+	};
+#define GCTF_TR(t) std::integral_constant<int, t>{}
+#undef GCTF_EVAL
 	int maxph = 61;
 	if (phase_range > 61.0f) maxph = std::min(kMaxCands, (int)phase_range + 3);
 	const int last = pg.fine_n >= 2 ? NX_FINE : NX_FINISH;
-	step(begin);
-	eval(1);
+	const bool phase = phase_range > 0.0f;
+	eval_tr(GCTF_TR(TR_BEGIN), 1, begin);
+	// the astigmatism grid: its launch is large, its sums are many
 	step(NX_ASTIG);
-	eval(std::min(kMaxCands, pg.n_ast * pg.n_ang));
+	eval_tr(GCTF_TR(TR_NONE), std::min(kMaxCands, pg.n_ast * pg.n_ang));
 	step(NX_ASTMAG);
 	for (int i = 1; i < pg.iters; ++i) {
 		// line stages hold at most n + 1 candidates (odd counts, prep_line / prep_dfmean)
-		eval(pg.n_mag + 1);
-		step(NX_ASTANG);
-		eval(pg.n_angl + 1);
-		step(NX_DFMEAN);
-		eval(pg.n_df + 1);
-		const int after = i < pg.iters - 1 ? NX_ASTMAG : last;
-		if (phase_range > 0.0f) {
-			step(NX_PHASE);
-			eval(maxph);
-			step(after);
-		} else {
-			step(NX_PHASE, after);   // the phase stage prepares nothing
-		}
+		if (i == 1) eval_tr(GCTF_TR(TR_NONE), pg.n_mag + 1);
+		else if (phase) eval_tr(GCTF_TR(TR_PHASE_ASTMAG), pg.n_mag + 1);
+		else eval_tr(GCTF_TR(TR_ASTMAG), pg.n_mag + 1);
+		eval_tr(GCTF_TR(TR_ASTANG), pg.n_angl + 1);
+		eval_tr(GCTF_TR(TR_DFMEAN), pg.n_df + 1);
+		if (phase) eval_tr(GCTF_TR(TR_PHASE), maxph);
 	}
+	// the transition that ends the rounds: of the phase stage, or of one that
+	// evaluates nothing and then the one after it
+	int next = phase ? last : NX_PHASE, next2 = phase ? -1 : last;
 	if (last == NX_FINE) {
-		eval(pg.fine_n + 1);
-		step(NX_FINISH);
+		eval_tr(GCTF_TR(TR_FINE), pg.fine_n + 1, next, next2);
+		next = NX_FINISH; next2 = -1;
 	}
-	PROF(c, "k_ctf_map", k_ctf_map<<<dim3(v.T, m), 256, 0, s>>>(v.plans, v.cx, v.T, v.st, v.ctfmap));
-	PROF(c, "k_shell_bins", k_shell_bins<<<dim3(v.nbins, m), 64, 0, s>>>(v.spect, v.ctfmap, v.T * v.cx, v.boff,
+#undef GCTF_TR
+	alt = v.st;                              // the last transition ends in the caller's states
+	step(next, next2);
+	PROF(c, "k_shell_bins", k_shell_bins<<<dim3(v.nbins, m), 64, 0, s>>>(v.plans, v.spect, v.cx, v.T, v.boff,
 		v.bcnt, v.bidx, v.nbins, v.st, v.bins));
-	PROF(c, "k_shell_cc", k_shell_cc<<<dim3((v.cx + 63) / 64, m), 64, 0, s>>>(v.bins, v.nbins, v.cx, 10, v.st,
-		v.shell_cc));
-	PROF(c, "k_ctf_res", k_ctf_res<<<(m + 63) / 64, 64, 0, s>>>(v.shell_cc, v.cx, v.T, v.plans, v.st, m));
+	PROF(c, "k_ctf_res", k_ctf_res<<<m, 256, 0, s>>>(v.bins, v.nbins, v.cx, v.T, 10, v.plans, v.st));
 	HIPCHK(c, hipGetLastError());
 	return GCTF_OK;
 }
@@ -1835,8 +1849,7 @@ int gctf_do2d_batch_static(gctf_ctx* ctx, const float* d_spect, int n, gctf_resu
 	v.st = st;
 	v.part = reinterpret_cast<double2*>(base + kStPart);
 	v.refine = reinterpret_cast<RefineArgs*>(base + kStRefine);
-	v.shell_cc = reinterpret_cast<float*>(base + kStShellCc);
-	v.ctfmap = reinterpret_cast<float*>(base + kStCtfMap);
+	v.st2 = reinterpret_cast<SearchState*>(base + kStStates2);
 	v.bins = reinterpret_cast<double*>(base + kStBins);
 	v.nbins = tt.nbins;
 	v.boff = tt.boff.as<int>();
@@ -1979,7 +1992,7 @@ int gctf_radial_average(gctf_ctx* ctx, const float* d_spect, int n, float* d_rad
 	HIPCHK(ctx, hipSetDevice(ctx->device));
 	TileTables* tt;
 	CHK(get_tile_tables(ctx, T, &tt));
-	k_radial<<<dim3((cx + 63) / 64, n), 64, 0, ctx->stream>>>(d_spect, cx, T, tt->roff.as<int>(),
+	k_radial<<<dim3((cx + kRadialBins - 1) / kRadialBins, n), 256, 0, ctx->stream>>>(d_spect, cx, T, tt->roff.as<int>(),
 		tt->rcnt.as<int>(), tt->ridx.as<int>(), d_radial, ld);
 	HIPCHK(ctx, hipGetLastError());
 	HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -2048,7 +2061,7 @@ int launch_grid(gctf_ctx* c, const BatchJob& j, int n)
 	const SearchPlan& r = *j.gring;
 	const int T = r.T, cx = T / 2 + 1;
 	const int K = r.ring.n, kpad = (K + kGemmKs - 1) / kGemmKs * kGemmKs;
-	PROF(c, "k_ring_gather", k_ring_gather_uniform<<<n, 1024, 0, s>>>(c->spect.as<float>(), T * cx, r.ring,
+	PROF(c, "k_ring_gather", k_ring_gather_uniform<<<dim3(kRingParts, n), 256, 0, s>>>(c->spect.as<float>(), T * cx, r.ring,
 		c->ring_spec.as<float>(), c->ring_ss.as<double>()));
 	PROF(c, "k_grid_tables", k_grid_tables<<<(kpad + 255) / 256, 256, 0, s>>>(r.cc, r.ring,
 		c->prm.ext_phase_deg, kpad, c->g_gt.as<float>()));
@@ -2086,7 +2099,7 @@ int record_batch(gctf_ctx* c, const RescalePlan& rp, SearchPlan& sp, TileTables&
 	if (job.mode == 2 || job.mode == 3) {
 		const int T = sp.T, cx = T / 2 + 1;
 		hipStream_t s = c->stream;
-		PROF(c, "k_radial", k_radial<<<dim3((cx + 63) / 64, n), 64, 0, s>>>(c->spect.as<float>(), cx, T, tt.roff.as<int>(),
+		PROF(c, "k_radial", k_radial<<<dim3((cx + kRadialBins - 1) / kRadialBins, n), 256, 0, s>>>(c->spect.as<float>(), cx, T, tt.roff.as<int>(),
 			tt.rcnt.as<int>(), tt.ridx.as<int>(), c->radial.as<float>(), cx));
 		if (job.mode == 3) {
 			HIPCHK(c, hipMemcpy2DAsync(job.radial_out, sizeof(float) * job.radial_ld, c->radial.p,

@@ -23,6 +23,13 @@ enum StageKind : int {
 constexpr int kMaxCands = 2601;
 // Pixel chunks the 2D correlation is split into (partial sums per chunk).
 constexpr int kPixChunks = 8;
+// Partial sums of one image's stage; its buffer holds two stages (a launch
+// reads the previous stage's sums and writes its own).
+constexpr long long kPartStages = 2;
+constexpr long long kPartStage = (long long)kMaxCands * kPixChunks;
+constexpr long long kPartStride = kPartStages * kPartStage;
+// Parts of a ring spectrum's FP64 energy.
+constexpr int kRingParts = 16;
 
 // Per-plan CTF constants in pixel units (CCTFTheory.cpp:77-78,
 // GCalcCTF2D.cu:88-97).
@@ -92,10 +99,8 @@ struct SearchState {
 struct RingTables {
 	int n;                 // ring pixel count
 	const int* idx;        // y * cmpx + x
-	const float* a;        // (pi'/pi) * wl * s^2          (chi/pi per unit df)
-	const float* b;        // (pi'/pi) * 0.5 * wl^3 * s^4 * Cs
-	const float* c2;       // cos(2 theta)
-	const float* s2;       // sin(2 theta)
+	const float4* abcs;    // a = (pi'/pi) * wl * s^2 (chi/pi per unit df), b = (pi'/pi) * 0.5 * wl^3 * s^4 * Cs,
+	                       // cos(2 theta), sin(2 theta)
 	const float* w;        // exp(-16 s^2)
 };
 

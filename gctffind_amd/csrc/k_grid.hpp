@@ -89,11 +89,11 @@ __global__ __launch_bounds__(256) void k_grid_tables(CtfConsts cc, RingTables ri
 	const float ph0 = cand_ctf(cc, 0.f, 0.f, 0.f, ext_phase_deg).ph0;
 	float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 	if (k < ring.n) {
-		const float a = ring.a[k];
-		t[0] = 0.5f * a;
-		t[1] = 0.5f * a * ring.c2[k];
-		t[2] = 0.5f * a * ring.s2[k];
-		t[3] = 0.5f * (ph0 - ring.b[k]);
+		const float4 r = ring.abcs[k];
+		t[0] = 0.5f * r.x;
+		t[1] = 0.5f * r.x * r.z;
+		t[2] = 0.5f * r.x * r.w;
+		t[3] = 0.5f * (ph0 - r.y);
 		t[4] = ring.w[k];
 		t[5] = 0.5f * ring.w[k];
 	}
@@ -341,7 +341,8 @@ __global__ __launch_bounds__(256) void k_grid_rescore(GridSpec g, CtfConsts cc, 
 #pragma unroll
 	for (int j = 0; j < CPB; ++j) { acs[j] = 0.f; acc2[j] = 0.f; cd[j] = cand[j]; }
 	for (int k = k0 + threadIdx.x; k < k1; k += 256) {
-		const float a = ring.a[k], b = ring.b[k], c2 = ring.c2[k], s2 = ring.s2[k], w = ring.w[k], sv = sp[k];
+		const float4 r = ring.abcs[k];
+		const float a = r.x, b = r.y, c2 = r.z, s2 = r.w, w = ring.w[k], sv = sp[k];
 #pragma unroll
 		for (int j = 0; j < CPB; ++j) {
 			float gg = fmaf(c2, cd[j].ca, s2 * cd[j].sa);
@@ -383,7 +384,7 @@ __global__ void k_grid_pick(GridSpec g, const double2* __restrict__ part, const 
 			double2 v = part[((long long)img * kGridTopK + c) * kPixChunks + k];
 			x += v.x; y += v.y;
 		}
-		const double d = sqrt(y * ring_ss[img]);
+		const double d = sqrt(y * ring_energy(ring_ss + img * kRingParts));
 		const float ccv = d == 0.0 ? 0.0f : (float)(x / d);
 		if (rescored) rescored[img * kGridTopK + c] = ccv;
 		if (m >= g.m) continue;

@@ -33,6 +33,31 @@ __device__ __forceinline__ float sinpi_dev(float v)
 	return fmaf(z, p, 0.5f);
 }
 
+// Sums of M values over a wavefront, value i ending in the lanes of group i
+// (lanes [i 64 / M, (i + 1) 64 / M)): each exchange step halves the values a
+// lane still carries, M - 1 exchanges and log2(64 / M) more instead of
+// M log2(64).  Every value is added in the order of the plain xor butterfly.
+template <int M, int O>
+__device__ __forceinline__ double wave_sum_groups(double* v, int lane)
+{
+	if constexpr (O == 0) {
+		return v[0];
+	} else if constexpr (M > 1) {
+		constexpr int H = M / 2;
+		const bool up = (lane & O) != 0;
+		double keep[H];
+#pragma unroll
+		for (int i = 0; i < H; ++i) {
+			const double k = up ? v[i + H] : v[i], g = up ? v[i] : v[i + H];
+			keep[i] = k + __shfl_xor(g, O);
+		}
+		return wave_sum_groups<H, O / 2>(keep, lane);
+	} else {
+		double k[1] = {v[0] + __shfl_xor(v[0], O)};
+		return wave_sum_groups<1, O / 2>(k, lane);
+	}
+}
+
 // ---------------------------------------------------------------------------
 // 1D search (CFindDefocus1D::mBrutalForceSearch, CFindDefocus1D.cpp:76-119;
 // CFindCtf1D::mFindDefocus / mRefineDefocus, CFindCtf1D.cpp:73-111).
@@ -104,14 +129,9 @@ __device__ __forceinline__ void s1d_refine_lattice(SearchState& S, float df_min,
 }
 
 // First stage of Do1D (mFindDefocus) or Refine1D (mRefineDefocus directly).
-__global__ void k_s1d_begin(Search1DParams p, const ImgPlan* __restrict__ plans, SearchState* __restrict__ st,
-	int n)
+__device__ __forceinline__ void s1d_begin(SearchState& S, const Search1DParams& p, float pix)
 {
-	const int b = blockIdx.x * blockDim.x + threadIdx.x;
-	if (b >= n) return;
-	SearchState& S = st[b];
 	if (S.skip) return;
-	const float pix = plans[b].cc.pix;
 	if (p.mode == 0) {
 		const float p2 = pix * pix;
 		const float dfr0 = p.scan_lo > 0.0f ? p.scan_lo : 3000.0f * p2;
@@ -123,6 +143,17 @@ __global__ void k_s1d_begin(Search1DParams p, const ImgPlan* __restrict__ plans,
 	} else {
 		s1d_refine_lattice(S, p.init_df, S.ext_phase, p.range, pix);
 	}
+}
+
+// Radial averages and the first 1D stage of each micrograph (k_radial's
+// grid): neither reads what the other writes.
+__global__ __launch_bounds__(256) void k_radial_s1d(const float* __restrict__ spect, int cmpx, int cmpy,
+	const int* __restrict__ roff, const int* __restrict__ rcnt, const int* __restrict__ ridx,
+	float* __restrict__ radial, Search1DParams p, const ImgPlan* __restrict__ plans, SearchState* __restrict__ st)
+{
+	if (blockIdx.x == 0 && threadIdx.x == 0) s1d_begin(st[blockIdx.y], p, plans[blockIdx.y].cc.pix);
+	radial_body(spect + (long long)blockIdx.y * cmpx * cmpy, cmpx, roff, rcnt, ridx,
+		radial + (long long)blockIdx.y * cmpx, blockIdx.x);
 }
 
 // CC of the pending stage's candidates (GCalcCTF1D.cu:23-32, GCC1D.cu:15-125):
@@ -179,15 +210,14 @@ __global__ __launch_bounds__(256) void k_s1d_eval(int cmpx, const ImgPlan* __res
 	}
 	double dss = ass;
 	for (int o = 32; o > 0; o >>= 1) dss += __shfl_xor(dss, o);
+	double v[2 * kS1dCand];
 #pragma unroll
-	for (int j = 0; j < kS1dCand; ++j) {
-		double dcs = acs[j], dcc = acc[j];
-		for (int o = 32; o > 0; o >>= 1) {
-			dcs += __shfl_xor(dcs, o);
-			dcc += __shfl_xor(dcc, o);
-		}
-		if (lane == 0) s_cc[wave * kS1dCand + j] = (dcc > 0 && dss > 0) ? (float)(dcs / sqrt(dcc * dss)) : 0.0f;
-	}
+	for (int j = 0; j < kS1dCand; ++j) { v[j] = acs[j]; v[kS1dCand + j] = acc[j]; }
+	const double t = wave_sum_groups<2 * kS1dCand, 32>(v, lane);
+	constexpr int GL = 64 / (2 * kS1dCand);      // lanes per sum: cs in the lower half, cc in the upper
+	const double dcc = __shfl_xor(t, 32);
+	if (lane < 32 && lane % GL == 0)
+		s_cc[wave * kS1dCand + lane / GL] = (dcc > 0 && dss > 0) ? (float)(t / sqrt(dcc * dss)) : 0.0f;
 	__syncthreads();
 	if (threadIdx.x == 0) {
 		float best = (float)-1e20;
@@ -259,25 +289,22 @@ __global__ __launch_bounds__(256) void k_s1d_pick(SearchState* __restrict__ st, 
 
 // Candidate c of the pending stage -> (dfmean, ast, ang, phase); false for
 // phase candidates outside the window (CFindDefocus2D.cpp:347).
-__device__ __forceinline__ bool stage_candidate(const SearchState& s, int c, float& dfm, float& ast,
+// kind: the stage's kind (a constant where the caller knows it).
+__device__ __forceinline__ bool stage_candidate(const SearchState& s, int kind, int c, float& dfm, float& ast,
 	float& ang, float& ph)
 {
-	dfm = s.dfmean; ast = s.ast; ang = s.ang; ph = s.phase;
-	switch (s.st_kind) {
-	case ST_ASTIG: {
-		int j = c / s.st_nast, i = c % s.st_nast;
-		ang = s.st_b0 + (float)j * s.st_bstep;
-		ast = s.st_a0 + (float)i * s.st_astep;
-		return true;
-	}
-	case ST_ASTMAG: ast = s.st_a0 + (float)c * s.st_astep; return true;
-	case ST_ASTANG: ang = s.st_a0 + (float)c * s.st_astep; return true;
-	case ST_DFMEAN: dfm = s.st_a0 + (float)c * s.st_astep; return true;
-	case ST_PHASE:
-		ph = s.phase + (float)(c - s.st_n / 2) * s.st_astep;
-		return !(ph < s.st_lo || ph > s.st_hi);
-	default: return true;
-	}
+	// selects, not branches: stores of one value to different variables would
+	// be merged into a store through a pointer, and those kept in memory
+	const float line = s.st_a0 + (float)c * s.st_astep;
+	const int j = kind == ST_ASTIG ? c / s.st_nast : 0, i = c - j * s.st_nast;
+	const float grid_ang = s.st_b0 + (float)j * s.st_bstep;
+	const float grid_ast = s.st_a0 + (float)i * s.st_astep;
+	const float phase = s.phase + (float)(c - s.st_n / 2) * s.st_astep;
+	dfm = kind == ST_DFMEAN ? line : s.dfmean;
+	ast = kind == ST_ASTIG ? grid_ast : kind == ST_ASTMAG ? line : s.ast;
+	ang = kind == ST_ASTIG ? grid_ang : kind == ST_ASTANG ? line : s.ang;
+	ph = kind == ST_PHASE ? phase : s.phase;
+	return kind != ST_PHASE || !(phase < s.st_lo || phase > s.st_hi);
 }
 
 // Per-candidate CTF parameters (CFindDefocus2D::mCorrelate :363-380 and
@@ -341,123 +368,105 @@ __device__ __forceinline__ void cc2d_pixel(const CandCtf* cd, float a, float b, 
 // address arithmetic and waits on the LDS counter too.  The tables are
 // device memory: gload reads them as global memory, from a uniform base and
 // a 32-bit index.
+typedef float float4v __attribute__((ext_vector_type(4)));
 typedef const float __attribute__((address_space(1)))* gfloat_ptr;
+typedef const float4v __attribute__((address_space(1)))* gfloat4_ptr;
 __device__ __forceinline__ float gload(const float* p, int i) { return ((gfloat_ptr)p)[i]; }
+__device__ __forceinline__ float4v gload(const float4* p, int i) { return ((gfloat4_ptr)p)[i]; }
 
-// The pixel loop is unrolled so that the loads of four pixels are in flight
-// together: the small stages run few waves per SIMD, which cannot hide the
-// latency of one pixel's loads behind another wave's arithmetic.
-template <int CPB, bool SHARED>
+// U ring pixels of one thread, 256 apart: the tables and the spectrum.
+template <int U>
+struct PixBatch {
+	float4v t[U];       // a, b, c2, s2
+	float w[U], s[U];
+	// pixels k, k + 256, ...; indexes past the ring read its last pixel
+	__device__ __forceinline__ void load(const RingTables& ring, const float* sp, int k)
+	{
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const int i = min(k + 256 * u, ring.n - 1);
+			t[u] = gload(ring.abcs, i);
+			w[u] = gload(ring.w, i);
+			s[u] = gload(sp, i);
+		}
+	}
+};
+
+// The pixels k0 + thread, + 256, ... below k1, in that order; `cur` holds the
+// first U of them.  The loads of the next U pixels are in flight while the
+// current ones are computed: the small stages run one or two waves per SIMD,
+// which cannot hide the latency of a load behind another wave's arithmetic.
+template <int CPB, bool SHARED, int U>
 __device__ __forceinline__ void cc2d_pixels(const CandCtf* cd, const RingTables& ring, const float* sp,
-	int k0, int k1, float* acc_cs, float* acc_cc)
+	int k0, int k1, PixBatch<U>& cur, float* acc_cs, float* acc_cc)
 {
-#pragma unroll 4
-	for (int k = k0 + (int)threadIdx.x; k < k1; k += 256)
-		cc2d_pixel<CPB, SHARED>(cd, gload(ring.a, k), gload(ring.b, k), gload(ring.c2, k), gload(ring.s2, k),
-			gload(ring.w, k), gload(sp, k), acc_cs, acc_cc);
-}
-
-// Candidate evaluation.  Grid (ceil(max candidates / CPB), kPixChunks,
-// images); 256 threads.  part[image][cand][chunk] = {sum c*S, sum c*c}.
-template <int CPB>
-__global__ __launch_bounds__(256) void k_cc2d_eval(const ImgPlan* __restrict__ plans,
-	const float* __restrict__ ring_spec, int kstride, const SearchState* __restrict__ st,
-	double2* __restrict__ part)
-{
-	const CtfConsts cc = plans[blockIdx.z].cc;
-	const RingTables ring = plans[blockIdx.z].ring;
-	__shared__ CandCtf cand[CPB];
-	__shared__ int cvalid[CPB];
-	__shared__ double red[2][CPB][4];
-	const SearchState& S = st[blockIdx.z];
-	if (S.skip || S.done || S.st_kind == ST_NONE) return;
-	const int n = S.st_n;
-	const int c0 = blockIdx.x * CPB;
-	if (c0 >= n) return;
-	if (threadIdx.x < CPB) {
-		int c = c0 + threadIdx.x;
-		float dfm, ast, ang, ph;
-		bool ok = c < n && stage_candidate(S, c, dfm, ast, ang, ph);
-		cvalid[threadIdx.x] = ok;
-		cand[threadIdx.x] = ok ? cand_ctf(cc, dfm, ast, ang, ph) : CandCtf{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-	}
-	__syncthreads();
-	const int chunk = blockIdx.y;
-	const int per = (ring.n + kPixChunks - 1) / kPixChunks;
-	const int k0 = chunk * per, k1 = min(ring.n, k0 + per);
-	const float* sp = ring_spec + (long long)blockIdx.z * kstride;
-	float acc_cs[CPB], acc_cc[CPB];
+	for (int kb = k0; kb < k1; kb += 256 * U) {
+		PixBatch<U> nxt;
+		nxt.load(ring, sp, kb + 256 * U + (int)threadIdx.x);
+		if (kb + 256 * U <= k1) {
 #pragma unroll
-	for (int j = 0; j < CPB; ++j) { acc_cs[j] = 0.f; acc_cc[j] = 0.f; }
-	CandCtf cd[CPB];
-	bool shared = true;
+			for (int u = 0; u < U; ++u)
+				cc2d_pixel<CPB, SHARED>(cd, cur.t[u].x, cur.t[u].y, cur.t[u].z, cur.t[u].w, cur.w[u], cur.s[u],
+					acc_cs, acc_cc);
+		} else {
 #pragma unroll
-	for (int j = 0; j < CPB; ++j) {
-		cd[j] = cand[j];
-		// invalid candidates are zero and their sums are not stored
-		if (c0 + j < n && cvalid[j])
-			shared = shared && cd[j].ca == cand[0].ca && cd[j].sa == cand[0].sa && cd[j].ph0h == cand[0].ph0h;
-	}
-	if (shared && cvalid[0]) cc2d_pixels<CPB, true>(cd, ring, sp, k0, k1, acc_cs, acc_cc);
-	else cc2d_pixels<CPB, false>(cd, ring, sp, k0, k1, acc_cs, acc_cc);
-	// reduce: wave shuffles in double, then across the 4 waves in LDS
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-	for (int j = 0; j < CPB; ++j) {
-		double x = acc_cs[j], y = acc_cc[j];
-		for (int o = 32; o > 0; o >>= 1) {
-			x += __shfl_xor(x, o);
-			y += __shfl_xor(y, o);
+			for (int u = 0; u < U; ++u)
+				if (kb + 256 * u + (int)threadIdx.x < k1)
+					cc2d_pixel<CPB, SHARED>(cd, cur.t[u].x, cur.t[u].y, cur.t[u].z, cur.t[u].w, cur.w[u], cur.s[u],
+						acc_cs, acc_cc);
 		}
-		if (lane == 0) { red[0][j][wave] = x; red[1][j][wave] = y; }
-	}
-	__syncthreads();
-	if (threadIdx.x < CPB) {
-		const int j = threadIdx.x, c = c0 + j;
-		if (c < n) {
-			double x = red[0][j][0] + red[0][j][1] + red[0][j][2] + red[0][j][3];
-			double y = red[1][j][0] + red[1][j][1] + red[1][j][2] + red[1][j][3];
-			part[((long long)blockIdx.z * kMaxCands + c) * kPixChunks + chunk] = make_double2(x, y);
-		}
+		cur = nxt;
 	}
 }
 
-// Gather the ring pixels of each spectrum and their FP64 energy: ring
-// spectrum of image i at ring_spec + i * kstride.
+// Gather the ring pixels of each spectrum and their FP64 energy, in
+// kRingParts parts (ring_ss[image][part]; ring_energy adds them in order):
+// one workgroup per spectrum left 47 dependent index and pixel loads in a
+// row (14 us on one spectrum).  Ring spectrum of image i at ring_spec +
+// i * kstride.
 __device__ __forceinline__ void ring_gather(const float* __restrict__ in, const RingTables& ring,
-	float* __restrict__ out, double* __restrict__ ss, double* red)
+	float* __restrict__ out, double* __restrict__ ss, int part, double* red)
 {
+	const int per = (ring.n + kRingParts - 1) / kRingParts;
+	const int k0 = part * per, k1 = min(ring.n, k0 + per);
 	double acc = 0.0;
-	for (int k = threadIdx.x; k < ring.n; k += 1024) {
+#pragma unroll 4
+	for (int k = k0 + (int)threadIdx.x; k < k1; k += 256) {
 		float v = in[ring.idx[k]];
 		out[k] = v;
 		acc += (double)v * v;
 	}
-	red[threadIdx.x] = acc;
+	for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+	if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
 	__syncthreads();
-	for (int s = 512; s > 0; s >>= 1) {
-		if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-		__syncthreads();
-	}
-	if (threadIdx.x == 0) *ss = red[0];
+	if (threadIdx.x == 0) ss[part] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ __launch_bounds__(1024) void k_ring_gather(const float* __restrict__ spect, int npix,
+__device__ __forceinline__ double ring_energy(const double* __restrict__ ss)
+{
+	double e = 0.0;
+#pragma unroll
+	for (int p = 0; p < kRingParts; ++p) e += ss[p];
+	return e;
+}
+
+// Grid (kRingParts, images).
+__global__ __launch_bounds__(256) void k_ring_gather(const float* __restrict__ spect, int npix,
 	const ImgPlan* __restrict__ plans, int kstride, float* __restrict__ ring_spec, double* __restrict__ ring_ss)
 {
-	__shared__ double red[1024];
-	const RingTables ring = plans[blockIdx.x].ring;
-	ring_gather(spect + (long long)blockIdx.x * npix, ring, ring_spec + (long long)blockIdx.x * kstride,
-		ring_ss + blockIdx.x, red);
+	__shared__ double red[4];
+	const RingTables ring = plans[blockIdx.y].ring;
+	ring_gather(spect + (long long)blockIdx.y * npix, ring, ring_spec + (long long)blockIdx.y * kstride,
+		ring_ss + blockIdx.y * kRingParts, blockIdx.x, red);
 }
 
 // The same with one ring for the whole batch (the grid search).
-__global__ __launch_bounds__(1024) void k_ring_gather_uniform(const float* __restrict__ spect, int npix,
+__global__ __launch_bounds__(256) void k_ring_gather_uniform(const float* __restrict__ spect, int npix,
 	RingTables ring, float* __restrict__ ring_spec, double* __restrict__ ring_ss)
 {
-	__shared__ double red[1024];
-	ring_gather(spect + (long long)blockIdx.x * npix, ring, ring_spec + (long long)blockIdx.x * ring.n,
-		ring_ss + blockIdx.x, red);
+	__shared__ double red[4];
+	ring_gather(spect + (long long)blockIdx.y * npix, ring, ring_spec + (long long)blockIdx.y * ring.n,
+		ring_ss + blockIdx.y * kRingParts, blockIdx.x, red);
 }
 
 // ---- controller -----------------------------------------------------------
@@ -466,7 +475,7 @@ __global__ __launch_bounds__(1024) void k_ring_gather_uniform(const float* __res
 __device__ __forceinline__ void prep_none(SearchState& s) { s.st_kind = ST_NONE; s.st_n = 0; }
 
 // mFindAstig (CFindDefocus2D.cpp:185-200)
-__device__ void prep_astig(SearchState& s)
+__device__ __forceinline__ void prep_astig(SearchState& s)
 {
 	const float tiny = (float)1e-20;
 	float astr = s.astrange[1] - s.astrange[0];
@@ -486,13 +495,13 @@ __device__ void prep_astig(SearchState& s)
 }
 
 // mRefineAstMag / mRefineAstAng (CFindDefocus2D.cpp:224-286)
-__device__ void prep_line(SearchState& s, int kind, float cur, const float* lim, float range,
+__device__ __forceinline__ void prep_line(SearchState& s, int kind, float cur, float lo, float hi, float range,
 	int n0, float minstep)
 {
 	const float tiny = (float)1e-20;
 	if (range < tiny) { prep_none(s); return; }
-	float mn = fmaxf(cur - range * 0.5f, lim[0]);
-	float mx = fminf(cur + range * 0.5f, lim[1]);
+	float mn = fmaxf(cur - range * 0.5f, lo);
+	float mx = fminf(cur + range * 0.5f, hi);
 	int n = n0;
 	float step = (mx - mn) / (float)(n - 1);
 	if (step < minstep) step = minstep;
@@ -502,7 +511,7 @@ __device__ void prep_line(SearchState& s, int kind, float cur, const float* lim,
 }
 
 // mRefineDfMean (CFindDefocus2D.cpp:288-322)
-__device__ void prep_dfmean(SearchState& s, float range)
+__device__ __forceinline__ void prep_dfmean(SearchState& s, float range)
 {
 	const float tiny = (float)1e-30;
 	if (range < tiny) { prep_none(s); return; }
@@ -518,7 +527,7 @@ __device__ void prep_dfmean(SearchState& s, float range)
 }
 
 // mRefinePhase (CFindDefocus2D.cpp:324-361)
-__device__ void prep_phase(SearchState& s, float range)
+__device__ __forceinline__ void prep_phase(SearchState& s, float range)
 {
 	const float tiny = (float)1e-30;
 	if (range < tiny) { prep_none(s); return; }
@@ -545,7 +554,7 @@ __device__ __forceinline__ float iter_scale(const SearchState& s, int i)
 
 // Learned path's last stage: s.pg.fine_n defocus candidates s.pg.fine_step
 // apart around the current mean defocus, inside the window.
-__device__ void prep_fine(SearchState& s)
+__device__ __forceinline__ void prep_fine(SearchState& s)
 {
 	if (s.pg.fine_n < 2) { prep_none(s); return; }
 	const int h = s.pg.fine_n / 2;
@@ -577,7 +586,7 @@ struct RefineArgs {
 
 // Prepare stage `next` of state s (prev_kind: the kind of the stage just
 // consumed) and, at the end of the search, write the results.
-__device__ void advance_state(SearchState& s, int prev_kind, int next)
+__device__ __forceinline__ void advance_state(SearchState& s, int prev_kind, int next)
 {
 	if (!s.done) {
 		switch (next) {
@@ -594,13 +603,13 @@ __device__ void advance_state(SearchState& s, int prev_kind, int next)
 				s.tot_ang = s.angrange[1] - s.angrange[0];
 			}
 			s.iter += 1;
-			prep_line(s, ST_ASTMAG, s.ast, s.astrange, iter_scale(s, s.iter) * s.tot_ast, s.pg.n_mag, 0.001f);
+			prep_line(s, ST_ASTMAG, s.ast, s.astrange[0], s.astrange[1], iter_scale(s, s.iter) * s.tot_ast, s.pg.n_mag, 0.001f);
 			break;
 		case NX_ASTANG:
 			// CFindDefocus2D.cpp:171-173
 			if (s.oldcc > s.ccmax) { s.done = 1; break; }
 			s.ccmax = s.oldcc;
-			prep_line(s, ST_ASTANG, s.ang, s.angrange, iter_scale(s, s.iter) * s.tot_ang, s.pg.n_angl, 1.0f);
+			prep_line(s, ST_ASTANG, s.ang, s.angrange[0], s.angrange[1], iter_scale(s, s.iter) * s.tot_ang, s.pg.n_angl, 1.0f);
 			break;
 		case NX_DFMEAN:
 			prep_dfmean(s, iter_scale(s, s.iter) * s.tot_df);
@@ -628,187 +637,369 @@ __device__ void advance_state(SearchState& s, int prev_kind, int next)
 	}
 }
 
-// One workgroup (256 threads) per micrograph: consume the CCs of the stage
-// just evaluated (first strict maximum, `<= continue` order), update the
-// state as the reference method does, and prepare the next stage (then
-// next2's, when next2 >= 0 and stage `next` evaluates nothing).
-__global__ __launch_bounds__(256) void k_s2d_step(SearchState* __restrict__ st,
-	const double2* __restrict__ part, const double* __restrict__ ring_ss, int next, int next2,
-	const RefineArgs* __restrict__ refine, SearchProgram prog)
+__device__ __forceinline__ void step_program(SearchProgram& d, const SearchProgram& s)
+{
+	d.n_ast = s.n_ast; d.n_ang = s.n_ang; d.n_mag = s.n_mag; d.n_angl = s.n_angl;
+	d.n_df = s.n_df; d.iters = s.iters; d.df_minstep = s.df_minstep;
+	d.fine_n = s.fine_n; d.fine_step = s.fine_step;
+}
+
+// The fields of a state that a transition reads or writes, one by one (a
+// struct assignment would keep the copy in memory instead of registers).
+__device__ __forceinline__ void step_fields(SearchState& d, const SearchState& s)
+{
+	d.df_min = s.df_min; d.df_max = s.df_max; d.ast_ang = s.ast_ang; d.ext_phase = s.ext_phase; d.score = s.score;
+	d.phase_range = s.phase_range;
+	d.dfmean = s.dfmean; d.ast = s.ast; d.ang = s.ang; d.phase = s.phase; d.ccmax = s.ccmax; d.oldcc = s.oldcc;
+#pragma unroll
+	for (int i = 0; i < 2; ++i) {
+		d.dfrange[i] = s.dfrange[i]; d.astrange[i] = s.astrange[i];
+		d.angrange[i] = s.angrange[i]; d.phrange[i] = s.phrange[i];
+	}
+	d.tot_df = s.tot_df; d.tot_ast = s.tot_ast; d.tot_ang = s.tot_ang;
+	d.done = s.done; d.iter = s.iter; d.skip = s.skip;
+	d.st_kind = s.st_kind; d.st_n = s.st_n; d.st_nast = s.st_nast;
+	d.st_a0 = s.st_a0; d.st_astep = s.st_astep; d.st_b0 = s.st_b0; d.st_bstep = s.st_bstep;
+	d.st_lo = s.st_lo; d.st_hi = s.st_hi; d.st_old = s.st_old;
+	step_program(d.pg, s.pg);
+}
+
+// The new state s of a transition from `in` into `out` by the lanes of one
+// wavefront: the words of `in`, then the transition's fields over them.
+__device__ __forceinline__ void step_store(SearchState* out, const SearchState* in, const SearchState& s, int lane)
+{
+	static_assert(sizeof(SearchState) % 4 == 0, "copied by words");
+	if (out != in)
+		for (int i = lane; i < (int)(sizeof(SearchState) / 4); i += 64)
+			reinterpret_cast<int*>(out)[i] = reinterpret_cast<const int*>(in)[i];
+	if (lane == 0) step_fields(*out, s);
+}
+
+// The transitions that start a 2D search from the 1D result or a proposal.
+__device__ __forceinline__ void step_begin(SearchState& s, int next, const RefineArgs* refine, const SearchProgram& prog)
+{
+	step_program(s.pg, plain_program());
+	if (next == NX_BEGIN_PROPOSAL) {
+		// the reference's DoIt box (CFindDefocus2D.cpp:113-118) with the
+		// defocus window of the proposal
+		const RefineArgs& r = *refine;
+		step_program(s.pg, prog);
+		s.dfmean = r.dfmean[0]; s.ast = 0.0f; s.ang = 0.0f;
+		s.phrange[0] = s.ext_phase;
+		s.phrange[1] = s.phase_range;
+		const float h = 0.5f * r.dfmean[1];
+		s.dfrange[0] = fmaxf(s.dfmean - h, 3000.0f);
+		s.dfrange[1] = s.dfmean + h;
+		s.astrange[0] = 0.0f; s.astrange[1] = 0.06f;
+		s.angrange[0] = -90.0f; s.angrange[1] = 90.0f;
+	} else if (next == NX_BEGIN_DO2D) {
+		// CFindCtf2D::Do2D (CFindCtf2D.cpp:44-53) + DoIt (:110-124)
+		float dfmean = (s.df_min + s.df_max) * 0.5f;
+		s.dfmean = dfmean; s.ast = 0.0f; s.ang = 0.0f;
+		s.phrange[0] = s.ext_phase;
+		s.phrange[1] = s.phase_range;
+		s.dfrange[0] = s.dfmean * 0.9f; s.dfrange[1] = s.dfmean * 1.1f;
+		s.astrange[0] = 0.0f; s.astrange[1] = 0.06f;
+		s.angrange[0] = -90.0f; s.angrange[1] = 90.0f;
+	} else {
+		// CFindCtf2D::Refine (CFindCtf2D.cpp:55-68) + Refine (:126-151)
+		const RefineArgs& r = *refine;
+		s.dfmean = r.dfmean[0]; s.ast = r.ast[0]; s.ang = r.ang[0];
+		s.phrange[0] = r.phase[0];
+		float h = 0.5f * r.dfmean[1];
+		s.dfrange[0] = fmaxf(s.dfmean - h, 3000.0f);
+		s.dfrange[1] = s.dfmean + h;
+		h = 0.5f * r.ast[1];
+		s.astrange[0] = fmaxf(s.ast - h, 0.0f);
+		s.astrange[1] = fminf(s.ast + h, 0.02f);
+		h = 0.5f * r.ang[1];
+		s.angrange[0] = fmaxf(s.ang - h, -90.0f);
+		s.angrange[1] = fminf(s.ang + h, 90.0f);
+		s.phrange[1] = r.phase[1];
+	}
+	s.done = 0; s.iter = 0;
+	s.st_kind = ST_INIT; s.st_n = 1;
+}
+
+// The stage's winner (candidate win with CC wcc; ran: the stage evaluated
+// anything) into the state as the reference method does, then the
+// preparation of stage `next` (then next2's, when next2 >= 0: a second
+// transition with no stage evaluated in between, after the phase stage of a
+// search without phase range).
+__device__ __forceinline__ void step_consume(SearchState& s, int kind, int win, float wcc, bool ran, int next,
+	int next2)
+{
+	const int prev = s.st_kind;
+	if (ran && win >= 0) {
+		float dfm, ast, ang, ph;
+		stage_candidate(s, kind, win, dfm, ast, ang, ph);
+		// INIT sets the score, the others take a strictly better one; the
+		// candidate's other parameters are the state's own
+		const bool init = kind == ST_INIT;
+		if (init || wcc > s.ccmax) {
+			s.dfmean = dfm; s.ast = ast; s.ang = ang; s.phase = ph;
+			s.ccmax = wcc;
+			s.oldcc = init ? wcc : s.oldcc;
+		}
+	}
+	advance_state(s, prev, next);
+	if (next2 >= 0 && !s.done) advance_state(s, s.st_kind, next2);
+}
+
+// Candidate evaluation.  Grid (ceil(max candidates / CPB), kPixChunks,
+// images); 256 threads.  part[image][cand][chunk] = {sum c*S, sum c*c}, an
+// image's sums kPartStride apart.
+//
+// TR: the launch also makes this transition into the stage it evaluates (a
+// template parameter: each instance holds the code of one transition only).
+// Wave 0 of every workgroup takes the maximum of the previous stage's sums
+// (prev) and prepares the stage from st_in; workgroup (0, 0) of an image
+// leaves the new state in st_out, so st_in and st_out, and prev and part,
+// must not overlap.  The transition is small (at most a few hundred
+// candidates' sums, the same for every workgroup, and the first pixels load
+// meanwhile), where a launch of its own costs about 8 us of a chain of 59
+// stages: a search of one spectrum took 1350 us with two launches per stage.
+enum StageTransition : int {
+	TR_NONE = -1,
+	TR_BEGIN = 0,          // begin (StepArgs::next) -> INIT
+	TR_ASTANG = 1,         // ASTMAG -> ASTANG
+	TR_DFMEAN = 2,         // ASTANG -> DFMEAN
+	TR_PHASE = 3,          // DFMEAN -> PHASE
+	TR_ASTMAG = 4,         // DFMEAN -> next round's ASTMAG (no phase range)
+	TR_PHASE_ASTMAG = 5,   // PHASE -> next round's ASTMAG
+	TR_FINE = 6,           // DFMEAN or PHASE -> the fine defocus stage (StepArgs::next, next2)
+};
+struct StepArgs {
+	const SearchState* st_in;
+	SearchState* st_out;
+	const double2* prev;
+	const double* ring_ss;
+	int next, next2;
+	const RefineArgs* refine;
+	SearchProgram prog;
+};
+
+// CC of candidate c from its chunks' sums p[0 .. kPixChunks).
+__device__ __forceinline__ float step_cc(const double2* p, double ss)
+{
+	double x = 0.0, y = 0.0;
+#pragma unroll
+	for (int k = 0; k < kPixChunks; ++k) { x += p[k].x; y += p[k].y; }
+	const double d = sqrt(y * ss);
+	return d == 0.0 ? 0.0f : (float)(x / d);
+}
+
+// First strict maximum of the stage's CCs over the candidates c = i, i + n,
+// ... (ties keep the smaller index, CFindDefocus2D.cpp's `<= continue`);
+// `first` holds candidate i's sums.
+__device__ __forceinline__ void step_scan(const SearchState& s, int kind, const double2* __restrict__ pp,
+	const double2* first, double ss, int i, int n, float& best, int& bi)
+{
+	best = (float)-1e20;
+	bi = -1;
+	for (int c = i; c < s.st_n; c += n) {
+		float dfm, ast, ang, ph;
+		if (!stage_candidate(s, kind, c, dfm, ast, ang, ph)) continue;
+		double2 v[kPixChunks];
+#pragma unroll
+		for (int k = 0; k < kPixChunks; ++k) v[k] = c == i ? first[k] : pp[(long long)c * kPixChunks + k];
+		const float cc = step_cc(v, ss);
+		if (cc > best) { best = cc; bi = c; }
+	}
+}
+__device__ __forceinline__ bool step_better(float c2, int i2, float c1, int i1)
+{
+	return i2 >= 0 && (i1 < 0 || c2 > c1 || (c2 == c1 && i2 < i1));
+}
+
+template <int CPB, int U, int TR>
+__global__ __launch_bounds__(256, CPB >= 4 && CPB <= 8 ? 4 : 2) void k_cc2d_eval(const ImgPlan* __restrict__ plans,
+	const float* __restrict__ ring_spec, int kstride, const SearchState* __restrict__ st,
+	double2* __restrict__ part, StepArgs sa)
+{
+	const int img = blockIdx.z;
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+	const int c0 = blockIdx.x * CPB;
+	__shared__ CandCtf cand[CPB];
+	__shared__ int cvalid[CPB];
+	__shared__ int s_n;
+	__shared__ double red[2 * CPB][4];
+	constexpr bool STEP = TR != TR_NONE;
+	if constexpr (!STEP) {
+		const SearchState& S = st[img];
+		if (S.skip || S.done || S.st_kind == ST_NONE || c0 >= S.st_n) return;
+	}
+	const CtfConsts cc = plans[img].cc;
+	const RingTables ring = plans[img].ring;
+	const int chunk = blockIdx.y;
+	const int per = (ring.n + kPixChunks - 1) / kPixChunks;
+	const int k0 = chunk * per, k1 = min(ring.n, k0 + per);
+	const float* sp = ring_spec + (long long)img * kstride;
+	// candidate `lane`'s sums of the previous stage, read along with its state
+	// (in the buffer whatever the stage's count)
+	static_assert(kMaxCands >= 64, "a wave's first candidates are in the buffer");
+	double2 first[kPixChunks];
+	const double2* pp = sa.prev + (long long)img * kPartStride;
+	if constexpr (STEP && TR != TR_BEGIN) {
+		if (wave == 0) {
+#pragma unroll
+			for (int k = 0; k < kPixChunks; ++k) first[k] = pp[lane * kPixChunks + k];
+		}
+	}
+	PixBatch<U> cur;
+	cur.load(ring, sp, k0 + tid);
+	if (wave == 0) {
+		SearchState s;
+		if constexpr (STEP) {
+			step_fields(s, sa.st_in[img]);
+			if (!s.skip) {
+				if constexpr (TR == TR_BEGIN) {
+					step_begin(s, sa.next, sa.refine + img, sa.prog);
+				} else {
+					const int kind = TR == TR_ASTANG ? ST_ASTMAG : TR == TR_DFMEAN ? ST_ASTANG
+						: TR == TR_PHASE || TR == TR_ASTMAG ? ST_DFMEAN : TR == TR_PHASE_ASTMAG ? ST_PHASE : s.st_kind;
+					const int next = TR == TR_ASTANG ? NX_ASTANG : TR == TR_DFMEAN ? NX_DFMEAN
+						: TR == TR_PHASE || TR == TR_ASTMAG ? NX_PHASE : TR == TR_PHASE_ASTMAG ? NX_ASTMAG : sa.next;
+					const int next2 = TR == TR_ASTMAG ? NX_ASTMAG : TR == TR_FINE ? sa.next2 : -1;
+					const bool ran = !s.done && s.st_kind != ST_NONE && s.st_n > 0;
+					float best = (float)-1e20;
+					int bi = -1;
+					if (ran)
+						step_scan(s, kind, pp, first, ring_energy(sa.ring_ss + img * kRingParts), lane, 64, best, bi);
+					for (int o = 32; o > 0; o >>= 1) {
+						const float c2 = __shfl_xor(best, o);
+						const int i2 = __shfl_xor(bi, o);
+						if (step_better(c2, i2, best, bi)) { best = c2; bi = i2; }
+					}
+					step_consume(s, kind, bi, best, ran, next, next2);
+				}
+			}
+			if (blockIdx.x == 0 && chunk == 0) step_store(sa.st_out + img, sa.st_in + img, s, lane);
+		} else {
+			step_fields(s, st[img]);
+		}
+		const int n = (s.skip || s.done || s.st_kind == ST_NONE) ? 0 : s.st_n;
+		if (lane == 0) s_n = n;
+		if (lane < CPB) {
+			const int c = c0 + lane;
+			float dfm, ast, ang, ph;
+			const bool ok = c < n && stage_candidate(s, s.st_kind, c, dfm, ast, ang, ph);
+			cvalid[lane] = ok;
+			cand[lane] = ok ? cand_ctf(cc, dfm, ast, ang, ph) : CandCtf{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+		}
+	}
+	__syncthreads();
+	const int n = s_n;
+	if (c0 >= n) return;
+	float acc_cs[CPB], acc_cc[CPB];
+#pragma unroll
+	for (int j = 0; j < CPB; ++j) { acc_cs[j] = 0.f; acc_cc[j] = 0.f; }
+	CandCtf cd[CPB];
+	bool shared = true;
+#pragma unroll
+	for (int j = 0; j < CPB; ++j) {
+		cd[j] = cand[j];
+		// invalid candidates are zero and their sums are not stored
+		if (c0 + j < n && cvalid[j])
+			shared = shared && cd[j].ca == cand[0].ca && cd[j].sa == cand[0].sa && cd[j].ph0h == cand[0].ph0h;
+	}
+	if (shared && cvalid[0]) cc2d_pixels<CPB, true, U>(cd, ring, sp, k0, k1, cur, acc_cs, acc_cc);
+	else cc2d_pixels<CPB, false, U>(cd, ring, sp, k0, k1, cur, acc_cs, acc_cc);
+	// reduce: over the wave in double, then across the 4 waves in LDS
+	double v[2 * CPB];
+#pragma unroll
+	for (int j = 0; j < CPB; ++j) { v[j] = acc_cs[j]; v[CPB + j] = acc_cc[j]; }
+	const double t = wave_sum_groups<2 * CPB, 32>(v, lane);
+	constexpr int GL = 64 / (2 * CPB);      // lanes per value
+	if (lane % GL == 0) red[lane / GL][wave] = t;
+	__syncthreads();
+	if (tid < CPB) {
+		const int j = tid, c = c0 + j;
+		if (c < n) {
+			const double x = red[j][0] + red[j][1] + red[j][2] + red[j][3];
+			const double y = red[CPB + j][0] + red[CPB + j][1] + red[CPB + j][2] + red[CPB + j][3];
+			part[(long long)img * kPartStride + (long long)c * kPixChunks + chunk] = make_double2(x, y);
+		}
+	}
+}
+
+// One workgroup (256 threads) per micrograph: the transition alone, for the
+// stages whose sums are too many for every workgroup of the next one to read
+// (the astigmatism grid), and the last.  st_out may be st_in.
+__global__ __launch_bounds__(256) void k_s2d_step(StepArgs sa)
 {
 	__shared__ float s_cc[256];
 	__shared__ int s_i[256];
-	SearchState* S = st + blockIdx.x;
-	const int tid = threadIdx.x;
-	if (S->skip) return;
-	if (next == NX_BEGIN_DO2D || next == NX_BEGIN_REFINE || next == NX_BEGIN_PROPOSAL) {
-		if (tid == 0) {
-			SearchState s = *S;
-			s.pg = plain_program();
-			if (next == NX_BEGIN_PROPOSAL) {
-				// the reference's DoIt box (CFindDefocus2D.cpp:113-118) with the
-				// defocus window of the proposal
-				const RefineArgs& r = refine[blockIdx.x];
-				s.pg = prog;
-				s.dfmean = r.dfmean[0]; s.ast = 0.0f; s.ang = 0.0f;
-				s.phrange[0] = s.ext_phase;
-				s.phrange[1] = s.phase_range;
-				const float h = 0.5f * r.dfmean[1];
-				s.dfrange[0] = fmaxf(s.dfmean - h, 3000.0f);
-				s.dfrange[1] = s.dfmean + h;
-				s.astrange[0] = 0.0f; s.astrange[1] = 0.06f;
-				s.angrange[0] = -90.0f; s.angrange[1] = 90.0f;
-			} else if (next == NX_BEGIN_DO2D) {
-				// CFindCtf2D::Do2D (CFindCtf2D.cpp:44-53) + DoIt (:110-124)
-				float dfmean = (s.df_min + s.df_max) * 0.5f;
-				s.dfmean = dfmean; s.ast = 0.0f; s.ang = 0.0f;
-				s.phrange[0] = s.ext_phase;
-				s.phrange[1] = s.phase_range;
-				s.dfrange[0] = s.dfmean * 0.9f; s.dfrange[1] = s.dfmean * 1.1f;
-				s.astrange[0] = 0.0f; s.astrange[1] = 0.06f;
-				s.angrange[0] = -90.0f; s.angrange[1] = 90.0f;
-			} else {
-				// CFindCtf2D::Refine (CFindCtf2D.cpp:55-68) + Refine (:126-151)
-				const RefineArgs& r = refine[blockIdx.x];
-				s.dfmean = r.dfmean[0]; s.ast = r.ast[0]; s.ang = r.ang[0];
-				s.phrange[0] = r.phase[0];
-				float h = 0.5f * r.dfmean[1];
-				s.dfrange[0] = fmaxf(s.dfmean - h, 3000.0f);
-				s.dfrange[1] = s.dfmean + h;
-				h = 0.5f * r.ast[1];
-				s.astrange[0] = fmaxf(s.ast - h, 0.0f);
-				s.astrange[1] = fminf(s.ast + h, 0.02f);
-				h = 0.5f * r.ang[1];
-				s.angrange[0] = fmaxf(s.ang - h, -90.0f);
-				s.angrange[1] = fminf(s.ang + h, 90.0f);
-				s.phrange[1] = r.phase[1];
-			}
-			s.done = 0; s.iter = 0;
-			s.st_kind = ST_INIT; s.st_n = 1;
-			*S = s;
-		}
+	const int img = blockIdx.x, tid = threadIdx.x;
+	SearchState s;
+	step_fields(s, sa.st_in[img]);
+	if (s.skip) {
+		if (tid < 64) step_store(sa.st_out + img, sa.st_in + img, s, tid);
 		return;
 	}
-	// ---- argmax of the evaluated stage
-	const SearchState s0 = *S;
-	const bool ran = !s0.done && s0.st_kind != ST_NONE && s0.st_n > 0;
+	const bool ran = !s.done && s.st_kind != ST_NONE && s.st_n > 0;
 	float best = (float)-1e20;
 	int bi = -1;
 	if (ran) {
-		const double ss = ring_ss[blockIdx.x];
-		const double2* pp = part + (long long)blockIdx.x * kMaxCands * kPixChunks;
-		for (int c = tid; c < s0.st_n; c += 256) {
-			float dfm, ast, ang, ph;
-			if (!stage_candidate(s0, c, dfm, ast, ang, ph)) continue;
-			double x = 0.0, y = 0.0;
-			for (int k = 0; k < kPixChunks; ++k) {
-				double2 v = pp[(long long)c * kPixChunks + k];
-				x += v.x; y += v.y;
-			}
-			double d = sqrt(y * ss);
-			float cc = d == 0.0 ? 0.0f : (float)(x / d);
-			if (cc > best) { best = cc; bi = c; }
-		}
+		const double2* pp = sa.prev + (long long)img * kPartStride;
+		double2 first[kPixChunks];
+#pragma unroll
+		for (int k = 0; k < kPixChunks; ++k) first[k] = pp[tid * kPixChunks + k];
+		step_scan(s, s.st_kind, pp, first, ring_energy(sa.ring_ss + img * kRingParts), tid, 256, best, bi);
 	}
 	s_cc[tid] = best; s_i[tid] = bi;
 	__syncthreads();
 	for (int o = 128; o > 0; o >>= 1) {
-		if (tid < o) {
-			float c2 = s_cc[tid + o];
-			int i2 = s_i[tid + o];
-			float c1 = s_cc[tid];
-			int i1 = s_i[tid];
-			if (i2 >= 0 && (i1 < 0 || c2 > c1 || (c2 == c1 && i2 < i1))) {
-				s_cc[tid] = c2; s_i[tid] = i2;
-			}
+		if (tid < o && step_better(s_cc[tid + o], s_i[tid + o], s_cc[tid], s_i[tid])) {
+			s_cc[tid] = s_cc[tid + o];
+			s_i[tid] = s_i[tid + o];
 		}
 		__syncthreads();
 	}
-	if (tid != 0) return;
-	SearchState s = s0;
-	const int win = s_i[0];
-	const float wcc = s_cc[0];
-	if (ran && win >= 0) {
-		float dfm, ast, ang, ph;
-		stage_candidate(s0, win, dfm, ast, ang, ph);
-		switch (s0.st_kind) {
-		case ST_INIT:
-			s.ccmax = wcc; s.oldcc = wcc;
-			break;
-		case ST_ASTIG:
-			if (wcc > s.ccmax) { s.ast = ast; s.ang = ang; s.ccmax = wcc; }
-			break;
-		case ST_ASTMAG:
-			if (wcc > s.ccmax) { s.ast = ast; s.ccmax = wcc; }
-			break;
-		case ST_ASTANG:
-			if (wcc > s.ccmax) { s.ang = ang; s.ccmax = wcc; }
-			break;
-		case ST_DFMEAN:
-			if (wcc > s.ccmax) { s.dfmean = dfm; s.ccmax = wcc; }
-			break;
-		case ST_PHASE:
-			if (wcc > s.ccmax) { s.phase = ph; s.ccmax = wcc; }
-			break;
-		default: break;
-		}
-	}
-	advance_state(s, s0.st_kind, next);
-	// a second transition with no stage evaluated in between (the phase
-	// stage of a search without phase range prepares nothing)
-	if (next2 >= 0 && !s.done) advance_state(s, s.st_kind, next2);
-	*S = s;
+	if (tid >= 64) return;
+	step_consume(s, s.st_kind, s_i[0], s_cc[0], ran, sa.next, sa.next2);
+	step_store(sa.st_out + img, sa.st_in + img, s, tid);
 }
 
 // ---------------------------------------------------------------------------
-// The CTF at the final parameters over the half spectrum, in FP32 with the
-// reference formula (GCalcCTF2D.cu:23-37, GSpectralCC2D.cu:12-109), once
-// per pixel: every pixel belongs to about ten shells.  Grid (cmpy, images).
-__global__ __launch_bounds__(256) void k_ctf_map(const ImgPlan* __restrict__ plans, int cmpx, int cmpy,
-	const SearchState* __restrict__ st, float* __restrict__ ctfmap)
-{
-	const SearchState& S = st[blockIdx.y];
-	if (S.skip) return;
-	const CtfConsts cc = plans[blockIdx.y].cc;
-	const int y = blockIdx.x;
-	float ph_rad = S.phase * kD2R2D, az = S.ang * kD2R2D;
-	float dmin = S.dfmean * (1.0f - S.ast) / cc.pix;
-	float dmax = S.dfmean * (1.0f + S.ast) / cc.pix;
-	float mean = 0.5f * (dmin + dmax), sig = 0.5f * (dmax - dmin);
-	float add = cc.amp_phase + ph_rad;
-	float w2 = cc.wl * cc.wl;
-	float* out = ctfmap + ((long long)blockIdx.y * cmpy + y) * cmpx;
-	const float fY = (float)(y - cmpy / 2) / (float)cmpy;
-	for (int x = threadIdx.x; x < cmpx; x += 256) {
-		float fX = (float)x * 0.5f / (float)(cmpx - 1);
-		float s2 = fX * fX + fY * fY;
-		float th = atanf(fY / (fX + (float)1e-30));
-		float df = mean + sig * cosf(2.0f * (th - az));
-		out[x] = -sinf(add + kPi2D * cc.wl * s2 * (df - 0.5f * s2 * w2 * cc.cs));
-	}
-}
-
-// Spectral CC shells (GSpectralCC2D.cu:12-109): Pearson CC of CTF and
-// spectrum over the pixels with lo <= |(x, y - cmpy/2)| < hi of each shell
-// (width 10, clamped at the ends).  The shell bounds are integers, so a
-// pixel with radius fr belongs to shell [lo, hi) exactly when
-// lo <= floor(fr) < hi: the six sums of each integer radius bin are formed
-// once (k_shell_bins, from a host table listing the pixels of every bin,
-// radii in the kernel's float arithmetic), and each shell adds its bins.
+// Spectral CC shells (GSpectralCC2D.cu:12-109): Pearson CC of the CTF at the
+// final parameters and the spectrum over the pixels with lo <= |(x, y -
+// cmpy/2)| < hi of each shell (width 10, clamped at the ends).  The shell
+// bounds are integers, so a pixel with radius fr belongs to shell [lo, hi)
+// exactly when lo <= floor(fr) < hi: the six sums of each integer radius bin
+// are formed once (k_shell_bins, from a host table listing the pixels of
+// every bin, radii in the kernel's float arithmetic), and each shell adds
+// its bins.  A pixel is in one bin, so its CTF (FP32, the reference formula,
+// GCalcCTF2D.cu:23-37) is formed where it is summed.
 // Grid (nbins, images), one wavefront per bin; bins[image][bin][6].
-__global__ __launch_bounds__(64) void k_shell_bins(const float* __restrict__ spect,
-	const float* __restrict__ ctfmap, int npix, const int* __restrict__ boff, const int* __restrict__ bcnt,
+__global__ __launch_bounds__(64) void k_shell_bins(const ImgPlan* __restrict__ plans, const float* __restrict__ spect,
+	int cmpx, int cmpy, const int* __restrict__ boff, const int* __restrict__ bcnt,
 	const int* __restrict__ bidx, int nbins, const SearchState* __restrict__ st, double* __restrict__ bins)
 {
 	const int b = blockIdx.x, img = blockIdx.y;
-	if (st[img].skip) return;
-	const float* sp = spect + (long long)img * npix;
-	const float* cm = ctfmap + (long long)img * npix;
+	const SearchState& S = st[img];
+	if (S.skip) return;
+	const CtfConsts cc = plans[img].cc;
+	const float ph_rad = S.phase * kD2R2D, az = S.ang * kD2R2D;
+	const float dmin = S.dfmean * (1.0f - S.ast) / cc.pix;
+	const float dmax = S.dfmean * (1.0f + S.ast) / cc.pix;
+	const float mean = 0.5f * (dmin + dmax), sig = 0.5f * (dmax - dmin);
+	const float add = cc.amp_phase + ph_rad;
+	const float w2 = cc.wl * cc.wl;
+	const float* sp = spect + (long long)img * cmpx * cmpy;
 	const int o = boff[b], n = bcnt[b];
 	double a[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 4
 	for (int i = threadIdx.x; i < n; i += 64) {
 		const int p = bidx[o + i];
-		const float c = cm[p], sv = sp[p];
+		const int y = p / cmpx, x = p - y * cmpx;
+		const float fY = (float)(y - cmpy / 2) / (float)cmpy;
+		const float fX = (float)x * 0.5f / (float)(cmpx - 1);
+		const float s2 = fX * fX + fY * fY;
+		const float th = atanf(fY / (fX + (float)1e-30));
+		const float df = mean + sig * cosf(2.0f * (th - az));
+		const float c = -sinf(add + kPi2D * cc.wl * s2 * (df - 0.5f * s2 * w2 * cc.cs));
+		const float sv = sp[p];
 		a[0] += c; a[1] += sv; a[2] += (double)c * sv; a[3] += (double)c * c; a[4] += (double)sv * sv;
 	}
 	a[5] = (double)n;
@@ -818,52 +1009,64 @@ __global__ __launch_bounds__(64) void k_shell_bins(const float* __restrict__ spe
 	if (threadIdx.x < 6) bins[((long long)img * nbins + b) * 6 + threadIdx.x] = a[threadIdx.x];
 }
 
-// Shell k = the bins [lo, hi); grid (ceil(cmpx / 64), images).
-__global__ __launch_bounds__(64) void k_shell_cc(const double* __restrict__ bins, int nbins, int cmpx, int width,
-	const SearchState* __restrict__ st, float* __restrict__ shell_cc)
+// Shell k = the bins [lo, hi), then GSpectralCC2D::DoIt's shell pick
+// (:157-171) and m_fCtfRes (CFindDefocus2D.cpp:399).  One workgroup per
+// micrograph, at most kShellMax shells and kShellBinMax radius bins (those of
+// the 1024 tile), the bins' sums staged in LDS.
+constexpr int kShellMax = 513, kShellBinMax = 726;
+__global__ __launch_bounds__(256) void k_ctf_res(const double* __restrict__ bins, int nbins, int cmpx, int cmpy,
+	int width, const ImgPlan* __restrict__ plans, SearchState* __restrict__ st)
 {
-	const int k = blockIdx.x * 64 + threadIdx.x, img = blockIdx.y;
-	if (k >= cmpx || st[img].skip) return;
-	int lo = k - width / 2, hi = lo + width;
-	if (lo < 0) { lo = 0; hi = width; }
-	else if (hi > cmpx) { lo = cmpx - width; hi = cmpx; }
-	double a[6] = {0, 0, 0, 0, 0, 0};
-	const double* bb = bins + (long long)img * nbins * 6;
-	for (int r = lo; r < hi && r < nbins; ++r)
+	__shared__ float cc[kShellMax];
+	__shared__ double bb[6 * kShellBinMax];
+	__shared__ int s_max, s_end;
+	const int img = blockIdx.x;
+	if (st[img].skip) return;
+	const double* gb = bins + (long long)img * nbins * 6;
+#pragma unroll 4
+	for (int i = threadIdx.x; i < nbins * 6; i += 256) bb[i] = gb[i];
+	__syncthreads();
+	for (int k = threadIdx.x; k < cmpx; k += 256) {
+		int lo = k - width / 2, hi = lo + width;
+		if (lo < 0) { lo = 0; hi = width; }
+		else if (hi > cmpx) { lo = cmpx - width; hi = cmpx; }
+		double a[6] = {0, 0, 0, 0, 0, 0};
+		for (int r = lo; r < hi && r < nbins; ++r)
 #pragma unroll
-		for (int j = 0; j < 6; ++j) a[j] += bb[r * 6 + j];
-	float out = 0.f;
-	const double n = a[5];
-	if (n > 0) {
-		double mc = a[0] / n, ms = a[1] / n, mcs = a[2] / n;
-		double vc = a[3] / n - mc * mc, vs = a[4] / n - ms * ms;
-		if (vc > 0 && vs > 0) out = (float)((mcs - mc * ms) / sqrt(vc * vs));
-	}
-	shell_cc[(long long)img * cmpx + k] = out;
-}
-
-// GSpectralCC2D::DoIt shell pick (:157-171) and m_fCtfRes (CFindDefocus2D.cpp:399).
-__global__ void k_ctf_res(const float* __restrict__ shell_cc, int cmpx, int cmpy,
-	const ImgPlan* __restrict__ plans, SearchState* __restrict__ st, int nimg)
-{
-	const int b = blockIdx.x * blockDim.x + threadIdx.x;
-	if (b >= nimg || st[b].skip) return;
-	const float pix = plans[b].cc.pix;
-	const float* cc = shell_cc + (long long)b * cmpx;
-	int imax = 1;
-	float fmax = (float)-1e30;
-	for (int i = 1; i < cmpx; ++i) {
-		if (cc[i] <= fmax) continue;
-		fmax = cc[i]; imax = i;
-	}
-	int shell = imax;
-	if (!(fmax < 0.143f)) {
-		for (int i = imax; i < cmpx; ++i) {
-			if (cc[i] < 0.143f) break;
-			shell = i;
+			for (int j = 0; j < 6; ++j) a[j] += bb[r * 6 + j];
+		float out = 0.f;
+		const double n = a[5];
+		if (n > 0) {
+			double mc = a[0] / n, ms = a[1] / n, mcs = a[2] / n;
+			double vc = a[3] / n - mc * mc, vs = a[4] / n - ms * ms;
+			if (vc > 0 && vs > 0) out = (float)((mcs - mc * ms) / sqrt(vc * vs));
 		}
+		cc[k] = out;
 	}
-	st[b].ctf_res = (float)cmpy * pix / (float)shell;
+	if (threadIdx.x == 0) s_end = cmpx;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		int imax = 1;
+		float fmax = (float)-1e30;
+#pragma unroll 8
+		for (int i = 1; i < cmpx; ++i) {
+			const float v = cc[i];
+			const bool up = !(v <= fmax);
+			fmax = up ? v : fmax;
+			imax = up ? i : imax;
+		}
+		s_max = fmax < 0.143f ? -imax : imax;
+	}
+	__syncthreads();
+	// the last shell before the first below 0.143 from the maximum on
+	const int imax = s_max;
+	for (int i = threadIdx.x; i < cmpx; i += 256)
+		if (i >= imax && cc[i] < 0.143f) atomicMin(&s_end, i);
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		const int shell = imax < 0 ? -imax : s_end - 1;
+		st[img].ctf_res = (float)cmpy * plans[img].cc.pix / (float)shell;
+	}
 }
 
 }  // namespace gctf

@@ -132,7 +132,7 @@ GCTF_API int gctf_refine(gctf_ctx* ctx, const float* df_mean, const float* ast_r
  * parameters of the last gctf_setup1 and the -ExtPhase values of
  * gctf_create; d_out gets n results in device memory.  Tile size 512 only.
  * Calls no hipMalloc/hipFree: its search buffers live in one static device
- * array per GPU (about 18 MB, held until the process ends), so calls that
+ * array per GPU (about 15 MB, held until the process ends), so calls that
  * overlap on one GPU, from any context, race.  Returns once the work is
  * enqueued on the context's stream (gctf_synchronize waits for it).
  * GCTF_ERR_ARG for n > 16; GCTF_ERR_STATE before gctf_setup1 or while
