@@ -1,14 +1,14 @@
 // gctf_net.hip -- forward, backward and optimiser kernels of the
 // defocus-proposal network, and the C-ABI of its trainer.
 //
-// All GEMM-shaped work (conv2-4 as im2col GEMMs, fc1, and their weight and
-// input gradients) goes through one MFMA kernel, k_gemm: 64 x 64 output
+// The BF16 path, which training, inference and the learned search take, is
+// k_net.hpp.  The kernels here keep the operands in FP32
+// (v_mfma_f32_32x32x2f32) for gradient checks: conv2-4 as im2col GEMMs, fc1,
+// and their weight and input gradients go through k_gemm: 64 x 64 output
 // tiles, 4 waves of 32 x 32, K staged through LDS 16 at a time, operands
-// read with arbitrary element strides (so transposes cost nothing),
-// converted to BF16 for v_mfma_f32_32x32x16_bf16 or kept in FP32 for
-// v_mfma_f32_32x32x2f32.  Long K (weight gradients over batch x length)
-// is split over workgroups and reduced in a fixed order, so training is
-// deterministic.
+// read with arbitrary element strides (so transposes cost nothing).  Long K
+// (weight gradients over batch x length) is split over workgroups and reduced
+// in a fixed order.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -19,11 +19,9 @@
 
 #include "../../include/gctf_hip.h"
 #include "gctf_net.hpp"
+#include "k_net.hpp"
 
 namespace gctf {
-
-typedef __bf16 nbf16x8 __attribute__((ext_vector_type(8)));
-typedef float nfloatx16 __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------
 // GEMM: C[m][n] = sum_k A(m, k) B(k, n) (+ beta C)
@@ -38,7 +36,6 @@ struct GemmArgs {
 	float* part;     // [split][M][N] when gridDim.z > 1
 };
 
-template <bool BF16>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
 {
 	__shared__ float sA[64][17];
@@ -61,20 +58,10 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
 			sB[kk][c] = (n < g.N && k < ke) ? g.B[(long long)k * g.sbk + (long long)n * g.sbn] : 0.f;
 		}
 		__syncthreads();
-		if constexpr (BF16) {
-			nbf16x8 a, b;
 #pragma unroll
-			for (int j = 0; j < 8; ++j) {
-				a[j] = (__bf16)sA[wm * 32 + row][8 * h + j];
-				b[j] = (__bf16)sB[8 * h + j][wn * 32 + row];
-			}
-			acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-		} else {
-#pragma unroll
-			for (int kk = 0; kk < 16; kk += 2)
-				acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sA[wm * 32 + row][kk + h], sB[kk + h][wn * 32 + row],
-					acc, 0, 0, 0);
-		}
+		for (int kk = 0; kk < 16; kk += 2)
+			acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sA[wm * 32 + row][kk + h], sB[kk + h][wn * 32 + row],
+				acc, 0, 0, 0);
 		__syncthreads();
 	}
 #pragma unroll
@@ -225,39 +212,13 @@ __global__ __launch_bounds__(256) void k_fc2(const float* __restrict__ h, const 
 	o[i] = s;
 }
 
-// Loss per spectrum and its gradient (divided by B).  target[b] =
-// (mean defocus A, astigmatism A, azimuth deg, confidence label).
-//   100 (o0 - ln(df / 1e4))^2 + 0.25 (o1 - ast / 1e3)^2
-//   + 0.05 (1 - cos 2 (o2 - az)) + 0.5 w BCE(sigmoid(o3), c)
-// The label is measured on the micrograph (whether the learned path's
-// narrowed search ended within 20 A of the full search): > 0 gives c = 1,
-// < 0 gives c = 0, and 0 (unlabelled) drops the confidence term (w = 0).
+// Loss per spectrum and its gradient (net_loss).
 __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ o, const float* __restrict__ tg, int B,
 	float* __restrict__ dO, double* __restrict__ lpart)
 {
 	const int b = blockIdx.x * 256 + threadIdx.x;
 	if (b >= B) return;
-	const float* ob = o + b * kNetOut;
-	const float* tb = tg + b * 4;
-	const float y0 = logf(tb[0] * 1.0e-4f), y1 = tb[1] * 1.0e-3f;
-	const float az = tb[2] * 0.017453292519943295f;
-	const float e0 = ob[0] - y0, e1 = ob[1] - y1;
-	const float d2 = 2.0f * (ob[2] - az);
-	const float c = tb[3] > 0.0f ? 1.0f : 0.0f;
-	const float w = tb[3] != 0.0f ? 1.0f : 0.0f;
-	const float x = ob[3];
-	// softplus forms of the log-sigmoid terms
-	const float sp_pos = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));   // -log(1 - p)
-	const float sp_neg = sp_pos - x;                                 // -log p
-	const float bce = c * sp_neg + (1.0f - c) * sp_pos;
-	const float p = 1.0f / (1.0f + expf(-x));
-	const float L = 100.0f * e0 * e0 + 0.25f * e1 * e1 + 0.05f * (1.0f - cosf(d2)) + 0.5f * w * bce;
-	const float inv = 1.0f / (float)B;
-	dO[b * kNetOut + 0] = 200.0f * e0 * inv;
-	dO[b * kNetOut + 1] = 0.5f * e1 * inv;
-	dO[b * kNetOut + 2] = 0.1f * sinf(d2) * inv;
-	dO[b * kNetOut + 3] = 0.5f * w * (p - c) * inv;
-	lpart[b] = (double)L;
+	lpart[b] = (double)net_loss(o + b * kNetOut, tg + b * 4, B, dO + b * kNetOut);
 }
 
 __global__ __launch_bounds__(256) void k_loss_sum(const double* __restrict__ lpart, int B, double* __restrict__ out)
@@ -410,6 +371,9 @@ struct NetBuffers {
 	float *dO = nullptr, *dh = nullptr, *dF = nullptr, *dA = nullptr, *dA2 = nullptr, *dZ = nullptr;
 	float *dcol = nullptr, *grad = nullptr, *part = nullptr;
 	double *lpart = nullptr, *loss = nullptr;
+	// BF16 path: weight fragments, activation signs
+	uint4* frag = nullptr;
+	unsigned char* sgn = nullptr;
 	long long part_cap = 0;
 };
 
@@ -431,22 +395,32 @@ hipError_t alloc_f(NetBuffers* b, float** p, long long n)
 		if (e_ != hipSuccess) return e_;           \
 	} while (0)
 
-hipError_t gemm(NetBuffers* nb, bool bf16, GemmArgs g, hipStream_t s)
+// K values per split (a multiple of 16) and splits of a GEMM's sums: long K is
+// split so that the grid has enough workgroups.
+struct KSplit {
+	int ksplit, splits;
+};
+KSplit gemm_splits(const NetBuffers* nb, int M, int N, int K)
 {
-	// split long K so that the grid has enough workgroups
-	const int tiles = ((g.N + 63) / 64) * ((g.M + 63) / 64);
+	const int tiles = ((N + 63) / 64) * ((M + 63) / 64);
 	int splits = 1;
-	if (tiles < 256 && g.K >= 128 && nb->part) {
+	if (tiles < 256 && K >= 128 && nb->part) {
 		// at least 64 K per split, enough workgroups to cover the chip
-		splits = std::min(g.K / 64, std::max(1, 512 / tiles));
-		while (splits > 1 && (long long)splits * g.M * g.N > nb->part_cap) --splits;
+		splits = std::min(K / 64, std::max(1, 512 / tiles));
+		while (splits > 1 && (long long)splits * M * N > nb->part_cap) --splits;
 	}
-	g.ksplit = ((g.K + splits - 1) / splits + 15) / 16 * 16;
-	splits = (g.K + g.ksplit - 1) / g.ksplit;
+	const int ksplit = ((K + splits - 1) / splits + 15) / 16 * 16;
+	return {ksplit, (K + ksplit - 1) / ksplit};
+}
+
+hipError_t gemm(NetBuffers* nb, GemmArgs g, hipStream_t s)
+{
+	const KSplit sp = gemm_splits(nb, g.M, g.N, g.K);
+	const int splits = sp.splits;
+	g.ksplit = sp.ksplit;
 	g.part = nb->part;
 	dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, splits);
-	if (bf16) k_gemm<true><<<grid, 256, 0, s>>>(g);
-	else k_gemm<false><<<grid, 256, 0, s>>>(g);
+	k_gemm<<<grid, 256, 0, s>>>(g);
 	if (splits > 1) {
 		const long long mn = (long long)g.M * g.N;
 		k_splitk_reduce<<<(unsigned)((mn + 255) / 256), 256, 0, s>>>(g.part, splits, g.M, g.N, g.C, g.scm, g.scn,
@@ -459,7 +433,7 @@ inline unsigned nblk(long long n) { return (unsigned)((n + 255) / 256); }
 
 // conv layer l (2..4) forward: input a_in [64][B L], im2col, GEMM, bias,
 // ReLU, pool into a_out [64][B L / 2]; y keeps the post-ReLU values.
-hipError_t conv_fwd(NetBuffers* nb, bool bf16, const float* prm, long long woff, long long boff,
+hipError_t conv_fwd(NetBuffers* nb, const float* prm, long long woff, long long boff,
 	const float* a_in, int B, int L, float* y, float* a_out, hipStream_t s)
 {
 	const long long BL = (long long)B * L;
@@ -469,26 +443,25 @@ hipError_t conv_fwd(NetBuffers* nb, bool bf16, const float* prm, long long woff,
 	g.A = prm + woff; g.sam = kNetCol; g.sak = 1;
 	g.B = nb->col; g.sbk = BL; g.sbn = 1;
 	g.C = y; g.scm = BL; g.scn = 1;
-	NETCHK(gemm(nb, bf16, g, s));
+	NETCHK(gemm(nb, g, s));
 	k_bias_relu_pool<<<dim3(nblk(BL / 2), kNetCh), 256, 0, s>>>(y, prm + boff, BL, a_out);
 	return hipGetLastError();
 }
 
-hipError_t forward_all(NetBuffers* nb, const float* prm, const float* radial, int ld, int B, bool bf16,
-	hipStream_t s)
+hipError_t forward_f32(NetBuffers* nb, const float* prm, const float* radial, int ld, int B, hipStream_t s)
 {
 	k_net_input<<<B, 256, 0, s>>>(radial, ld, nb->x0);
 	k_conv1_fwd<<<dim3(nblk((long long)B * kNetBins / 2), kNetCh), 256, 0, s>>>(nb->x0, prm, B, nb->y1, nb->a1);
-	NETCHK(conv_fwd(nb, bf16, prm, kNetW2, kNetB2, nb->a1, B, kNetBins / 2, nb->y2, nb->a2, s));
-	NETCHK(conv_fwd(nb, bf16, prm, kNetW3, kNetB3, nb->a2, B, kNetBins / 4, nb->y3, nb->a3, s));
-	NETCHK(conv_fwd(nb, bf16, prm, kNetW4, kNetB4, nb->a3, B, kNetBins / 8, nb->y4, nb->a4, s));
+	NETCHK(conv_fwd(nb, prm, kNetW2, kNetB2, nb->a1, B, kNetBins / 2, nb->y2, nb->a2, s));
+	NETCHK(conv_fwd(nb, prm, kNetW3, kNetB3, nb->a2, B, kNetBins / 4, nb->y3, nb->a3, s));
+	NETCHK(conv_fwd(nb, prm, kNetW4, kNetB4, nb->a3, B, kNetBins / 8, nb->y4, nb->a4, s));
 	k_flatten<<<nblk((long long)kNetFlat * B), 256, 0, s>>>(nb->a4, B, nb->f);
 	GemmArgs g{};
 	g.M = kNetHidden; g.N = B; g.K = kNetFlat;
 	g.A = prm + kNetW5; g.sam = kNetFlat; g.sak = 1;
 	g.B = nb->f; g.sbk = B; g.sbn = 1;
 	g.C = nb->h; g.scm = B; g.scn = 1;
-	NETCHK(gemm(nb, bf16, g, s));
+	NETCHK(gemm(nb, g, s));
 	k_bias_relu<<<nblk((long long)kNetHidden * B), 256, 0, s>>>(nb->h, prm + kNetB5, B);
 	k_fc2<<<nblk((long long)B * kNetOut), 256, 0, s>>>(nb->h, prm, B, nb->o);
 	return hipGetLastError();
@@ -496,7 +469,7 @@ hipError_t forward_all(NetBuffers* nb, const float* prm, const float* radial, in
 
 // conv layer backward: dA_out [64][B L / 2] -> grads of W, b and (when
 // dA_in) the layer input.
-hipError_t conv_back(NetBuffers* nb, bool bf16, const float* prm, long long woff, long long boff,
+hipError_t conv_back(NetBuffers* nb, const float* prm, long long woff, long long boff,
 	const float* a_in, const float* y, const float* dA_out, int B, int L, float* dA_in, hipStream_t s)
 {
 	const long long BL = (long long)B * L;
@@ -508,7 +481,7 @@ hipError_t conv_back(NetBuffers* nb, bool bf16, const float* prm, long long woff
 	g.A = nb->dZ; g.sam = BL; g.sak = 1;
 	g.B = nb->col; g.sbk = 1; g.sbn = BL;
 	g.C = nb->grad + woff; g.scm = kNetCol; g.scn = 1;
-	NETCHK(gemm(nb, bf16, g, s));
+	NETCHK(gemm(nb, g, s));
 	k_rowsum<<<kNetCh, 256, 0, s>>>(nb->dZ, BL, nb->grad + boff);
 	if (dA_in) {
 		GemmArgs d{};
@@ -516,13 +489,13 @@ hipError_t conv_back(NetBuffers* nb, bool bf16, const float* prm, long long woff
 		d.A = prm + woff; d.sam = 1; d.sak = kNetCol;
 		d.B = nb->dZ; d.sbk = BL; d.sbn = 1;
 		d.C = nb->dcol; d.scm = BL; d.scn = 1;
-		NETCHK(gemm(nb, bf16, d, s));
+		NETCHK(gemm(nb, d, s));
 		k_col2im<<<dim3(nblk(BL), kNetCh), 256, 0, s>>>(nb->dcol, B, L, dA_in);
 	}
 	return hipGetLastError();
 }
 
-hipError_t backward_all(NetBuffers* nb, const float* prm, const float* target, int B, bool bf16, hipStream_t s)
+hipError_t backward_f32(NetBuffers* nb, const float* prm, const float* target, int B, hipStream_t s)
 {
 	k_loss<<<nblk(B), 256, 0, s>>>(nb->o, target, B, nb->dO, nb->lpart);
 	k_loss_sum<<<1, 256, 0, s>>>(nb->lpart, B, nb->loss);
@@ -533,23 +506,115 @@ hipError_t backward_all(NetBuffers* nb, const float* prm, const float* target, i
 	g.A = nb->dh; g.sam = B; g.sak = 1;
 	g.B = nb->f; g.sbk = 1; g.sbn = B;
 	g.C = nb->grad + kNetW5; g.scm = kNetFlat; g.scn = 1;
-	NETCHK(gemm(nb, bf16, g, s));
+	NETCHK(gemm(nb, g, s));
 	k_rowsum<<<kNetHidden, 256, 0, s>>>(nb->dh, B, nb->grad + kNetB5);
 	GemmArgs d{};
 	d.M = kNetFlat; d.N = B; d.K = kNetHidden;
 	d.A = prm + kNetW5; d.sam = 1; d.sak = kNetFlat;
 	d.B = nb->dh; d.sbk = B; d.sbn = 1;
 	d.C = nb->dF; d.scm = B; d.scn = 1;
-	NETCHK(gemm(nb, bf16, d, s));
+	NETCHK(gemm(nb, d, s));
 	k_unflatten<<<nblk((long long)kNetFlat * B), 256, 0, s>>>(nb->dF, B, nb->dA);
 	// conv4: dA (pooled, [64][B 16]) -> dA2 ([64][B 32])
-	NETCHK(conv_back(nb, bf16, prm, kNetW4, kNetB4, nb->a3, nb->y4, nb->dA, B, kNetBins / 8, nb->dA2, s));
-	NETCHK(conv_back(nb, bf16, prm, kNetW3, kNetB3, nb->a2, nb->y3, nb->dA2, B, kNetBins / 4, nb->dA, s));
-	NETCHK(conv_back(nb, bf16, prm, kNetW2, kNetB2, nb->a1, nb->y2, nb->dA, B, kNetBins / 2, nb->dA2, s));
+	NETCHK(conv_back(nb, prm, kNetW4, kNetB4, nb->a3, nb->y4, nb->dA, B, kNetBins / 8, nb->dA2, s));
+	NETCHK(conv_back(nb, prm, kNetW3, kNetB3, nb->a2, nb->y3, nb->dA2, B, kNetBins / 4, nb->dA, s));
+	NETCHK(conv_back(nb, prm, kNetW2, kNetB2, nb->a1, nb->y2, nb->dA, B, kNetBins / 2, nb->dA2, s));
 	// conv1
 	const long long BL = (long long)B * kNetBins;
 	k_pool_relu_back<<<dim3(nblk(BL), kNetCh), 256, 0, s>>>(nb->y1, nb->dA2, BL, nb->dZ);
 	k_conv1_dw<<<kNetCh, 256, 0, s>>>(nb->dZ, nb->x0, B, nb->grad);
+	return hipGetLastError();
+}
+
+// ---- BF16 path -------------------------------------------------------------
+void launch_conv(NetBuffers* nb, const float* a, const uint4* frag, const float* bias, int B, int L, float* out,
+	unsigned char* sgn, hipStream_t s)
+{
+	// 128 positions per workgroup where that still fills the chip's 256 CUs, else 64
+	const int BL = B * L, spl = gemm_splits(nb, kNetCh, BL, kNetCol).ksplit / 16;
+	if (BL >= 128 * 256) k_net_conv<4><<<(BL + 127) / 128, 256, 0, s>>>(a, frag, bias, BL, L, spl, out, sgn);
+	else k_net_conv<2><<<(BL + 63) / 64, 128, 0, s>>>(a, frag, bias, BL, L, spl, out, sgn);
+}
+
+void launch_conv_back(const float* dP, const unsigned char* sin, const uint4* frag, int B, int L, float* out,
+	hipStream_t s)
+{
+	// 128 positions (a weight fragment serves two tiles) or 64, as above
+	const int BL = B * L;
+	if (BL >= 128 * 256) k_net_conv_back<2><<<(BL + 127) / 128, 256, 0, s>>>(dP, sin, frag, BL, L, out);
+	else k_net_conv_back<1><<<(BL + 63) / 64, 256, 0, s>>>(dP, sin, frag, BL, L, out);
+}
+
+// Signs of layer l's activations (0: conv1 .. 3: conv4), pooled length 128 >> l.
+unsigned char* layer_signs(NetBuffers* nb, int B, int l)
+{
+	unsigned char* p = nb->sgn;
+	for (int i = 0; i < l; ++i) p += (long long)kNetCh * B * (kNetBins / 2 >> i);
+	return p;
+}
+
+// The forward pass; with target the loss and the gradients up to conv4's
+// pooled output.
+hipError_t forward_bf16(NetBuffers* nb, const float* prm, const float* radial, int ld, int B, const float* target,
+	hipStream_t s)
+{
+	const bool tr = target != nullptr;
+	auto sg = [&](int l) { return tr ? layer_signs(nb, B, l) : nullptr; };
+	k_net_weights<<<((tr ? kFragTotal : kFragFc1Back) + 3) / 4, 256, 0, s>>>(prm, tr ? 1 : 0, nb->frag);
+	k_net_front<<<B, 256, 0, s>>>(radial, ld, prm, B, nb->x0, nb->a1, sg(0));
+	const uint4* fr = nb->frag;
+	const long long layer = 2LL * kFragConv * 64;
+	launch_conv(nb, nb->a1, fr, prm + kNetB2, B, kNetBins / 2, nb->a2, sg(1), s);
+	launch_conv(nb, nb->a2, fr + layer, prm + kNetB3, B, kNetBins / 4, nb->a3, sg(2), s);
+	launch_conv(nb, nb->a3, fr + 2 * layer, prm + kNetB4, B, kNetBins / 8, nb->a4, sg(3), s);
+	k_net_fc<<<(B + 31) / 32, 1024, 0, s>>>(nb->a4, fr, prm, B, gemm_splits(nb, kNetHidden, B, kNetFlat).ksplit / 16,
+		gemm_splits(nb, kNetFlat, B, kNetHidden).ksplit / 16, nb->o, target, nb->h, nb->dO, nb->lpart, nb->dh,
+		nb->dF);
+	return hipGetLastError();
+}
+
+// After forward_bf16 with a target.  Pooled-output gradients: conv4 dF,
+// conv3 dZ, conv2 dA, conv1 dA2.
+hipError_t backward_bf16(NetBuffers* nb, int B, hipStream_t s)
+{
+	const uint4* fr = nb->frag;
+	const long long layer = 2LL * kFragConv * 64, back = (long long)kFragConv * 64;
+	launch_conv_back(nb->dF, layer_signs(nb, B, 3), fr + 2 * layer + back, B, kNetBins / 8, nb->dZ, s);
+	launch_conv_back(nb->dZ, layer_signs(nb, B, 2), fr + layer + back, B, kNetBins / 4, nb->dA, s);
+	launch_conv_back(nb->dA, layer_signs(nb, B, 1), fr + back, B, kNetBins / 2, nb->dA2, s);
+	NetDwArgs g{};
+	g.B = B;
+	const float* in[3] = {nb->a1, nb->a2, nb->a3};
+	const float* da[3] = {nb->dA, nb->dZ, nb->dF};
+	float* p = nb->part;
+	int items = 0;
+	for (int l = 0; l < 3; ++l) {
+		g.L[l] = kNetBins / 2 >> l;
+		const KSplit sp = gemm_splits(nb, kNetCh, kNetCol, B * g.L[l]);
+		g.ksplit[l] = sp.ksplit;
+		g.splits[l] = sp.splits;
+		g.a[l] = in[l];
+		g.dA[l] = da[l];
+		g.sgn[l] = layer_signs(nb, B, l + 1);
+		g.part[l] = p;
+		p += (long long)sp.splits * kNetCh * kNetCol;
+		g.first[l] = items;
+		items += sp.splits;
+	}
+	g.x0 = nb->x0; g.dA1 = nb->dA2; g.m1 = layer_signs(nb, B, 0);
+	g.a4 = nb->a4; g.dh = nb->dh; g.h = nb->h; g.dO = nb->dO; g.lpart = nb->lpart;
+	g.ksplit5 = gemm_splits(nb, kNetHidden, kNetFlat, B).ksplit;
+	g.grad = nb->grad; g.loss = nb->loss;
+	g.first[3] = items;
+	items += kNetCh;
+	g.first[4] = items;
+	items += 3 * kNetCh;
+	g.first[5] = items;
+	items += (kNetHidden / 32) * (kNetFlat / 32);
+	g.first[6] = items;
+	items += kNetHidden / 8;
+	k_net_dw<<<items, 256, 0, s>>>(g);
+	k_net_dw_reduce<<<nblk(3LL * kNetCh * kNetCol), 256, 0, s>>>(g);
 	return hipGetLastError();
 }
 
@@ -580,8 +645,17 @@ hipError_t net_buffers_create(int max_batch, bool train, NetBuffers** out)
 	A(&nb->o, kNetOut * B);
 	// split-K partials of the GEMMs (forward and backward)
 	nb->part_cap = std::max<long long>(1LL << 20, (long long)kNetCh * B * L * 2);
-	A(&nb->part, nb->part_cap);
+	// the BF16 path keeps the partials of three layers' weights (64 x 448, at
+	// most 512 / 7 splits each) at once
+	const long long dw = 3 * std::min<long long>(nb->part_cap, (512LL / 7) * kNetCh * kNetCol);
+	A(&nb->part, std::max(nb->part_cap, dw));
+	float* fr = nullptr;
+	A(&fr, 4LL * 64 * kFragTotal);
+	nb->frag = (uint4*)fr;
 	if (train) {
+		float* sg = nullptr;
+		A(&sg, kNetCh * B * (L / 2 + L / 4 + L / 8 + L / 16) / 4);
+		nb->sgn = (unsigned char*)sg;
 		A(&nb->dO, kNetOut * B);
 		A(&nb->dh, kNetHidden * B);
 		A(&nb->dF, kNetFlat * B);
@@ -618,7 +692,8 @@ hipError_t net_forward(NetBuffers* b, const float* params, const float* radial, 
 	float* out, hipStream_t s)
 {
 	if (!b || n < 1 || n > b->cap || ld < kNetBins) return hipErrorInvalidValue;
-	NETCHK(forward_all(b, params, radial, ld, n, bf16, s));
+	if (bf16) NETCHK(forward_bf16(b, params, radial, ld, n, nullptr, s));
+	else NETCHK(forward_f32(b, params, radial, ld, n, s));
 	return hipMemcpyAsync(out, b->o, sizeof(float) * kNetOut * n, hipMemcpyDeviceToDevice, s);
 }
 
@@ -726,7 +801,8 @@ int gctf_net_forward(gctf_net* n, const float* d_radial, int ld, int count, int 
 	if (count < 1 || count > n->nb->cap) return net_fail(n, GCTF_ERR_ARG, "batch exceeds the network capacity");
 	if (ld < kNetBins) return net_fail(n, GCTF_ERR_ARG, "radial row shorter than 256 bins");
 	NETHIP(n, hipSetDevice(n->device));
-	NETHIP(n, forward_all(n->nb, n->params, d_radial, ld, count, bf16 != 0, n->stream));
+	NETHIP(n, bf16 ? forward_bf16(n->nb, n->params, d_radial, ld, count, nullptr, n->stream)
+		: forward_f32(n->nb, n->params, d_radial, ld, count, n->stream));
 	NETHIP(n, hipMemcpyAsync(host_out, n->nb->o, sizeof(float) * kNetOut * count, hipMemcpyDeviceToHost,
 		n->stream));
 	NETHIP(n, hipStreamSynchronize(n->stream));
@@ -740,8 +816,13 @@ int gctf_net_loss_grad(gctf_net* n, const float* d_radial, int ld, const float* 
 	if (count < 1 || count > n->nb->cap) return net_fail(n, GCTF_ERR_ARG, "batch exceeds the network capacity");
 	if (ld < kNetBins) return net_fail(n, GCTF_ERR_ARG, "radial row shorter than 256 bins");
 	NETHIP(n, hipSetDevice(n->device));
-	NETHIP(n, forward_all(n->nb, n->params, d_radial, ld, count, bf16 != 0, n->stream));
-	NETHIP(n, backward_all(n->nb, n->params, d_target, count, bf16 != 0, n->stream));
+	if (bf16) {
+		NETHIP(n, forward_bf16(n->nb, n->params, d_radial, ld, count, d_target, n->stream));
+		NETHIP(n, backward_bf16(n->nb, count, n->stream));
+	} else {
+		NETHIP(n, forward_f32(n->nb, n->params, d_radial, ld, count, n->stream));
+		NETHIP(n, backward_f32(n->nb, n->params, d_target, count, n->stream));
+	}
 	if (loss) NETHIP(n, hipMemcpyAsync(loss, n->nb->loss, sizeof(double), hipMemcpyDeviceToHost, n->stream));
 	if (host_grad)
 		NETHIP(n, hipMemcpyAsync(host_grad, n->nb->grad, sizeof(float) * kNetParams, hipMemcpyDeviceToHost,
