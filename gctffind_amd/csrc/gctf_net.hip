@@ -527,22 +527,37 @@ hipError_t backward_f32(NetBuffers* nb, const float* prm, const float* target, i
 }
 
 // ---- BF16 path -------------------------------------------------------------
-void launch_conv(NetBuffers* nb, const float* a, const uint4* frag, const float* bias, int B, int L, float* out,
+template <int L>
+void launch_conv(NetBuffers* nb, const float* a, const uint4* frag, const float* bias, int B, float* out,
 	unsigned char* sgn, hipStream_t s)
 {
-	// 128 positions per workgroup where that still fills the chip's 256 CUs, else 64
 	const int BL = B * L, spl = gemm_splits(nb, kNetCh, BL, kNetCol).ksplit / 16;
-	if (BL >= 128 * 256) k_net_conv<4><<<(BL + 127) / 128, 256, 0, s>>>(a, frag, bias, BL, L, spl, out, sgn);
-	else k_net_conv<2><<<(BL + 63) / 64, 128, 0, s>>>(a, frag, bias, BL, L, spl, out, sgn);
+	auto go = [&](auto n) {
+		k_net_conv<2, decltype(n)::value, L><<<(BL + 63) / 64, 256, 0, s>>>(a, frag, bias, BL, out, sgn);
+	};
+	// 28 slices in 1 to 7 splits; 128 positions per workgroup where that still
+	// fills the chip's 256 CUs (such a layer has one split), else 64
+	switch (spl) {
+	case 28:
+		if (BL >= 128 * 256) k_net_conv<4, 28, L><<<(BL + 127) / 128, 256, 0, s>>>(a, frag, bias, BL, out, sgn);
+		else go(std::integral_constant<int, 28>{});
+		return;
+	case 14: go(std::integral_constant<int, 14>{}); return;
+	case 10: go(std::integral_constant<int, 10>{}); return;
+	case 7: go(std::integral_constant<int, 7>{}); return;
+	case 6: go(std::integral_constant<int, 6>{}); return;
+	case 5: go(std::integral_constant<int, 5>{}); return;
+	default: go(std::integral_constant<int, 4>{}); return;
+	}
 }
 
-void launch_conv_back(const float* dP, const unsigned char* sin, const uint4* frag, int B, int L, float* out,
-	hipStream_t s)
+template <int L>
+void launch_conv_back(const float* dP, const unsigned char* sin, const uint4* frag, int B, float* out, hipStream_t s)
 {
 	// 128 positions (a weight fragment serves two tiles) or 64, as above
 	const int BL = B * L;
-	if (BL >= 128 * 256) k_net_conv_back<2><<<(BL + 127) / 128, 256, 0, s>>>(dP, sin, frag, BL, L, out);
-	else k_net_conv_back<1><<<(BL + 63) / 64, 256, 0, s>>>(dP, sin, frag, BL, L, out);
+	if (BL >= 128 * 256) k_net_conv_back<2, L><<<(BL + 127) / 128, 256, 0, s>>>(dP, sin, frag, BL, out);
+	else k_net_conv_back<1, L><<<(BL + 63) / 64, 256, 0, s>>>(dP, sin, frag, BL, out);
 }
 
 // Signs of layer l's activations (0: conv1 .. 3: conv4), pooled length 128 >> l.
@@ -564,9 +579,9 @@ hipError_t forward_bf16(NetBuffers* nb, const float* prm, const float* radial, i
 	k_net_front<<<B, 256, 0, s>>>(radial, ld, prm, B, nb->x0, nb->a1, sg(0));
 	const uint4* fr = nb->frag;
 	const long long layer = 2LL * kFragConv * 64;
-	launch_conv(nb, nb->a1, fr, prm + kNetB2, B, kNetBins / 2, nb->a2, sg(1), s);
-	launch_conv(nb, nb->a2, fr + layer, prm + kNetB3, B, kNetBins / 4, nb->a3, sg(2), s);
-	launch_conv(nb, nb->a3, fr + 2 * layer, prm + kNetB4, B, kNetBins / 8, nb->a4, sg(3), s);
+	launch_conv<kNetBins / 2>(nb, nb->a1, fr, prm + kNetB2, B, nb->a2, sg(1), s);
+	launch_conv<kNetBins / 4>(nb, nb->a2, fr + layer, prm + kNetB3, B, nb->a3, sg(2), s);
+	launch_conv<kNetBins / 8>(nb, nb->a3, fr + 2 * layer, prm + kNetB4, B, nb->a4, sg(3), s);
 	k_net_fc<<<(B + 31) / 32, 1024, 0, s>>>(nb->a4, fr, prm, B, gemm_splits(nb, kNetHidden, B, kNetFlat).ksplit / 16,
 		gemm_splits(nb, kNetFlat, B, kNetHidden).ksplit / 16, nb->o, target, nb->h, nb->dO, nb->lpart, nb->dh,
 		nb->dF);
@@ -579,9 +594,9 @@ hipError_t backward_bf16(NetBuffers* nb, int B, hipStream_t s)
 {
 	const uint4* fr = nb->frag;
 	const long long layer = 2LL * kFragConv * 64, back = (long long)kFragConv * 64;
-	launch_conv_back(nb->dF, layer_signs(nb, B, 3), fr + 2 * layer + back, B, kNetBins / 8, nb->dZ, s);
-	launch_conv_back(nb->dZ, layer_signs(nb, B, 2), fr + layer + back, B, kNetBins / 4, nb->dA, s);
-	launch_conv_back(nb->dA, layer_signs(nb, B, 1), fr + back, B, kNetBins / 2, nb->dA2, s);
+	launch_conv_back<kNetBins / 8>(nb->dF, layer_signs(nb, B, 3), fr + 2 * layer + back, B, nb->dZ, s);
+	launch_conv_back<kNetBins / 4>(nb->dZ, layer_signs(nb, B, 2), fr + layer + back, B, nb->dA, s);
+	launch_conv_back<kNetBins / 2>(nb->dA, layer_signs(nb, B, 1), fr + back, B, nb->dA2, s);
 	NetDwArgs g{};
 	g.B = B;
 	const float* in[3] = {nb->a1, nb->a2, nb->a3};
@@ -589,8 +604,7 @@ hipError_t backward_bf16(NetBuffers* nb, int B, hipStream_t s)
 	float* p = nb->part;
 	int items = 0;
 	for (int l = 0; l < 3; ++l) {
-		g.L[l] = kNetBins / 2 >> l;
-		const KSplit sp = gemm_splits(nb, kNetCh, kNetCol, B * g.L[l]);
+		const KSplit sp = gemm_splits(nb, kNetCh, kNetCol, B * (kNetBins / 2 >> l));
 		g.ksplit[l] = sp.ksplit;
 		g.splits[l] = sp.splits;
 		g.a[l] = in[l];

@@ -112,7 +112,10 @@ __global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ rad
 {
 	__shared__ double r1[256], r2[256];
 	__shared__ float xs[kNetBins + 8];
+	__shared__ float ws[kNetCh * (kNetTaps + 1)];         // weights, then biases
 	const int b = blockIdx.x, t = threadIdx.x;
+	for (int i = t; i < kNetCh * (kNetTaps + 1); i += 256) ws[i] = prm[kNetW1 + i];
+	static_assert(kNetB1 == kNetW1 + kNetCh * kNetTaps, "weights and biases are neighbours");
 	const float v = radial[(long long)b * ld + t];
 	const bool use = t >= kNetBin0;
 	r1[t] = use ? (double)v : 0.0;
@@ -136,13 +139,14 @@ __global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ rad
 	float win[kNetTaps + 1];
 #pragma unroll
 	for (int i = 0; i <= kNetTaps; ++i) win[i] = xs[2 * p + i];
-	const int c0 = __builtin_amdgcn_readfirstlane(t / L2);
+	const int c0 = t / L2;
+#pragma unroll 4
 	for (int c = c0; c < kNetCh; c += 2) {
-		const float* w = prm + kNetW1 + c * kNetTaps;
+		const float* w = ws + c * kNetTaps;
 		float y[2];
 #pragma unroll
 		for (int q = 0; q < 2; ++q) {
-			float z = prm[kNetB1 + c];
+			float z = ws[kNetCh * kNetTaps + c];
 #pragma unroll
 			for (int i = 0; i < kNetTaps; ++i) z = fmaf(w[i], win[i + q], z);
 			y[q] = fmaxf(z, 0.f);
@@ -157,26 +161,32 @@ __global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ rad
 // A 64 -> 64 channel, 7-tap convolution over rows of length L (zero padding
 // 3) as an implicit GEMM, K = 7 channel + tap: input a [64][B L], output bias +
 // ReLU + pool in out [64][B L / 2], the signs in sgn (when not null).  A
-// workgroup takes 32 NW positions and a wave 64 channels x 32 of them, so that
-// an input fragment serves two MFMAs.  LDS holds a channel's positions in a
+// workgroup takes 128 positions, a wave 64 channels x 32 of them (an input
+// fragment serves two MFMAs), or 64 positions and 32 x 32.  LDS holds a channel's positions in a
 // row (each row segment with its halo of 3 on either side): the taps of a
 // position are neighbours, and 8 consecutive k are at most two runs, at
 // addresses that are constants but for the lane's half: k + 8 is the next
 // channel's next tap, or the channel's after that first one.
-// A sum of K is formed in splits of `spl` slices of 16 (gemm_splits).
+// A sum of K is formed in splits of SPL slices of 16 (gemm_splits), a template
+// parameter: with a runtime count each slice ended in a branch, and its weight
+// fragments were loaded where they were used, 24 us for any batch.
 // ---------------------------------------------------------------------------
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_net_conv(const float* __restrict__ a, const uint4* __restrict__ frag,
-	const float* __restrict__ bias, int BL, int L, int spl, float* __restrict__ out, unsigned char* __restrict__ sgn)
+template <int NW, int SPL, int L>
+__global__ __launch_bounds__(256) void k_net_conv(const float* __restrict__ a, const uint4* __restrict__ frag,
+	const float* __restrict__ bias, int BL, float* __restrict__ out, unsigned char* __restrict__ sgn)
 {
-	constexpr int TN = 32 * NW, NT = 64 * NW;
-	constexpr int PT = TN + 6 * NW + 2;                  // segments are at least 32 long
+	constexpr int TN = 32 * NW;
+	constexpr int MW = NW == 4 ? 2 : 1;                  // 32-channel tiles per wave
+	constexpr int seg = L < TN ? L : TN, pitch = seg + 6, pairs = TN / seg * (pitch / 2);
+	constexpr int PT = 2 * pairs + 2;
 	__shared__ __attribute__((aligned(16))) unsigned short xs[kNetCh * PT];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int row = lane & 31, h = lane >> 5;
 	const int q0 = blockIdx.x * TN;
-	const int seg = min(L, TN), pitch = seg + 6, pairs = (TN / seg) * (pitch / 2);
-	for (int i = tid; i < pairs * kNetCh; i += NT) {
+	const int m0 = NW == 4 ? 0 : wave >> 1;
+	// the loads of 6 passes over the tile in flight at once
+#pragma unroll 6
+	for (int i = tid; i < pairs * kNetCh; i += 256) {
 		const int ci = i / pairs, r = (i - ci * pairs) * 2;
 		const int sg = r / pitch, o = r - sg * pitch - 3;
 		const int qs = q0 + sg * seg;
@@ -190,20 +200,28 @@ __global__ __launch_bounds__(64 * NW) void k_net_conv(const float* __restrict__ 
 		}
 		*reinterpret_cast<unsigned int*>(xs + ci * PT + r) = pack_bf16(v[0], v[1]);
 	}
-	__syncthreads();
-	const int p = wave * 32 + row;                        // position in the tile
+	const int p = (NW == 4 ? wave : wave & 1) * 32 + row; // position in the tile
 	const int sg = p / seg;
 	const unsigned short* base = xs + sg * pitch + p - sg * seg;
 	const unsigned short* b1 = base + h * (PT + 1);       // k + 8 one channel and one tap on
 	const unsigned short* b2 = base + h * (2 * PT - 6);   // from tap 6: two channels on, tap 0
-	nfloatx16 acc[2], tot[2];
+	nfloatx16 acc[MW], tot[MW];
 #pragma unroll
-	for (int m = 0; m < 2; ++m)
+	for (int m = 0; m < MW; ++m)
 #pragma unroll
 		for (int r = 0; r < 16; ++r) { acc[m][r] = 0.f; tot[m][r] = 0.f; }
-	int left = spl;
+	// weight fragments of G slices ahead
+	constexpr int G = 4;
+	static_assert(kConvSlices % G == 0, "whole groups of slices");
+	nbf16x8 wc[MW * G], wx[MW * G];
+#pragma unroll
+	for (int i = 0; i < MW * G; ++i) wc[i] = load_frag(frag, i / MW * 2 + m0 + i % MW, lane);
+	__syncthreads();
 #pragma unroll
 	for (int s = 0; s < kConvSlices; ++s) {
+		if (s % G == 0 && s + G < kConvSlices)
+#pragma unroll
+			for (int i = 0; i < MW * G; ++i) wx[i] = load_frag(frag, (s + G + i / MW) * 2 + m0 + i % MW, lane);
 		unsigned int u[4];
 #pragma unroll
 		for (int j = 0; j < 8; ++j) {
@@ -214,22 +232,24 @@ __global__ __launch_bounds__(64 * NW) void k_net_conv(const float* __restrict__ 
 		}
 		const nbf16x8 x = __builtin_bit_cast(nbf16x8, make_uint4(u[0], u[1], u[2], u[3]));
 #pragma unroll
-		for (int m = 0; m < 2; ++m)
-			acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_frag(frag, s * 2 + m, lane), x, acc[m], 0, 0, 0);
-		if (--left == 0 || s == kConvSlices - 1) {
-			left = spl;
+		for (int m = 0; m < MW; ++m)
+			acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wc[MW * (s % G) + m], x, acc[m], 0, 0, 0);
+		if (s % G == G - 1)
 #pragma unroll
-			for (int m = 0; m < 2; ++m)
+			for (int i = 0; i < MW * G; ++i) wc[i] = wx[i];
+		if ((s + 1) % SPL == 0 || s == kConvSlices - 1) {
+#pragma unroll
+			for (int m = 0; m < MW; ++m)
 #pragma unroll
 				for (int r = 0; r < 16; ++r) { tot[m][r] += acc[m][r]; acc[m][r] = 0.f; }
 		}
 	}
 	const int q = q0 + p;
 #pragma unroll
-	for (int m = 0; m < 2; ++m)
+	for (int m = 0; m < MW; ++m)
 #pragma unroll
 		for (int r = 0; r < 16; ++r) {
-			const int c = 32 * m + mfma_row(r, h);
+			const int c = 32 * (m0 + m) + mfma_row(r, h);
 			const float y = fmaxf(tot[m][r] + bias[c], 0.f);
 			const float y1 = __shfl_xor(y, 1);
 			if ((lane & 1) == 0 && q < BL) {
@@ -249,18 +269,18 @@ __global__ __launch_bounds__(64 * NW) void k_net_conv(const float* __restrict__ 
 // that spread over all banks.
 constexpr int kConvPitch = kNetCh + 8;
 
-template <int NS>
+template <int NS, int L>
 __global__ __launch_bounds__(256) void k_net_conv_back(const float* __restrict__ dP,
-	const unsigned char* __restrict__ sin, const uint4* __restrict__ frag, int BL, int L, float* __restrict__ out)
+	const unsigned char* __restrict__ sin, const uint4* __restrict__ frag, int BL, float* __restrict__ out)
 {
 	constexpr int TN = 64 * NS;
-	constexpr int MAXROWS = TN + 6 * (TN / 32);          // segments are at least 32 long
-	__shared__ __attribute__((aligned(16))) __bf16 xs[MAXROWS * kConvPitch];
+	constexpr int seg = L < TN ? L : TN, pitch = seg + 6, rows = TN / seg * pitch;
+	__shared__ __attribute__((aligned(16))) __bf16 xs[rows * kConvPitch];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int row = lane & 31, h = lane >> 5;
 	const int mt = wave >> 1, wn = wave & 1;
 	const int q0 = blockIdx.x * TN;
-	const int seg = min(L, TN), pitch = seg + 6, rows = (TN / seg) * pitch;
+#pragma unroll 2
 	for (int i = tid; i < rows * (kNetCh / 8); i += 256) {
 		const int cg = i / rows, r = i - cg * rows;
 		const int sg = r / pitch, o = r - sg * pitch - 3;
@@ -365,11 +385,14 @@ __global__ __launch_bounds__(1024) void k_net_fc(const float* __restrict__ a4, c
 	constexpr int NB = 32, LD = NB + 1, HP = kNetHidden + 8;
 	__shared__ float hs[kNetHidden * LD];
 	__shared__ float os[NB][kNetOut], ds[NB][kNetOut];
+	__shared__ float w6[kNetOut * (kNetHidden + 1)];        // fc2's weights, then its biases
+	static_assert(kNetB6 == kNetW6 + kNetOut * kNetHidden, "weights and biases are neighbours");
 	__shared__ __attribute__((aligned(16))) __bf16 dhs[NB * HP];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int row = lane & 31, hf = lane >> 5;
 	const int b0 = blockIdx.x * NB;
 	const int bl = min(b0 + row, B - 1);
+	if (tid < kNetOut * (kNetHidden + 1)) w6[tid] = prm[kNetW6 + tid];
 	{
 		// quarter ks of the slices to wave group ks, where it holds whole
 		// splits (batches up to 4096); else group 0 takes them all
@@ -433,9 +456,9 @@ __global__ __launch_bounds__(1024) void k_net_fc(const float* __restrict__ a4, c
 	__syncthreads();
 	if (tid < NB * kNetOut) {
 		const int k = tid / NB, b = tid % NB;
-		const float* w = prm + kNetW6 + k * kNetHidden;
-		float s = prm[kNetB6 + k];
-#pragma unroll 8
+		const float* w = w6 + k * kNetHidden;
+		float s = w6[kNetOut * kNetHidden + k];
+#pragma unroll 16
 		for (int j = 0; j < kNetHidden; ++j) s = fmaf(w[j], hs[j * LD + b], s);
 		os[b][k] = s;
 		if (b0 + b < B) o[(long long)(b0 + b) * kNetOut + k] = s;
@@ -456,7 +479,7 @@ __global__ __launch_bounds__(1024) void k_net_fc(const float* __restrict__ a4, c
 		const int j = i / NB, b = i % NB;
 		float s = 0.f;
 #pragma unroll
-		for (int k = 0; k < kNetOut; ++k) s = fmaf(prm[kNetW6 + k * kNetHidden + j], ds[b][k], s);
+		for (int k = 0; k < kNetOut; ++k) s = fmaf(w6[k * kNetHidden + j], ds[b][k], s);
 		s = hs[j * LD + b] > 0.f ? s : 0.f;
 		if (b0 + b < B) dh[(long long)j * B + b0 + b] = s;
 		dhs[b * HP + j] = (__bf16)s;
@@ -500,7 +523,7 @@ struct NetDwArgs {
 	const float* a[3];
 	const float* dA[3];
 	const unsigned char* sgn[3];
-	int L[3], ksplit[3], splits[3];
+	int ksplit[3], splits[3];
 	float* part[3];                   // [split][64][448]
 	// conv1
 	const float *x0, *dA1;
@@ -524,9 +547,11 @@ __device__ __forceinline__ float net_dz(float d, int sign) { return sign ? 0.5f 
 // of a is 24 values from 3 positions early on, so that the 16 around a lane's
 // 8 positions are two aligned 16-byte reads and the taps are their 7 shifts.
 constexpr int kDwZ = kDwChunk + 8, kDwA = kDwChunk / 16 * 24 + 8;   // odd multiples of 8: all banks
-__device__ __forceinline__ void net_dw_conv(const NetDwArgs& g, int layer, int split, __bf16* sm)
+template <int layer>
+__device__ __forceinline__ void net_dw_conv(const NetDwArgs& g, int split, __bf16* sm)
 {
-	const int L = g.L[layer], B = g.B, BL = B * L;
+	constexpr int L = kNetBins / 2 >> layer;
+	const int BL = g.B * L;
 	const float* a = g.a[layer];
 	const float* dA = g.dA[layer];
 	const unsigned char* sg = g.sgn[layer];
@@ -561,8 +586,9 @@ __device__ __forceinline__ void net_dw_conv(const NetDwArgs& g, int layer, int s
 				pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
 		}
 		// a: 64 channels x 8 slices x 3 groups of 8, 6 per thread
-#pragma unroll 2
-		for (int i = tid; i < kNetCh * 24; i += 256) {
+#pragma unroll
+		for (int n = 0; n < kNetCh * 24 / 256; ++n) {
+			const int i = tid + n * 256;
 			const int ci = i / 24, gr = i - ci * 24, s = gr / 3;
 			const int qs = q0 + 16 * s, o = (gr - 3 * s) * 8 - 3;
 			const int l0 = qs % L + o;                           // place in its row
@@ -671,7 +697,7 @@ __device__ __forceinline__ void net_dw_conv1(const NetDwArgs& g, int c, float* s
 // Bias of conv layer `layer`, channel c: thread sums positions tid, tid + 256, ...
 __device__ __forceinline__ void net_db_conv(const NetDwArgs& g, int layer, int c, float* sm)
 {
-	const int BL = g.B * g.L[layer];
+	const int BL = g.B * (kNetBins / 2 >> layer);
 	const float* dA = g.dA[layer] + (long long)c * (BL / 2);
 	const unsigned char* sg = g.sgn[layer] + (long long)c * (BL / 2);
 	float s = 0.f;
@@ -784,9 +810,9 @@ __global__ __launch_bounds__(256) void k_net_dw(NetDwArgs g)
 	__shared__ __attribute__((aligned(16))) unsigned char sm[kDwLds];
 	float* fs = reinterpret_cast<float*>(sm);
 	const int i = blockIdx.x;
-	if (i < g.first[1]) net_dw_conv(g, 0, i, reinterpret_cast<__bf16*>(sm));
-	else if (i < g.first[2]) net_dw_conv(g, 1, i - g.first[1], reinterpret_cast<__bf16*>(sm));
-	else if (i < g.first[3]) net_dw_conv(g, 2, i - g.first[2], reinterpret_cast<__bf16*>(sm));
+	if (i < g.first[1]) net_dw_conv<0>(g, i, reinterpret_cast<__bf16*>(sm));
+	else if (i < g.first[2]) net_dw_conv<1>(g, i - g.first[1], reinterpret_cast<__bf16*>(sm));
+	else if (i < g.first[3]) net_dw_conv<2>(g, i - g.first[2], reinterpret_cast<__bf16*>(sm));
 	else if (i < g.first[4]) net_dw_conv1(g, i - g.first[3], fs);
 	else if (i < g.first[5]) net_db_conv(g, (i - g.first[4]) / kNetCh, (i - g.first[4]) % kNetCh, fs);
 	else if (i < g.first[6]) net_dw_fc1(g, i - g.first[5], fs);
@@ -802,7 +828,7 @@ __global__ __launch_bounds__(256) void k_net_dw_reduce(NetDwArgs g)
 	const int l = i / NW, e = i - l * NW;
 	const float* p = g.part[l] + e;
 	float s = 0.f;
-#pragma unroll 8
+#pragma unroll 24
 	for (int z = 0; z < g.splits[l]; ++z) s += p[(long long)z * NW];
 	g.grad[(l == 0 ? kNetW2 : l == 1 ? kNetW3 : kNetW4) + e] = s;
 }
