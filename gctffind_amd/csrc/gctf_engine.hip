@@ -843,15 +843,18 @@ int ensure_image_buffers(gctf_ctx* c, int n, int T, int ring_n)
 // launch sequences
 // ---------------------------------------------------------------------------
 
-// Complex elements of one micrograph's part of each rescale buffer: the row
-// spectra (ny rows, spec_ld(ncx) apart) or the rescaled columns (nny x ncx),
-// rounded up to 256 bytes so that every micrograph's rows start on a line.
+// Complex elements of one micrograph's part of each rescale buffer (A the
+// rescaled columns, B the row spectra), rounded up to 256 bytes so that every
+// micrograph's part starts on a line.
 size_t cbuf_elems(const RescalePlan& rp)
 {
 	const int ncx = rp.nnx / 2 + 1;
-	const size_t e = std::max((size_t)rp.ny * spec_ld(ncx), (size_t)ncx * rp.nny);
-	return (e + 31) / 32 * 32;
+	const long long e = std::max(panel_size<kPanelIn>(ncx, rp.ny), panel_size<kPanelOut>(ncx, rp.nny));
+	return (size_t)(e + 31) / 32 * 32;
 }
+
+// A workgroup count rounded up for xcd_group.
+int xcd_items(int n) { return (n + 7) / 8 * 8; }
 
 // Rescale n images (CRescaleImage::DoIt) into padded rows at out + i * out_stride.
 // With tg, the C2R pass also leaves the row partials of tg's mean blocks in
@@ -865,33 +868,28 @@ int launch_rescale_t(gctf_ctx* c, const RescalePlan& rp, const Tin* in, long lon
 	float2* A = c->cbufA.as<float2>();
 	float2* B = c->cbufB.as<float2>();
 	const long long stA = (long long)cbuf_elems(rp), stB = stA;
-	// 1. rows R2C with x crop into A: A[y][kx], rows spec_ld(ncx) apart
+	// 1. rows R2C with x crop into B
 	{
 		const int m = rp.rows_maxn;
-		dim3 grid((rp.ny + 1) / 2, n);
+		dim3 grid(xcd_items((rp.ny + 1) / 2), n);
 		Fft1dPlan p = rp.rows->plan();
 		if (rp.rows_half) {
 			if (m == 8192)
-				PROF(c, "k_rescale_rows_r2c_half", k_rescale_rows_r2c_half<Tin, 1024, 8192><<<dim3(rp.ny, n), 1024,
-					0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA));
+				PROF(c, "k_rescale_rows_r2c_half", k_rescale_rows_r2c_half<Tin, 1024, 8192><<<dim3(xcd_items(rp.ny), n), 1024,
+					0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB));
 			else
-				PROF(c, "k_rescale_rows_r2c_half", k_rescale_rows_r2c_half<Tin, 1024, 16384><<<dim3(rp.ny, n), 1024,
-					0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA));
+				PROF(c, "k_rescale_rows_r2c_half", k_rescale_rows_r2c_half<Tin, 1024, 16384><<<dim3(xcd_items(rp.ny), n), 1024,
+					0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB));
 		} else
-		PROF(c, "k_rescale_rows_r2c", if (m <= 2048) k_rescale_rows_r2c<Tin, 256, 2048><<<grid, 256, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA);
-			else if (m <= 4096) k_rescale_rows_r2c<Tin, 512, 4096><<<grid, 512, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA);
-			else if (m <= 8192) k_rescale_rows_r2c<Tin, 1024, 8192><<<grid, 1024, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA);
-			else k_rescale_rows_r2c<Tin, 1024, 16384><<<grid, 1024, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, A, stA));
+		PROF(c, "k_rescale_rows_r2c", if (m <= 2048) k_rescale_rows_r2c<Tin, 256, 2048><<<grid, 256, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB);
+			else if (m <= 4096) k_rescale_rows_r2c<Tin, 512, 4096><<<grid, 512, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB);
+			else if (m <= 8192) k_rescale_rows_r2c<Tin, 1024, 8192><<<grid, 1024, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB);
+			else k_rescale_rows_r2c<Tin, 1024, 16384><<<grid, 1024, 0, s>>>(in, in_stride, rp.nx, rp.ny, p, ncx, B, stB));
 	}
-	// transpose (ny x ncx) -> B[kx][y]
-	{
-		dim3 grid((ncx + 31) / 32, (rp.ny + 31) / 32, n);
-		PROF(c, "k_transpose_c", k_transpose_c<<<grid, 256, 0, s>>>(A, stA, rp.ny, ncx, B, stB));
-	}
-	// 2. columns: forward ny, crop, inverse nny, written row-major into A: A[y'][kx]
+	// 2. columns B -> A: forward ny, crop, inverse nny
 	{
 		const int m = rp.cols_maxn;
-		dim3 grid(8 * ((ncx + 7) / 8), n);
+		dim3 grid(xcd_items(ncx), n);
 		Fft1dPlan pf = rp.cf->plan(), pi = rp.ci->plan();
 		if (rp.cols_split) {
 			if (m == 8192)
@@ -909,16 +907,16 @@ int launch_rescale_t(gctf_ctx* c, const RescalePlan& rp, const Tin* in, long lon
 	// 3. rows C2R into the padded image
 	{
 		const int m = rp.c2r_maxn;
-		dim3 grid((rp.nny + 1) / 2, n);
+		dim3 grid(xcd_items((rp.nny + 1) / 2), n);
 		Fft1dPlan p = rp.c2r->plan();
 		const TileGrid g = tg ? *tg : TileGrid{};
 		float* rs = tg ? (rowsum_out ? rowsum_out : c->rowsum.as<float>()) : nullptr;
 		if (rp.c2r_half) {
 			if (m == 8192)
-				PROF(c, "k_rescale_rows_c2r_half", k_rescale_rows_c2r_half<1024, 8192><<<dim3(rp.nny, n), 1024, 0,
+				PROF(c, "k_rescale_rows_c2r_half", k_rescale_rows_c2r_half<1024, 8192><<<dim3(xcd_items(rp.nny), n), 1024, 0,
 					s>>>(A, stA, rp.nny, rp.nnx, p, out, out_stride, rp.pitch, g, rs));
 			else
-				PROF(c, "k_rescale_rows_c2r_half", k_rescale_rows_c2r_half<1024, 16384><<<dim3(rp.nny, n), 1024, 0,
+				PROF(c, "k_rescale_rows_c2r_half", k_rescale_rows_c2r_half<1024, 16384><<<dim3(xcd_items(rp.nny), n), 1024, 0,
 					s>>>(A, stA, rp.nny, rp.nnx, p, out, out_stride, rp.pitch, g, rs));
 		} else
 		PROF(c, "k_rescale_rows_c2r", if (m <= 2048) k_rescale_rows_c2r<256, 2048><<<grid, 256, 0, s>>>(A, stA, rp.nny, rp.nnx, p, out, out_stride, rp.pitch, g, rs);
@@ -2639,7 +2637,7 @@ struct ListGroup {
 };
 
 // One rescale stage's launch over the micrographs of one kernel class.
-enum RsStage { RS_R2C = 0, RS_TRANSPOSE = 1, RS_COLS = 2, RS_C2R = 3 };
+enum RsStage { RS_R2C = 0, RS_COLS = 1, RS_C2R = 2, RS_STAGES = 3 };
 struct RsClass {
 	int stage = 0, variant = 0, maxn = 0, f16 = 0;   // variant: half rows (R2C, C2R) or split columns
 	std::vector<int> entries, first;                 // rescale jobs and their first items
@@ -2647,22 +2645,20 @@ struct RsClass {
 	size_t first_off = 0, job_off = 0;               // offsets into the uploaded int table
 };
 
-// Class keys and workgroup items of the four stages of one micrograph.
-int rescale_classes(gctf_ctx* c, const RescalePlan& rp, int f16, int key[4][3], int items[4])
+// Class keys and workgroup items of the stages of one micrograph.
+int rescale_classes(gctf_ctx* c, const RescalePlan& rp, int f16, int key[RS_STAGES][3], int items[RS_STAGES])
 {
 	const int ncx = rp.nnx / 2 + 1;
 	key[RS_R2C][0] = rp.rows_half; key[RS_R2C][1] = rp.rows_maxn;
 	key[RS_R2C][2] = f16;
-	items[RS_R2C] = rp.rows_half ? rp.ny : (rp.ny + 1) / 2;
-	key[RS_TRANSPOSE][0] = 0; key[RS_TRANSPOSE][1] = 0; key[RS_TRANSPOSE][2] = 0;
-	items[RS_TRANSPOSE] = ((ncx + 31) / 32) * ((rp.ny + 31) / 32);
+	items[RS_R2C] = xcd_items(rp.rows_half ? rp.ny : (rp.ny + 1) / 2);
 	key[RS_COLS][0] = rp.cols_split;
 	key[RS_COLS][1] = rp.cols_maxn;
 	key[RS_COLS][2] = 0;
-	items[RS_COLS] = 8 * ((ncx + 7) / 8);                // a multiple of 8: xcd_group sees the XCD
+	items[RS_COLS] = xcd_items(ncx);
 	key[RS_C2R][0] = rp.c2r_half; key[RS_C2R][1] = rp.c2r_maxn;
 	key[RS_C2R][2] = 0;
-	items[RS_C2R] = rp.c2r_half ? rp.nny : (rp.nny + 1) / 2;
+	items[RS_C2R] = xcd_items(rp.c2r_half ? rp.nny : (rp.nny + 1) / 2);
 	return GCTF_OK;
 }
 
@@ -2693,9 +2689,6 @@ int launch_rs_class(gctf_ctx* c, const RsClass& k, const RescaleJob* jobs, const
 	switch (k.stage) {
 	case RS_R2C:
 		CHK(k.f16 ? launch_rs_r2c<_Float16>(c, k, jobs, first, job) : launch_rs_r2c<float>(c, k, jobs, first, job));
-		break;
-	case RS_TRANSPOSE:
-		RS_LAUNCH("k_transpose_list", k_transpose_list, 256);
 		break;
 	case RS_COLS:
 		if (k.variant) {
@@ -2920,9 +2913,9 @@ int gctf_estimate_list(gctf_ctx* ctx, const gctf_image* imgs, int n, gctf_result
 			R.g = it[i].g;
 			const int rj = (int)rjobs.size();
 			rjobs.push_back(R);
-			int ck[4][3], items[4];
+			int ck[RS_STAGES][3], items[RS_STAGES];
 			CHK(rescale_classes(ctx, rp, imgs[i].dtype == GCTF_DTYPE_F16, ck, items));
-			for (int st = 0; st < 4; ++st) {
+			for (int st = 0; st < RS_STAGES; ++st) {
 				const std::vector<int> kk = {st, ck[st][0], ck[st][1], ck[st][2]};
 				auto f = index.find(kk);
 				if (f == index.end()) {
