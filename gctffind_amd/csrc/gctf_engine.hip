@@ -291,7 +291,9 @@ struct gctf_ctx {
 	hipStream_t stream = nullptr;
 	gctf_params prm{};
 	std::string err;
-	int chunk = 4, tile_splits = 8, use_graph = 1;
+	// images per launch of the spectrum stage: 32 x 4096^2 take 8246 us with 1,
+	// 7707 with 4, 7531 with 8, 7459 with 16 (and twice the memory)
+	int chunk = 8, tile_splits = 8, use_graph = 1;
 	int cpb = 8;          // candidates per 2D-evaluator workgroup (search blocking: 4, 8 or 16)
 	int list_queue = 1;   // tile row pass of a list: 1 persistent workgroups on a work queue, 0 one item each
 	int tune_gen = 0;     // bumped by gctf_autotune (list graphs read the tuned values)
@@ -945,6 +947,19 @@ int launch_rescale(gctf_ctx* c, const RescalePlan& rp, const void* in, int dtype
 	return launch_rescale_t<float>(c, rp, (const float*)in, in_stride, n, out, out_stride, tg, rowsum_out);
 }
 
+// Images per launch of the tile passes: as many as leave the row pass's
+// output (1 MB per tile of 512) in the 256 MB memory-side cache, where the
+// column pass reads it.  Per 4096^2 micrograph (144 tiles, 152 MB) the two
+// passes took 49.2 + 43.5 us four at a time and 54.4 + 34.3 us one at a time,
+// 41 x 3838x3710 5195 and 4735 us in all; with two at a time (304 MB) nothing
+// is gained any more.
+constexpr size_t kTileRtBytes = 192u << 20;
+int tile_images(const TileGrid& g, int T, int n)
+{
+	const size_t per = sizeof(float2) * (size_t)g.ntx * g.nty * (T / 2 + 1) * T;
+	return (int)std::min<size_t>((size_t)n, std::max<size_t>(1, kTileRtBytes / per));
+}
+
 int ensure_spectrum_buffers(gctf_ctx* c, const TileGrid& g, int T, int n)
 {
 	const size_t cx = T / 2 + 1;
@@ -952,7 +967,7 @@ int ensure_spectrum_buffers(gctf_ctx* c, const TileGrid& g, int T, int n)
 	CHK(ensure_buf(c, c->bsums, sizeof(float) * (size_t)g.nbx * g.nby * kSumParts * n));
 	const size_t nr = (size_t)(g.nby - 1) * g.step + g.bsize;   // rows of the mean blocks
 	CHK(ensure_buf(c, c->rowsum, sizeof(float) * nr * g.nbx * n));
-	CHK(ensure_buf(c, c->rt, sizeof(float2) * ntiles * cx * T * n));
+	CHK(ensure_buf(c, c->rt, sizeof(float2) * ntiles * cx * T * tile_images(g, T, n)));
 	CHK(ensure_buf(c, c->tpart, sizeof(float) * (size_t)c->tile_splits * T * cx * n));
 	return GCTF_OK;
 }
@@ -974,19 +989,24 @@ int launch_spectrum_t(gctf_ctx* c, const TileGrid& g, const TileTables& tt, cons
 			c->rowsum.as<float>()));
 	}
 	const int np = g.nbx * g.nby * kSumParts;
-	PROF(c, "k_block_rows", k_block_rows<<<dim3((np + 255) / 256, n), 256, 0, s>>>(c->rowsum.as<float>(), g,
+	PROF(c, "k_block_rows", k_block_rows<<<dim3((4 * np + 255) / 256, n), 256, 0, s>>>(c->rowsum.as<float>(), g,
 		c->bsums.as<float>()));
 	constexpr int ROWS = 16;                                 // rows per row-pass workgroup
 	const long long rts = (long long)ntiles * CX * T;
 	constexpr int RG = 2;                                    // row blocks per row-pass workgroup
-	PROF(c, "k_tile_rows", k_tile_rows<Tin, T, ROWS, RG><<<dim3((ntiles * (T / ROWS) + RG - 1) / RG, n),
-		(ROWS / 2) * (T / 8), 0, s>>>(
-		img, stride, pitch, g, c->bsums.as<float>(), tt.mask.as<float>(), tt.tw.as<float2>(),
-		c->rt.as<float2>(), rts));
 	constexpr int CPW = 4;
 	const float fac = 1.0f / (float)ntiles;                   // CGenAvgSpectrum.cpp:90
-	PROF(c, "k_tile_cols", k_tile_cols<T, CPW><<<dim3(tile_col_groups(CX, CPW), nsplit, n), CPW * (T / 8), 0, s>>>(
-		c->rt.as<float2>(), rts, ntiles, nsplit, fac, tt.tw.as<float2>(), c->tpart.as<float>()));
+	const int S = tile_images(g, T, n);
+	for (int i = 0; i < n; i += S) {
+		const int m = std::min(S, n - i);
+		PROF(c, "k_tile_rows", k_tile_rows<Tin, T, ROWS, RG><<<dim3((ntiles * (T / ROWS) + RG - 1) / RG, m),
+			(ROWS / 2) * (T / 8), 0, s>>>(
+			img + (long long)i * stride, stride, pitch, g, c->bsums.as<float>() + (size_t)i * np, tt.mask.as<float>(),
+			tt.tw.as<float2>(), c->rt.as<float2>(), rts));
+		PROF(c, "k_tile_cols", k_tile_cols<T, CPW><<<dim3(tile_col_groups(CX, CPW), nsplit, m), CPW * (T / 8), 0, s>>>(
+			c->rt.as<float2>(), rts, ntiles, nsplit, fac, tt.tw.as<float2>(),
+			c->tpart.as<float>() + (size_t)i * nsplit * T * CX));
+	}
 	const int npix = T * CX;
 	PROF(c, "k_tile_reduce", k_tile_reduce<<<dim3((npix + 255) / 256, n), 256, 0, s>>>(c->tpart.as<float>(), nsplit, npix,
 		c->raw.as<float>() + (size_t)slot0 * npix));
@@ -2735,7 +2755,7 @@ int launch_tile_list_t(gctf_ctx* c, const TileTables& tt, const TileJob* d_jobs,
 	const TileJob* jobs = d_jobs + G.j0;
 	if (G.max_nr > 0)
 		PROF(c, "k_row_sums", k_row_sums_list<Tin><<<dim3(G.max_nr, G.nj), 256, 0, s>>>(jobs, c->rowsum.as<float>()));
-	PROF(c, "k_block_rows", k_block_rows_list<<<dim3((G.max_np + 255) / 256, G.nj), 256, 0, s>>>(jobs,
+	PROF(c, "k_block_rows", k_block_rows_list<<<dim3((4 * G.max_np + 255) / 256, G.nj), 256, 0, s>>>(jobs,
 		c->rowsum.as<float>(), c->bsums.as<float>()));
 	// The row pass's items differ in cost (rows of 8-bit, 16-bit and float
 	// micrographs, edge tiles), so it runs on a work queue; the column pass's

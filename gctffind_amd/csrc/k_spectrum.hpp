@@ -562,19 +562,23 @@ __global__ __launch_bounds__(256) void k_row_sums_list(const TileJob* __restrict
 // Second step: part p of block (bi, bj) adds its rows' partials in FP32,
 // rows r0 + j into accumulator j % 4, then (a0 + a1) + (a2 + a3): a fixed
 // order whose rounding error grows with a quarter of the row count.  Grid
-// (ceil(nbx nby kSumParts / 256), images).
+// (ceil(4 nbx nby kSumParts / 256), images).
 __device__ __forceinline__ void block_rows_body(const float* __restrict__ rs, const TileGrid& g,
 	float* __restrict__ sums, int i)
 {
+	// four threads per part, one per accumulator
 	const int nblk = g.nbx * g.nby;
-	if (i >= nblk * kSumParts) return;
-	const int b = i / kSumParts, p = i % kSumParts;
+	const int b = i / (4 * kSumParts), p = i / 4 % kSumParts, q = i & 3;
+	if (b >= nblk) return;                      // all four of a part together
 	const int bi = b % g.nbx, bj = b / g.nbx;
 	const int rows = (g.bsize + kSumParts - 1) / kSumParts;
 	const int r0 = bj * g.step + p * rows, r1 = bj * g.step + min(g.bsize, (p + 1) * rows);
-	float a[4] = {0.f, 0.f, 0.f, 0.f};
-	for (int r = r0; r < r1; ++r) a[(r - r0) & 3] += rs[r * g.nbx + bi];
-	sums[(long long)b * kSumParts + p] = (a[0] + a[1]) + (a[2] + a[3]);
+	float a = 0.f;
+#pragma unroll 8
+	for (int r = r0 + q; r < r1; r += 4) a += rs[r * g.nbx + bi];
+	a += __shfl_xor(a, 1);
+	a += __shfl_xor(a, 2);
+	if (q == 0) sums[(long long)b * kSumParts + p] = a;
 }
 
 __global__ __launch_bounds__(256) void k_block_rows(const float* __restrict__ rowsum, TileGrid g,
@@ -585,7 +589,7 @@ __global__ __launch_bounds__(256) void k_block_rows(const float* __restrict__ ro
 		sums + (long long)blockIdx.y * g.nbx * g.nby * kSumParts, blockIdx.x * 256 + threadIdx.x);
 }
 
-// Grid (ceil(largest nbx nby kSumParts / 256), jobs).
+// Grid (ceil(4 largest nbx nby kSumParts / 256), jobs).
 __global__ __launch_bounds__(256) void k_block_rows_list(const TileJob* __restrict__ jobs,
 	const float* __restrict__ rowsum, float* __restrict__ sums)
 {
@@ -837,6 +841,7 @@ __device__ __forceinline__ void tile_reduce_body(const float* __restrict__ p, in
 {
 	if (i >= n) return;
 	float acc = 0.f;
+#pragma unroll 8
 	for (int s = 0; s < nsplit; ++s) acc += p[(long long)s * n + i];
 	raw[i] = acc;
 }
