@@ -156,18 +156,39 @@ bool smooth235(int n)
 // and 2^a 3^b 5^c (Stockham passes), else the fine grid's, at least 2 n - 1.
 int work_len(int n) { return is_pow2(n) || smooth235(n) ? n : next_pow2(2 * n - 1); }
 
-// Pass radices of a 2^a 3^b 5^c length: radix 8 while 8 divides what is
-// left of the power of two, then one pass of 4 or 2, then the 3s and 5s.
+// Pass radices of a 2^a 3^b 5^c length: the fewest passes, and among those
+// the smallest largest radix; 8s first (their reads and writes keep the LDS
+// padding regular), then the larger ones.
 std::vector<unsigned char> mixed_radices(int n)
 {
+	struct Rad { unsigned char r, a, b, c; };
+	static const Rad set[] = {{8, 3, 0, 0}, {12, 2, 1, 0}, {10, 1, 0, 1}, {9, 0, 2, 0}, {6, 1, 1, 0}, {5, 0, 0, 1},
+		{4, 2, 0, 0}, {3, 0, 1, 0}, {2, 1, 0, 0}};
+	int a = 0, b = 0, c = 0;
+	for (; n % 2 == 0; n /= 2) ++a;
+	for (; n % 3 == 0; n /= 3) ++b;
+	for (; n % 5 == 0; n /= 5) ++c;
+	// best[x][y][z]: passes (high part), largest radix, and the radix to take
+	const auto at = [nb = b + 1, nc = c + 1](int x, int y, int z) { return ((size_t)x * nb + y) * nc + z; };
+	std::vector<int> cost((size_t)(a + 1) * (b + 1) * (c + 1), 1 << 30), take(cost.size(), 0);
+	cost[0] = 0;
+	for (int x = 0; x <= a; ++x)
+		for (int y = 0; y <= b; ++y)
+			for (int z = 0; z <= c; ++z)
+				for (const Rad& q : set) {
+					if (q.a > x || q.b > y || q.c > z) continue;
+					const int prev = cost[at(x - q.a, y - q.b, z - q.c)];
+					if (prev >= 1 << 30) continue;
+					const int v = (prev / 256 + 1) * 256 + std::max(prev % 256, (int)q.r);
+					if (v < cost[at(x, y, z)]) { cost[at(x, y, z)] = v; take[at(x, y, z)] = (int)(&q - set); }
+				}
 	std::vector<unsigned char> r;
-	int p2 = 0;
-	while (n % 2 == 0) { n /= 2; ++p2; }
-	for (; p2 >= 3; p2 -= 3) r.push_back(8);
-	if (p2 == 2) r.push_back(4);
-	if (p2 == 1) r.push_back(2);
-	while (n % 3 == 0) { n /= 3; r.push_back(3); }
-	while (n % 5 == 0) { n /= 5; r.push_back(5); }
+	while (a + b + c > 0) {
+		const Rad& q = set[take[at(a, b, c)]];
+		r.push_back(q.r);
+		a -= q.a; b -= q.b; c -= q.c;
+	}
+	std::sort(r.begin(), r.end(), [](unsigned char x, unsigned char y) { return x == 8 ? y != 8 : y != 8 && x > y; });
 	return r;
 }
 

@@ -4,7 +4,7 @@
 // or 4) whose butterflies live in registers; one workgroup-wide barrier
 // separates the LDS reads of a pass from its writes, so one LDS buffer of N
 // complex values suffices.  Lengths 2^a 3^b 5^c run the same Stockham passes
-// with radix-3 and radix-5 butterflies added (fft_lds_mixed).  Other lengths
+// with further butterflies up to radix 12 (fft_mixed).  Other lengths
 // run on a power-of-two grid at least twice as fine, reached by an eight-point
 // interpolation (itp_fwd, itp_inv).  All are unnormalised; the forward
 // transform uses exp(-2 pi i k n / N).
@@ -150,6 +150,63 @@ template <>
 __device__ __forceinline__ void dft_small<5, false>(float2* u) { dft5<false>(u); }
 template <>
 __device__ __forceinline__ void dft_small<5, true>(float2* u) { dft5<true>(u); }
+
+// Composite radices: N = A B coprime (Good-Thomas, no twiddles): the inputs
+// (B a + A b) mod N, the outputs (KA a + KB b) mod N with KA = 1 mod A, 0 mod
+// B and KB the reverse.
+template <int A, int B, int KA, int KB, bool INV>
+__device__ __forceinline__ void dft_coprime(float2* u)
+{
+	constexpr int N = A * B;
+	static_assert(KA % A == 1 && KA % B == 0 && KB % B == 1 && KB % A == 0, "residues");
+	float2 v[A][B];
+#pragma unroll
+	for (int a = 0; a < A; ++a) {
+#pragma unroll
+		for (int b = 0; b < B; ++b) v[a][b] = u[(B * a + A * b) % N];
+		dft_small<B, INV>(v[a]);
+	}
+#pragma unroll
+	for (int b = 0; b < B; ++b) {
+		float2 c[A];
+#pragma unroll
+		for (int a = 0; a < A; ++a) c[a] = v[a][b];
+		dft_small<A, INV>(c);
+#pragma unroll
+		for (int a = 0; a < A; ++a) u[(KA * a + KB * b) % N] = c[a];
+	}
+}
+template <> __device__ __forceinline__ void dft_small<6, false>(float2* u) { dft_coprime<2, 3, 3, 4, false>(u); }
+template <> __device__ __forceinline__ void dft_small<6, true>(float2* u) { dft_coprime<2, 3, 3, 4, true>(u); }
+template <> __device__ __forceinline__ void dft_small<10, false>(float2* u) { dft_coprime<2, 5, 5, 6, false>(u); }
+template <> __device__ __forceinline__ void dft_small<10, true>(float2* u) { dft_coprime<2, 5, 5, 6, true>(u); }
+template <> __device__ __forceinline__ void dft_small<12, false>(float2* u) { dft_coprime<4, 3, 9, 4, false>(u); }
+template <> __device__ __forceinline__ void dft_small<12, true>(float2* u) { dft_coprime<4, 3, 9, 4, true>(u); }
+
+// 9 = 3 x 3, twiddles exp(-+2 pi i a b / 9)
+template <bool INV>
+__device__ __forceinline__ void dft9(float2* u)
+{
+	const float2 w1 = make_float2(0.76604444311897803520f, INV ? 0.64278760968653932632f : -0.64278760968653932632f);
+	const float2 w2 = make_float2(0.17364817766693034885f, INV ? 0.98480775301220805937f : -0.98480775301220805937f);
+	const float2 w4 = make_float2(-0.93969262078590838405f, INV ? 0.34202014332566873304f : -0.34202014332566873304f);
+	float2 v[3][3];
+#pragma unroll
+	for (int b = 0; b < 3; ++b) {
+		v[b][0] = u[b]; v[b][1] = u[b + 3]; v[b][2] = u[b + 6];
+		dft3<INV>(v[b]);
+	}
+	v[1][1] = cmul(v[1][1], w1); v[1][2] = cmul(v[1][2], w2);
+	v[2][1] = cmul(v[2][1], w2); v[2][2] = cmul(v[2][2], w4);
+#pragma unroll
+	for (int a = 0; a < 3; ++a) {
+		float2 c[3] = {v[0][a], v[1][a], v[2][a]};
+		dft3<INV>(c);
+		u[a] = c[0]; u[a + 3] = c[1]; u[a + 6] = c[2];
+	}
+}
+template <> __device__ __forceinline__ void dft_small<9, false>(float2* u) { dft9<false>(u); }
+template <> __device__ __forceinline__ void dft_small<9, true>(float2* u) { dft9<true>(u); }
 
 // u[r] *= w^r for r = 1 .. R-1 (w already conjugated for the inverse).
 template <int R>
@@ -381,58 +438,66 @@ struct LdsOut {
 	__device__ __forceinline__ void operator()(int i, float2 v) const { buf[pidx(i)] = v; }
 };
 
-template <int N, int R, int L, int NT, bool INV, class Ld, class St>
-__device__ __forceinline__ void fft_pass_io(float2* buf, const float2* __restrict__ tw, int tid,
-	const Ld& ld, const St& st)
+// A pass's twiddles are loaded before the barrier that precedes it, so that
+// their latency (L2, several hundred cycles) overlaps the stores and the wait.
+template <int N, int L>
+__host__ __device__ constexpr int fft_radix() { return N / L >= 8 ? 8 : N / L; }
+
+template <int N, int L, int NT>
+__device__ __forceinline__ void fft_tw_fetch(float2* w, const float2* __restrict__ tw, int tid)
 {
-	constexpr int T = N / R;
-	constexpr int BPT = (T + NT - 1) / NT;
-	float2 u[BPT][R];
+	constexpr int R = fft_radix<N, L>(), T = N / R, BPT = (T + NT - 1) / NT;
 #pragma unroll
 	for (int b = 0; b < BPT; ++b) {
 		const int j = tid + b * NT;
-		if (T % NT == 0 || j < T) {
-#pragma unroll
-			for (int r = 0; r < R; ++r) {
-				if constexpr (L == 1) u[b][r] = ld(j + r * T);
-				else u[b][r] = buf[pidx(j + r * T)];
-			}
-			if constexpr (L > 1) {
-				const int k = j & (L - 1);
-				constexpr int S = N / (L * R);
-				float2 w = tw[k * S];
-				if (INV) w.y = -w.y;
-				twiddle_powers<R>(u[b], w);
-			}
-			dft_small<R, INV>(u[b]);
-		}
+		if (T % NT == 0 || j < T) w[b] = tw[(j & (L - 1)) * (N / (L * R))];
 	}
-	fft_sync<NT>();
-#pragma unroll
-	for (int b = 0; b < BPT; ++b) {
-		const int j = tid + b * NT;
-		if (T % NT == 0 || j < T) {
-			const int k = j & (L - 1);
-			const int base = (j - k) * R + k;
-#pragma unroll
-			for (int r = 0; r < R; ++r) {
-				if constexpr (L * R == N) st(base + r * L, u[b][r]);
-				else buf[pidx(base + r * L)] = u[b][r];
-			}
-		}
-	}
-	fft_sync<NT>();
 }
 
 template <int N, int L, int NT, bool INV, class Ld, class St>
 __device__ __forceinline__ void fft_run_io(float2* buf, const float2* __restrict__ tw, int tid,
-	const Ld& ld, const St& st)
+	const Ld& ld, const St& st, const float2* w)
 {
 	if constexpr (L < N) {
-		constexpr int rem = N / L;
-		constexpr int R = rem >= 8 ? 8 : rem;
-		fft_pass_io<N, R, L, NT, INV>(buf, tw, tid, ld, st);
-		fft_run_io<N, L * R, NT, INV>(buf, tw, tid, ld, st);
+		constexpr int R = fft_radix<N, L>(), T = N / R;
+		constexpr int BPT = (T + NT - 1) / NT;
+		float2 u[BPT][R];
+#pragma unroll
+		for (int b = 0; b < BPT; ++b) {
+			const int j = tid + b * NT;
+			if (T % NT == 0 || j < T) {
+#pragma unroll
+				for (int r = 0; r < R; ++r) {
+					if constexpr (L == 1) u[b][r] = ld(j + r * T);
+					else u[b][r] = buf[pidx(j + r * T)];
+				}
+				if constexpr (L > 1) {
+					float2 wb = w[b];
+					if (INV) wb.y = -wb.y;
+					twiddle_powers<R>(u[b], wb);
+				}
+				dft_small<R, INV>(u[b]);
+			}
+		}
+		constexpr int L2 = L * R;
+		float2 wn[fft_max_bpt(N, NT)];
+		if constexpr (L2 < N) fft_tw_fetch<N, L2, NT>(wn, tw, tid);
+		fft_sync<NT>();
+#pragma unroll
+		for (int b = 0; b < BPT; ++b) {
+			const int j = tid + b * NT;
+			if (T % NT == 0 || j < T) {
+				const int k = j & (L - 1);
+				const int base = (j - k) * R + k;
+#pragma unroll
+				for (int r = 0; r < R; ++r) {
+					if constexpr (L2 == N) st(base + r * L, u[b][r]);
+					else buf[pidx(base + r * L)] = u[b][r];
+				}
+			}
+		}
+		fft_sync<NT>();
+		fft_run_io<N, L2, NT, INV>(buf, tw, tid, ld, st, wn);
 	}
 }
 
@@ -443,7 +508,7 @@ __device__ __forceinline__ void fft_lds_io(float2* buf, const float2* __restrict
 	const Ld& ld, const St& st)
 {
 	static_assert(N >= 16, "the first and last passes must differ");
-	fft_run_io<N, 1, NT, INV>(buf, tw, tid, ld, st);
+	fft_run_io<N, 1, NT, INV>(buf, tw, tid, ld, st, nullptr);
 }
 
 // ---- runtime-length power-of-two FFT (lengths up to MAXN) ----------------
@@ -520,7 +585,7 @@ struct Fft1dPlan {
 	                         // else the points of the fine grid, the kernel's MAXN
 	const float2* tw;        // twiddles of the passes: n points, or m / 2 points on the fine grid
 	int nrad;                // mixed-radix passes (lengths 2^a 3^b 5^c that are not powers of two), else 0
-	unsigned char rad[20];   // their radices, in pass order: 8s, then a 4 or 2, then 3s, then 5s
+	unsigned char rad[20];   // their radices, in pass order
 	// lengths on the fine grid (else null); S = 2 when n is even, else 1
 	const float2* mode;      // [2][n/2 + 1]: the modes' factors on the grid's even and odd points
 	const float4* w8;        // [n/S][2]: the 8 weights of output t around point p0[t] (inverse)
@@ -534,59 +599,139 @@ struct Fft1dPlan {
 // butterfly j (T = n / R of them) reads j + r T, multiplies element r by
 // w^r with w = exp(-+2 pi i k S / n), k = j mod L, S = n / (L R), and
 // writes (j - k) R + k + r L.
+//
+// What bounds it is the chain of a pass (LDS, twiddle load, barrier), so the
+// radices are as large as fit in registers (mixed_radices): 5760 = 8 8 10 9
+// in 4 passes instead of 8 8 2 3 3 5 in 6.  A pass enters with the barrier
+// that follows the last one's writes still to come and loads its twiddles
+// before it.  Where T (or L) is a multiple of 8, as after a first radix of 8,
+// the padded addresses of a butterfly's reads (writes) are equally spaced.
 template <int R, int NT, int MAXN, bool INV>
 __device__ __forceinline__ void fft_pass_mx(float2* buf, const float2* __restrict__ tw, int tid,
 	int L, int T, int S)
 {
 	constexpr int BPT = (MAXN / R + NT - 1) / NT;
-	const bool lpow2 = (L & (L - 1)) == 0;
-	float2 u[BPT][R];
+	// q = j / L: (j + 1/2) / L is at least 1 / (2 L) from an integer, and its
+	// rounding error below 2^-23 j / L, less for j < 2^14
+	const float rl = 1.0f / (float)L;
+	float2 u[BPT][R], w[BPT];
 	int kk[BPT];
 #pragma unroll
 	for (int b = 0; b < BPT; ++b) {
 		const int j = tid + b * NT;
-		kk[b] = 0;
-		if (j < T) {
-			kk[b] = lpow2 ? (j & (L - 1)) : j % L;
+		kk[b] = j - (int)(((float)j + 0.5f) * rl) * L;
+		if (j < T) w[b] = tw[kk[b] * S];
+	}
+	__syncthreads();
+	const bool even_reads = (T & 7) == 0;
 #pragma unroll
-			for (int r = 0; r < R; ++r) u[b][r] = buf[pidx(j + r * T)];
+	for (int b = 0; b < BPT; ++b) {
+		const int j = tid + b * NT;
+		if (j < T) {
+			if (even_reads) {
+				const float2* p = buf + pidx(j);
+				const int st = T + (T >> 3);
+#pragma unroll
+				for (int r = 0; r < R; ++r) u[b][r] = p[r * st];
+			} else {
+#pragma unroll
+				for (int r = 0; r < R; ++r) u[b][r] = buf[pidx(j + r * T)];
+			}
 			if (L > 1) {
-				float2 w = tw[kk[b] * S];
-				if (INV) w.y = -w.y;
-				twiddle_powers<R>(u[b], w);
+				float2 wb = w[b];
+				if (INV) wb.y = -wb.y;
+				twiddle_powers<R>(u[b], wb);
 			}
 			dft_small<R, INV>(u[b]);
 		}
 	}
 	__syncthreads();
+	const bool even_writes = (L & 7) == 0;
 #pragma unroll
 	for (int b = 0; b < BPT; ++b) {
 		const int j = tid + b * NT;
 		if (j < T) {
 			const int base = (j - kk[b]) * R + kk[b];
+			if (even_writes) {
+				float2* p = buf + pidx(base);
+				const int st = L + (L >> 3);
 #pragma unroll
-			for (int r = 0; r < R; ++r) buf[pidx(base + r * L)] = u[b][r];
+				for (int r = 0; r < R; ++r) p[r * st] = u[b][r];
+			} else {
+#pragma unroll
+				for (int r = 0; r < R; ++r) buf[pidx(base + r * L)] = u[b][r];
+			}
 		}
 	}
-	__syncthreads();
 }
 
-// In-place transform of a mixed-radix plan (n <= MAXN); same contract as
-// fft_lds_rt.
+// The passes of a mixed-radix plan (n <= MAXN) from pass i on; the data is in
+// buf, not necessarily visible yet; results are visible after.
 template <int NT, int MAXN, bool INV>
-__device__ __forceinline__ void fft_lds_mixed(float2* buf, const Fft1dPlan& p, int tid)
+__device__ __forceinline__ void fft_lds_mixed(float2* buf, const Fft1dPlan& p, int tid, int i, int L)
 {
-	int L = 1;
-	for (int i = 0; i < p.nrad; ++i) {
+	for (; i < p.nrad; ++i) {
 		const int R = p.rad[i];
 		const int T = p.n / R, S = p.n / (L * R);
 		if (R == 8) fft_pass_mx<8, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
+		else if (R == 10) fft_pass_mx<10, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
+		else if (R == 9) fft_pass_mx<9, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
+		else if (R == 12) fft_pass_mx<12, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
+		else if (R == 6) fft_pass_mx<6, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
 		else if (R == 4) fft_pass_mx<4, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
 		else if (R == 2) fft_pass_mx<2, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
 		else if (R == 3) fft_pass_mx<3, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
 		else fft_pass_mx<5, NT, MAXN, INV>(buf, p.tw, tid, L, T, S);
 		L *= R;
 	}
+	__syncthreads();
+}
+
+// The transform of src(i), i in [0, n), by a mixed-radix plan, result in
+// logical buf[0..n).  src may read buf.  A first radix of 8 takes its inputs
+// straight from src.
+template <int NT, int MAXN, bool INV, class Src>
+__device__ __forceinline__ void fft_mixed(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
+{
+	if (p.rad[0] == 8) {
+		constexpr int BPT = (MAXN / 8 + NT - 1) / NT;
+		const int T = p.n / 8;
+		float2 u[BPT][8];
+#pragma unroll
+		for (int b = 0; b < BPT; ++b) {
+			const int j = tid + b * NT;
+			if (j < T) {
+#pragma unroll
+				for (int r = 0; r < 8; ++r) u[b][r] = src(j + r * T);
+				dft8<INV>(u[b]);
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (int b = 0; b < BPT; ++b) {
+			const int j = tid + b * NT;
+			if (j < T) {
+#pragma unroll
+				for (int r = 0; r < 8; ++r) buf[9 * j + r] = u[b][r];     // pidx(8 j + r)
+			}
+		}
+		fft_lds_mixed<NT, MAXN, INV>(buf, p, tid, 1, 8);
+		return;
+	}
+	constexpr int PER = (MAXN + NT - 1) / NT;
+	float2 v[PER];
+#pragma unroll
+	for (int b = 0; b < PER; ++b) {
+		const int i = tid + b * NT;
+		if (i < p.n) v[b] = src(i);
+	}
+	__syncthreads();
+#pragma unroll
+	for (int b = 0; b < PER; ++b) {
+		const int i = tid + b * NT;
+		if (i < p.n) buf[pidx(i)] = v[b];
+	}
+	fft_lds_mixed<NT, MAXN, INV>(buf, p, tid, 0, 1);
 }
 
 // ---- other lengths: a transform on a finer power-of-two grid ---------------
@@ -788,6 +933,8 @@ __device__ __forceinline__ void fft_any_fwd(float2* buf, const Fft1dPlan& p, int
 		fft_lds_io<MAXN, NT, false>(buf, p.tw, tid, src, LdsOut{buf});
 	} else if (p.nrad == 0 && p.n == MAXN / 2) {
 		fft_lds_io<MAXN / 2, NT, false>(buf, p.tw, tid, src, LdsOut{buf});
+	} else if (p.nrad > 0) {
+		fft_mixed<NT, MAXN, false>(buf, p, tid, src);
 	} else {
 		constexpr int PER = (MAXN + NT - 1) / NT;
 		float2 v[PER];
@@ -803,8 +950,7 @@ __device__ __forceinline__ void fft_any_fwd(float2* buf, const Fft1dPlan& p, int
 			if (i < p.n) buf[pidx(i)] = v[b];
 		}
 		__syncthreads();
-		if (p.nrad > 0) fft_lds_mixed<NT, MAXN, false>(buf, p, tid);
-		else fft_lds_rt<NT, MAXN, false>(buf, p.n, p.tw, tid);
+		fft_lds_rt<NT, MAXN, false>(buf, p.n, p.tw, tid);
 	}
 }
 
@@ -812,6 +958,10 @@ __device__ __forceinline__ void fft_any_fwd(float2* buf, const Fft1dPlan& p, int
 template <int NT, int MAXN, class Src>
 __device__ __forceinline__ void fft_inv_passes(float2* buf, const Fft1dPlan& p, int tid, const Src& src)
 {
+	if (p.nrad > 0) {
+		fft_mixed<NT, MAXN, true>(buf, p, tid, [&](int i) -> float2 { return src(i > p.n / 2 ? i - p.n : i); });
+		return;
+	}
 	constexpr int PER = (MAXN + NT - 1) / NT;
 	float2 v[PER];
 #pragma unroll
@@ -826,8 +976,7 @@ __device__ __forceinline__ void fft_inv_passes(float2* buf, const Fft1dPlan& p, 
 		if (i < p.n) buf[pidx(i)] = v[b];
 	}
 	__syncthreads();
-	if (p.nrad > 0) fft_lds_mixed<NT, MAXN, true>(buf, p, tid);
-	else fft_lds_rt<NT, MAXN, true>(buf, p.n, p.tw, tid);
+	fft_lds_rt<NT, MAXN, true>(buf, p.n, p.tw, tid);
 }
 
 // Every output t handed to out(t, v) once; out may not write buf.
