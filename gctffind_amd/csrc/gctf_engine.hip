@@ -1004,14 +1004,18 @@ int launch_spectrum_t(gctf_ctx* c, const TileGrid& g, const TileTables& tt, cons
 	constexpr int CX = T / 2 + 1;
 	const int ntiles = g.ntx * g.nty;
 	const int nsplit = std::min(c->tile_splits, ntiles);
-	if (!rows_ready) {
-		const int nr = (g.nby - 1) * g.step + g.bsize;
-		PROF(c, "k_row_sums", k_row_sums<Tin><<<dim3(nr, n), 256, 0, s>>>(img, stride, pitch, g,
-			c->rowsum.as<float>()));
-	}
 	const int np = g.nbx * g.nby * kSumParts;
-	PROF(c, "k_block_rows", k_block_rows<<<dim3((4 * np + 255) / 256, n), 256, 0, s>>>(c->rowsum.as<float>(), g,
-		c->bsums.as<float>()));
+	// block sums of m images (of their pixels when the row partials are not there)
+	auto sums = [&](const Tin* p, int m) {
+		if (!rows_ready) {
+			const int nr = (g.nby - 1) * g.step + g.bsize;
+			PROF(c, "k_row_sums", k_row_sums<Tin><<<dim3(nr, m), 256, 0, s>>>(p, stride, pitch, g,
+				c->rowsum.as<float>()));
+		}
+		PROF(c, "k_block_rows", k_block_rows<<<dim3((4 * np + 255) / 256, m), 256, 0, s>>>(c->rowsum.as<float>(), g,
+			c->bsums.as<float>()));
+	};
+	if (rows_ready) sums(img, n);
 	constexpr int ROWS = 16;                                 // rows per row-pass workgroup
 	const long long rts = (long long)ntiles * CX * T;
 	constexpr int RG = 2;                                    // row blocks per row-pass workgroup
@@ -1020,9 +1024,15 @@ int launch_spectrum_t(gctf_ctx* c, const TileGrid& g, const TileTables& tt, cons
 	const int S = tile_images(g, T, n);
 	for (int i = 0; i < n; i += S) {
 		const int m = std::min(S, n - i);
+		const Tin* p = img + (long long)i * stride;
+		// reading the pixels for their sums leaves them in the memory-side cache
+		// for the row pass (41 x 3838x3710 4538 -> 4406 us); making the rescaled
+		// ones S images at a time as well costs more in part-filled launches of
+		// the C2R pass than it saves here (32 x 4096^2 7410 -> 7626 us)
+		if (!rows_ready) sums(p, m);
 		PROF(c, "k_tile_rows", k_tile_rows<Tin, T, ROWS, RG><<<dim3((ntiles * (T / ROWS) + RG - 1) / RG, m),
 			(ROWS / 2) * (T / 8), 0, s>>>(
-			img + (long long)i * stride, stride, pitch, g, c->bsums.as<float>() + (size_t)i * np, tt.mask.as<float>(),
+			p, stride, pitch, g, c->bsums.as<float>() + (rows_ready ? (size_t)i * np : 0), tt.mask.as<float>(),
 			tt.tw.as<float2>(), c->rt.as<float2>(), rts));
 		PROF(c, "k_tile_cols", k_tile_cols<T, CPW><<<dim3(tile_col_groups(CX, CPW), nsplit, m), CPW * (T / 8), 0, s>>>(
 			c->rt.as<float2>(), rts, ntiles, nsplit, fac, tt.tw.as<float2>(),
@@ -1055,21 +1065,15 @@ int launch_post_t(gctf_ctx* c, const TileTables& tt, int n)
 	hipStream_t s = c->stream;
 	constexpr int CX = T / 2 + 1;
 	const int npix = T * CX;
-	// box side (GRmBackground2D.cu:33-36) with fMinFreq = 1/15
-	int box = (int)((1.0f / 15.0f) * (float)T);
-	if ((float)box > 0.3f * (float)T) box = (int)(0.3f * (float)T);
-	box = box / 2 * 2 + 1;
-	if (box < 7) box = 7;
-	const int hb = box / 2;
 	const int ls = c->prm.log_spect ? 1 : 0;
-	PROF(c, "k_bg_rows", k_bg_rows<T><<<dim3(T, n), 256, 0, s>>>(c->raw.as<float>(), ls, hb, c->hsum.as<float>()));
-	const int nparts = (npix + 255) / 256;
-	PROF(c, "k_bg_cols", k_bg_cols<T><<<dim3(nparts, 1, n), 256, 0, s>>>(c->raw.as<float>(), c->hsum.as<float>(), ls, hb,
+	PROF(c, "k_bg_rows", k_bg_rows<T><<<dim3(T / kBgRows, n), 256, 0, s>>>(c->raw.as<float>(), ls, c->hsum.as<float>()));
+	constexpr int nparts = bg_col_groups<T>();
+	PROF(c, "k_bg_cols", k_bg_cols<T><<<dim3(nparts, n), 256, 0, s>>>(c->raw.as<float>(), c->hsum.as<float>(), ls,
 		c->spect.as<float>(), c->mom.as<double>()));
 	PROF(c, "k_gate", k_gate<<<n, 256, 0, s>>>(c->mom.as<double>(), nparts, npix, c->states.as<SearchState>()));
 	PROF(c, "k_lp_x", k_lp_x<T><<<dim3(T / 4, n), 2 * (T / 8), 0, s>>>(c->spect.as<float>(), c->states.as<SearchState>(),
 		tt.h1.as<float>(), tt.tw.as<float2>(), c->q.as<float>()));
-	PROF(c, "k_lp_y", k_lp_y<T><<<dim3((CX + 1) / 2, n), T / 8, 0, s>>>(c->q.as<float>(), c->states.as<SearchState>(),
+	PROF(c, "k_lp_y", k_lp_y<T><<<dim3((CX + 2 * kLpPairs - 1) / (2 * kLpPairs), n), kLpPairs * (T / 8), 0, s>>>(c->q.as<float>(), c->states.as<SearchState>(),
 		tt.h1.as<float>(), tt.tw.as<float2>(), c->spect.as<float>()));
 	HIPCHK(c, hipGetLastError());
 	return GCTF_OK;

@@ -868,60 +868,113 @@ __global__ __launch_bounds__(256) void k_tile_reduce_list(const TileJob* __restr
 //   X <  T/2: P = in[Y][X];  X >= T/2: P = in[(T-Y) mod T][T-X].
 // Box sums are separable: H = row sums, then column sums of H.
 // ---------------------------------------------------------------------------
+//
+// Both sums are added directly in the reference's order (a running sum would
+// round differently).  A thread forms kBgRun neighbouring sums from kBgRun + 2
+// half_box values it reads from LDS once each, where one thread per sum read
+// 2 half_box + 1 = 35 values, the columns' from L2: 2.6 us per 512 spectrum for
+// the columns and 1.1 for the rows.
+constexpr int kBgRun = 8;
+// The box half widths of the three tile sizes (GRmBackground2D.cu:33-36).
+template <int T>
+__host__ __device__ constexpr int bg_half()
+{
+	int box = (int)((1.0f / 15.0f) * (float)T);
+	if ((float)box > 0.3f * (float)T) box = (int)(0.3f * (float)T);
+	box = box / 2 * 2 + 1;
+	return (box < 7 ? 7 : box) / 2;
+}
+
+// Sums of 2 HB + 1 neighbours: sum[q] = v(q) + ... + v(q + 2 HB), in that order.
+template <int HB, class V>
+__device__ __forceinline__ void bg_sums(float* sum, const V& v)
+{
+	float w[kBgRun + 2 * HB];
+#pragma unroll
+	for (int i = 0; i < kBgRun + 2 * HB; ++i) w[i] = v(i);
+#pragma unroll
+	for (int q = 0; q < kBgRun; ++q) {
+		float s = 0.f;
+#pragma unroll
+		for (int i = 0; i <= 2 * HB; ++i) s += w[q + i];
+		sum[q] = s;
+	}
+}
+
+// Row sums.  kBgRows rows per workgroup, grid (T / kBgRows, images).  The LDS
+// row is the periodic plane's columns -HB .. T/2 + HB, a word of padding every
+// 8 (the threads of a row read runs 8 apart).
+constexpr int kBgRows = 8;
 template <int T>
 __global__ __launch_bounds__(256) void k_bg_rows(const float* __restrict__ raw, int log_spect,
-	int half_box, float* __restrict__ hsum)
+	float* __restrict__ hsum)
 {
-	constexpr int CX = T / 2 + 1;
-	__shared__ float p[T];
+	constexpr int CX = T / 2 + 1, HB = bg_half<T>();
+	constexpr int N = (CX + kBgRun - 1) / kBgRun * kBgRun + 2 * HB, LD = N + N / 8 + 1;
+	__shared__ float p[kBgRows * LD];
 	const float* in = raw + (long long)blockIdx.y * T * CX;
 	float* out = hsum + (long long)blockIdx.y * T * CX;
-	const int Y = blockIdx.x;
-	for (int X = threadIdx.x; X < T; X += 256) {
-		float v = X < T / 2 ? in[Y * CX + X] : in[((T - Y) & (T - 1)) * CX + (T - X)];
-		p[X] = log_spect ? v : sqrtf(v);
+	const int y0 = blockIdx.x * kBgRows;
+	for (int i = threadIdx.x; i < kBgRows * N; i += 256) {
+		const int r = i / N, e = i - r * N;
+		const int X = (e - HB + T) & (T - 1), Y = y0 + r;
+		const float v = X < T / 2 ? in[Y * CX + X] : in[((T - Y) & (T - 1)) * CX + (T - X)];
+		p[r * LD + e + (e >> 3)] = log_spect ? v : sqrtf(v);
 	}
 	__syncthreads();
-	for (int x = threadIdx.x; x < CX; x += 256) {
-		float acc = 0.f;
-		for (int j = -half_box; j <= half_box; ++j) acc += p[(x + j + T) & (T - 1)];
-		out[Y * CX + x] = acc;
+	constexpr int G = (CX + kBgRun - 1) / kBgRun;         // runs per row
+	for (int i = threadIdx.x; i < kBgRows * G; i += 256) {
+		const int r = i / G, x = (i - r * G) * kBgRun;
+		float s[kBgRun];
+		bg_sums<HB>(s, [&](int j) { return p[r * LD + x + j + ((x + j) >> 3)]; });
+#pragma unroll
+		for (int q = 0; q < kBgRun; ++q)
+			if (x + q < CX) out[(y0 + r) * CX + x + q] = s[q];
 	}
 }
 
 // Column sums, the subtraction, the r < 0.04 zeroing (evaluated in float as
 // the reference does) and per-workgroup moment partials for the gate (an
 // FP32 tree within the workgroup; k_gate adds the partials in FP64).
-// Grid (ceil(T*CX/256), images).
+// kBgCols columns x 8 kBgRun rows per workgroup, grid (bg_col_groups, images).
+constexpr int kBgCols = 32;
+template <int T>
+__host__ __device__ constexpr int bg_col_groups() { return (T / 2 + 1 + kBgCols - 1) / kBgCols * (T / (8 * kBgRun)); }
+
 template <int T>
 __global__ __launch_bounds__(256) void k_bg_cols(const float* __restrict__ raw,
-	const float* __restrict__ hsum, int log_spect, int half_box, float* __restrict__ spect,
-	double* __restrict__ mom)
+	const float* __restrict__ hsum, int log_spect, float* __restrict__ spect, double* __restrict__ mom)
 {
-	constexpr int CX = T / 2 + 1;
+	constexpr int CX = T / 2 + 1, HB = bg_half<T>(), CG = (CX + kBgCols - 1) / kBgCols;
+	constexpr int RY = 8 * kBgRun, N = RY + 2 * HB;
+	__shared__ float p[N * kBgCols];
 	__shared__ float r1[256], r2[256];
-	const int i = blockIdx.x * 256 + threadIdx.x;
-	const float* in = raw + (long long)blockIdx.z * T * CX;
-	const float* h = hsum + (long long)blockIdx.z * T * CX;
+	const int x0 = blockIdx.x % CG * kBgCols, y0 = blockIdx.x / CG * RY;
+	const float* in = raw + (long long)blockIdx.y * T * CX;
+	const float* h = hsum + (long long)blockIdx.y * T * CX;
+	const int c = threadIdx.x % kBgCols, x = x0 + c;
+#pragma unroll 4
+	for (int r = threadIdx.x / kBgCols; r < N; r += 256 / kBgCols)
+		p[r * kBgCols + c] = h[((y0 + r - HB + T) & (T - 1)) * CX + min(x, CX - 1)];
+	__syncthreads();
 	float m1 = 0.0f, m2 = 0.0f;
-	if (i < T * CX) {
-		const int y = i / CX, x = i % CX;
-		const int yc = y - T / 2;
-		float fr = (float)x * 0.5f / (float)(CX - 1);
-		fr = sqrtf(fr * fr + (float)(yc * yc) / (float)(T * T));
-		float o;
-		if ((double)fr < 0.04) {
-			o = 0.f;
-		} else {
-			float acc = 0.f;
-			for (int k = -half_box; k <= half_box; ++k) acc += h[((y + k + T) & (T - 1)) * CX + x];
-			const int b = 2 * half_box + 1;
-			acc /= (float)(b * b);
+	if (x < CX) {
+		const int l0 = threadIdx.x / kBgCols * kBgRun;
+		float s[kBgRun];
+		bg_sums<HB>(s, [&](int j) { return p[(l0 + j) * kBgCols + c]; });
+#pragma unroll
+		for (int q = 0; q < kBgRun; ++q) {
+			const int y = y0 + l0 + q, yc = y - T / 2;
+			float fr = (float)x * 0.5f / (float)(CX - 1);
+			fr = sqrtf(fr * fr + (float)(yc * yc) / (float)(T * T));
+			constexpr int b = 2 * HB + 1;
+			float acc = s[q] / (float)(b * b);
 			if (!log_spect) acc *= acc;
-			o = in[i] - acc;
+			const float o = (double)fr < 0.04 ? 0.f : in[y * CX + x] - acc;
+			spect[(long long)blockIdx.y * T * CX + y * CX + x] = o;
+			m1 += o;
+			m2 += o * o;
 		}
-		spect[(long long)blockIdx.z * T * CX + i] = o;
-		m1 = o; m2 = o * o;
 	}
 	r1[threadIdx.x] = m1; r2[threadIdx.x] = m2;
 	__syncthreads();
@@ -930,7 +983,7 @@ __global__ __launch_bounds__(256) void k_bg_cols(const float* __restrict__ raw,
 		__syncthreads();
 	}
 	if (threadIdx.x == 0) {
-		double* m = mom + ((long long)blockIdx.z * gridDim.x + blockIdx.x) * 2;
+		double* m = mom + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * 2;
 		m[0] = r1[0]; m[1] = r2[0];
 	}
 }
@@ -1008,37 +1061,45 @@ __global__ __launch_bounds__(2 * (T / 8)) void k_lp_x(const float* __restrict__ 
 	}
 }
 
-// y pass on columns c, c+1 of q; result into spect.  Grid (ceil(CX/2), images).
+// y pass on the column pairs of q; result into spect.  kLpPairs pairs per
+// workgroup, a transform each, so that a row's reads and writes are 2 kLpPairs
+// neighbours (one pair per workgroup moved 8 bytes per line: 1.7 us per 512
+// spectrum).  Grid (ceil(CX / (2 kLpPairs)), images).
+constexpr int kLpPairs = 4;
 template <int T>
-__global__ __launch_bounds__(T / 8) void k_lp_y(const float* __restrict__ q,
+__global__ __launch_bounds__(kLpPairs * (T / 8)) void k_lp_y(const float* __restrict__ q,
 	const SearchState* __restrict__ st, const float* __restrict__ h1,
 	const float2* __restrict__ tw, float* __restrict__ spect)
 {
-	constexpr int CX = T / 2 + 1, FT = T / 8;
-	__shared__ float2 buf[fft_lds_len(T)];
+	constexpr int CX = T / 2 + 1, FT = T / 8, NC = 2 * kLpPairs, NT = kLpPairs * FT;
+	constexpr int FL = fft_lds_len(T) + 8;      // the padding keeps a row's columns on different banks
+	__shared__ float2 buf[kLpPairs * FL];
 	if (!st[blockIdx.y].lowpassed) return;
-	const int c0 = 2 * blockIdx.x;
-	const bool two = c0 + 1 < CX;
+	const int c0 = NC * blockIdx.x;
 	const float* in = q + (long long)blockIdx.y * T * CX;
-	const int lane = threadIdx.x;
-	for (int y = lane; y < T; y += FT)
-		buf[pidx(y)] = make_float2(in[y * CX + c0], two ? in[y * CX + c0 + 1] : 0.f);
-	__syncthreads();
-	fft_lds<T, FT, false>(buf, tw, lane);
-	for (int k = lane; k < T; k += FT) {
-		float f = h1[k];
-		float2 z = buf[pidx(k)];
-		buf[pidx(k)] = make_float2(z.x * f, z.y * f);
-	}
-	__syncthreads();
-	fft_lds<T, FT, true>(buf, tw, lane);
 	float* out = spect + (long long)blockIdx.y * T * CX;
-	const float inv = 1.0f / (float)T;
-	for (int y = lane; y < T; y += FT) {
-		float2 z = buf[pidx(y)];
-		out[y * CX + c0] = z.x * inv;
-		if (two) out[y * CX + c0 + 1] = z.y * inv;
+	float* words = reinterpret_cast<float*>(buf);
+	// column c of the group: part c % 2 of transform c / 2
+	const int c = threadIdx.x % NC;
+	auto at = [&](int y) -> float& { return words[2 * (c / 2 * FL + pidx(y)) + c % 2]; };
+#pragma unroll 8
+	for (int y = threadIdx.x / NC; y < T; y += NT / NC) at(y) = c0 + c < CX ? in[y * CX + c0 + c] : 0.f;
+	__syncthreads();
+	const int grp = threadIdx.x / FT, lane = threadIdx.x % FT;
+	float2* fb = buf + grp * FL;
+	fft_lds<T, FT, false>(fb, tw, lane);
+	for (int k = lane; k < T; k += FT) {
+		const float f = h1[k];
+		const float2 z = fb[pidx(k)];
+		fb[pidx(k)] = make_float2(z.x * f, z.y * f);
 	}
+	fft_sync<FT>();
+	fft_lds<T, FT, true>(fb, tw, lane);
+	__syncthreads();
+	const float inv = 1.0f / (float)T;
+#pragma unroll 8
+	for (int y = threadIdx.x / NC; y < T; y += NT / NC)
+		if (c0 + c < CX) out[y * CX + c0 + c] = at(y) * inv;
 }
 
 // ---------------------------------------------------------------------------
