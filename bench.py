@@ -49,8 +49,8 @@ VALU_PEAK_TFLOPS = 78.6   # FP32 FMA without packed math: 256 CU x 64 lanes x 2 
 # scaled by the same counters on a 256 MiB device copy (fetch x2.000,
 # write x1.000); the table is profiles/pmc_traffic_plain_batch32_4096sq.md.
 MEASURED_TRAFFIC_PER_IMAGE = {
-    "k_rescale_rows_r2c": 123.08e6, "k_transpose_c": 112.03e6, "k_rescale_cols": 104.02e6,
-    "k_rescale_rows_c2r": 93.65e6, "k_tile_rows": 196.52e6, "k_tile_cols": 165.41e6,
+    "k_rescale_rows_r2c": 126.55e6, "k_rescale_cols": 103.76e6,
+    "k_rescale_rows_c2r": 93.52e6, "k_tile_rows": 197.63e6, "k_tile_cols": 156.80e6,
 }
 
 # Wave64 VALU instructions per 4096x4096 micrograph at 1.0 A (rocprofv3 --pmc
@@ -59,19 +59,19 @@ MEASURED_TRAFFIC_PER_IMAGE = {
 # measured against: one wave64 FP32 instruction per CU per cycle (a
 # microbenchmark of independent FMA/add/multiply chains reaches 0.97).
 MEASURED_VALU_INSTR_PER_IMAGE = {
-    "k_rescale_rows_r2c": 9.380e6, "k_rescale_cols": 36.724e6, "k_rescale_rows_c2r": 32.100e6,
+    "k_rescale_rows_r2c": 10.248e6, "k_rescale_cols": 26.395e6, "k_rescale_rows_c2r": 25.939e6,
 }
 VALU_ISSUE_PEAK = 256 * 2.4e9          # wave64 instructions per second
 
 # Spectrum-stage kernels (rescale a2, tile spectrum a5-a10, background a11,
 # gate a12, low-pass a13) and their measured HBM bytes per micrograph from the
 # same PMC table (the small kernels' launches there cover 32 or 16 micrographs).
-SPECTRUM_KERNELS = ("k_rescale_rows_r2c", "k_transpose_c", "k_rescale_cols", "k_rescale_rows_c2r",
+SPECTRUM_KERNELS = ("k_rescale_rows_r2c", "k_rescale_cols", "k_rescale_rows_c2r",
                     "k_row_sums", "k_block_rows", "k_tile_rows", "k_tile_cols", "k_tile_reduce",
                     "k_bg_rows", "k_bg_cols", "k_gate", "k_lp_x", "k_lp_y")
 MEASURED_TRAFFIC_SMALL_PER_IMAGE = {
-    "k_block_rows": 0.24e6, "k_tile_reduce": 2.63e6, "k_bg_rows": 1.57e6, "k_bg_cols": 5.29e6,
-    "k_gate": 0.01e6, "k_lp_x": 1.61e6, "k_lp_y": 7.21e6,
+    "k_block_rows": 0.45e6, "k_tile_reduce": 4.74e6, "k_bg_rows": 1.21e6, "k_bg_cols": 3.01e6,
+    "k_gate": 0.00e6, "k_lp_x": 1.60e6, "k_lp_y": 3.55e6,
 }
 
 
@@ -86,14 +86,12 @@ def spectrum_bytes_per_image(nx, ny, in_bytes, nnx, nny, rescaled, tile=512):
     return b + 4 * (tile // 2 + 1) * tile * 4
 
 
-# Arithmetic of the FFT kernels per micrograph (5 N log2 N per complex
-# transform of length N, 6 per complex multiply, 16 per radix-4 butterfly):
-# k_rescale_cols runs 1707 columns of FFT 4096 + an inverse of 3412 = 4 x 853
-# as four 853-point Bluestein transforms (each two FFTs of 2048 and three
-# pointwise products of 2048) joined by 853 radix-4 butterflies with three
-# twiddle products each.
+# FFT flops of the largest spectrum kernel per 4096x4096 micrograph at 1.0 A:
+# 1707 columns of a 4096-point transform, two 4096-point transforms of the
+# 3412-point inverse's fine grid with their mode factors (6 per mode and
+# half), and 8 complex-by-real multiply-adds per output.
 FFT_FLOP_PER_IMAGE = {
-    "k_rescale_cols": 1707 * (5 * 4096 * 12 + 4 * (2 * 5 * 2048 * 11 + 3 * 6 * 2048) + 853 * (3 * 6 + 16)),
+    "k_rescale_cols": 1707 * (3 * 5 * 4096 * 12 + 2 * 6 * 3412 + 3412 * 8 * 4),
 }
 
 
@@ -515,8 +513,6 @@ def kernel_bytes(name, g, per_launch_images, nsplit=8):
     c = per_launch_images
     if name == "k_rescale_rows_r2c":
         b = g["ny"] * g["nx"] * 4 + g["ny"] * g["ncx"] * 8
-    elif name == "k_transpose_c":
-        b = 2 * g["ny"] * g["ncx"] * 8          # the ny x ncx row spectrum read and written transposed
     elif name == "k_rescale_cols":
         b = g["ncx"] * g["ny"] * 8 + g["ncx"] * g["nny"] * 8
     elif name == "k_rescale_rows_c2r":
@@ -544,15 +540,11 @@ def roofline(ctx, ptr, n, a, run, tuned=None):
     run()
     rep = ctx.profile_report()
     ctx.profile(False)
-    chunk = min(tuned["chunk"] if tuned else (a.chunk or 4), n)
     nsplit = tuned["tile_splits"] if tuned else (a.splits or 8)
-    batch_kernels = {"k_tile_reduce"}
     rows = {}
     for name, (tot, cnt) in rep.items():
-        per = chunk if name.startswith(("k_rescale", "k_transpose", "k_block", "k_tile_rows",
-                                        "k_tile_cols")) else n
-        if name in batch_kernels:
-            per = chunk
+        # spectrum launches cover part of the batch, each micrograph once
+        per = n / cnt if name.split("<")[0] in SPECTRUM_KERNELS else n
         avg_ms = tot / cnt
         nb = kernel_bytes(name, g, per, nsplit)
         rows[name] = dict(ms_total=round(tot, 3), launches=cnt, avg_us=round(avg_ms * 1e3, 2),
@@ -588,12 +580,12 @@ def roofline(ctx, ptr, n, a, run, tuned=None):
     # the largest spectrum kernel on its own
     hbm = {k: v for k, v in rows.items() if v["gbs"] is not None}
     dom = max(hbm, key=lambda k: hbm[k]["ms_total"])
-    per = chunk
+    per = n / rows[dom]["launches"]
     nb = kernel_bytes(dom, g, per, nsplit)
     pk = {"kernel": dom, "achieved": round(nb / (rows[dom]["avg_us"] * 1e-6) / 1e9, 1), "peak": HBM_PEAK_GBS,
           "unit": "GB/s", "algorithmic_bytes_per_launch": int(nb), "avg_launch_us": rows[dom]["avg_us"],
-          "note": "this kernel's compulsory input reads and output writes per launch (the transposed "
-                  "spectrum in, the cropped columns out) over its average launch"}
+          "note": "this kernel's compulsory input reads and output writes per launch "
+                  "over its average launch"}
     pk["frac"] = round(pk["achieved"] / HBM_PEAK_GBS, 4)
     base = dom.split("<")[0]
     t1 = MEASURED_TRAFFIC_PER_IMAGE.get(base) if std else None
@@ -604,7 +596,8 @@ def roofline(ctx, ptr, n, a, run, tuned=None):
         pk["valu"] = {"achieved": round(tf, 1), "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
                       "frac": round(tf / VALU_PEAK_TFLOPS, 4), "flop_per_launch": int(fl * per),
                       "note": "FFT-bound: 5 N log2 N per complex transform of the transforms run (FFT 4096; "
-                              "four 853-point Bluestein transforms on 2048 joined by radix-4 butterflies)"}
+                              "two 4096-point transforms per 3412-point one on the fine grid) and the "
+                              "grid's interpolation"}
     vi = MEASURED_VALU_INSTR_PER_IMAGE.get(base) if std else None
     if vi:
         rate = vi * per / (rows[dom]["avg_us"] * 1e-6)
