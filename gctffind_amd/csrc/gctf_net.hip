@@ -575,8 +575,8 @@ hipError_t forward_bf16(NetBuffers* nb, const float* prm, const float* radial, i
 {
 	const bool tr = target != nullptr;
 	auto sg = [&](int l) { return tr ? layer_signs(nb, B, l) : nullptr; };
-	k_net_weights<<<((tr ? kFragTotal : kFragFc1Back) + 3) / 4, 256, 0, s>>>(prm, tr ? 1 : 0, nb->frag);
-	k_net_front<<<B, 256, 0, s>>>(radial, ld, prm, B, nb->x0, nb->a1, sg(0));
+	k_net_front<<<B + ((tr ? kFragTotal : kFragFc1Back) + 3) / 4, 256, 0, s>>>(radial, ld, prm, B, nb->x0, nb->a1,
+		sg(0), tr ? 1 : 0, nb->frag);
 	const uint4* fr = nb->frag;
 	const long long layer = 2LL * kFragConv * 64;
 	launch_conv<kNetBins / 2>(nb, nb->a1, fr, prm + kNetB2, B, nb->a2, sg(1), s);

@@ -1,5 +1,5 @@
-// k_net.hpp -- BF16 kernels of the defocus-proposal network: six launches
-// for a forward pass, eleven for a training step.
+// k_net.hpp -- BF16 kernels of the defocus-proposal network: five launches
+// for a forward pass, ten for a training step.
 //
 // The layers are too small to fill the chip one matrix at a time (conv2 of a
 // batch of 256 is 1.9 GFLOP), so what bounds them is launches and passes over
@@ -60,11 +60,10 @@ constexpr int kFragFc1Count = (kNetFlat / 16) * (kNetHidden / 32);
 constexpr int kFragFc1Back = kFragFc1 + kFragFc1Count;
 constexpr int kFragTotal = kFragFc1Back + kFragFc1Count;
 
-// Grid (ceil(fragments / 4)), a wave per fragment; directions 1 only when back.
-__global__ __launch_bounds__(256) void k_net_weights(const float* __restrict__ prm, int back,
-	uint4* __restrict__ frag)
+// Fragments 4 block .. + 3, a wave each; directions 1 only when back.
+__device__ __forceinline__ void net_weights(const float* __restrict__ prm, int back, uint4* __restrict__ frag, int block)
 {
-	const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+	const int f = block * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
 	const int row = lane & 31, h = lane >> 5;
 	if (f >= (back ? kFragTotal : kFragFc1Back)) return;
 	float v[8];
@@ -102,18 +101,18 @@ __device__ __forceinline__ nbf16x8 load_frag(const uint4* __restrict__ frag, int
 }
 
 // ---------------------------------------------------------------------------
-// Input z-score, conv1 (1 -> 64, 7 taps), bias, ReLU and pool.  One workgroup
-// per spectrum; thread = pooled position, half of the channels.  a1 the pooled
-// outputs, m1 the signs of the two pooled activations (bits 0 and 1).
+// Input z-score, conv1 (1 -> 64, 7 taps), bias, ReLU and pool of spectrum b;
+// thread = pooled position, half of the channels.  a1 the pooled outputs, m1 the
+// signs of the two pooled activations (bits 0 and 1).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ radial, int ld,
+__device__ __forceinline__ void net_front(const float* __restrict__ radial, int ld,
 	const float* __restrict__ prm, int B, float* __restrict__ x0, float* __restrict__ a1,
-	unsigned char* __restrict__ m1)
+	unsigned char* __restrict__ m1, int b)
 {
 	__shared__ double r1[256], r2[256];
 	__shared__ float xs[kNetBins + 8];
 	__shared__ float ws[kNetCh * (kNetTaps + 1)];         // weights, then biases
-	const int b = blockIdx.x, t = threadIdx.x;
+	const int t = threadIdx.x;
 	for (int i = t; i < kNetCh * (kNetTaps + 1); i += 256) ws[i] = prm[kNetW1 + i];
 	static_assert(kNetB1 == kNetW1 + kNetCh * kNetTaps, "weights and biases are neighbours");
 	const float v = radial[(long long)b * ld + t];
@@ -155,6 +154,18 @@ __global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ rad
 		a1[o] = 0.5f * (y[0] + y[1]);
 		if (m1) m1[o] = (unsigned char)((y[0] > 0.f ? 1 : 0) | (y[1] > 0.f ? 2 : 0));
 	}
+}
+
+// The pass's first launch: workgroups 0 .. B - 1 a spectrum each, the others the
+// weight fragments, which only the following launches read.  Launches of their own
+// cost proposals of 32 spectra 4 us of 77.
+__global__ __launch_bounds__(256) void k_net_front(const float* __restrict__ radial, int ld,
+	const float* __restrict__ prm, int B, float* __restrict__ x0, float* __restrict__ a1,
+	unsigned char* __restrict__ m1, int back, uint4* __restrict__ frag)
+{
+	const int b = blockIdx.x;
+	if (b < B) net_front(radial, ld, prm, B, x0, a1, m1, b);
+	else net_weights(prm, back, frag, b - B);
 }
 
 // ---------------------------------------------------------------------------
@@ -391,7 +402,15 @@ __global__ __launch_bounds__(1024) void k_net_fc(const float* __restrict__ a4, c
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int row = lane & 31, hf = lane >> 5;
 	const int b0 = blockIdx.x * NB;
-	const int bl = min(b0 + row, B - 1);
+	// the tile's inputs, read once for the four hidden tiles: row = spectrum
+	constexpr int XP = kNetFlat + 8;
+	__shared__ __attribute__((aligned(16))) __bf16 fs[NB * XP];
+#pragma unroll
+	for (int i = 0; i < kNetFlat * NB / 4 / 1024; ++i) {
+		const int e = tid + i * 1024, q = e % 4, b = e / 4 % NB, c = e / (4 * NB);
+		const float4 v = *reinterpret_cast<const float4*>(a4 + ((long long)c * B + min(b0 + b, B - 1)) * kNetL4 + 4 * q);
+		*reinterpret_cast<uint2*>(fs + b * XP + c * kNetL4 + 4 * q) = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
+	}
 	if (tid < kNetOut * (kNetHidden + 1)) w6[tid] = prm[kNetW6 + tid];
 	{
 		// quarter ks of the slices to wave group ks, where it holds whole
@@ -399,13 +418,10 @@ __global__ __launch_bounds__(1024) void k_net_fc(const float* __restrict__ a4, c
 		const int jt = wave & 3, ks = wave >> 2;
 		constexpr int NK = kNetFlat / 16, QK = NK / 4;
 		auto slice = [&](int c, nfloatx16 acc) {             // channel c: inputs 16 c .. 16 c + 15
-			const float4* src = reinterpret_cast<const float4*>(a4 + ((long long)c * B + bl) * kNetL4 + 8 * hf);
-			const float4 u = src[0], v = src[1];
-			const uint4 x = make_uint4(pack_bf16(u.x, u.y), pack_bf16(u.z, u.w), pack_bf16(v.x, v.y),
-				pack_bf16(v.z, v.w));
-			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_frag(frag, kFragFc1 + c * 4 + jt, lane),
-				__builtin_bit_cast(nbf16x8, x), acc, 0, 0, 0);
+			const nbf16x8 x = *reinterpret_cast<const nbf16x8*>(fs + row * XP + c * kNetL4 + 8 * hf);
+			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_frag(frag, kFragFc1 + c * 4 + jt, lane), x, acc, 0, 0, 0);
 		};
+		__syncthreads();
 		nfloatx16 zero, acc;
 #pragma unroll
 		for (int r = 0; r < 16; ++r) zero[r] = 0.f;
