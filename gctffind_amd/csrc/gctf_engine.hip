@@ -315,7 +315,7 @@ struct gctf_ctx {
 	// images per launch of the spectrum stage: 32 x 4096^2 take 8246 us with 1,
 	// 7707 with 4, 7531 with 8, 7459 with 16 (and twice the memory)
 	int chunk = 8, tile_splits = 8, use_graph = 1;
-	int cpb = 8;          // candidates per 2D-evaluator workgroup (search blocking: 4, 8 or 16)
+	int cpb = 8;          // search blocking: most candidates per 2D-evaluator workgroup (2, 4, 8 or 16)
 	int list_queue = 1;   // tile row pass of a list: 1 persistent workgroups on a work queue, 0 one item each
 	int tune_gen = 0;     // bumped by gctf_autotune (list graphs read the tuned values)
 	float scan_lo = 0, scan_hi = 0, scan_step = 0;  // Do1D scan (gctf_set_search1d; 0: reference)

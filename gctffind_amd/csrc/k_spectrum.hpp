@@ -31,7 +31,9 @@ __device__ __forceinline__ int xcd_group(int b, int n)
 // W-th value of a contiguous range.  Both sides then move whole lines or find
 // the rest of them in their XCD's L2, where the neighbouring workgroups
 // (xcd_group) work on it, and no transpose runs in between (19.5 us of 267 us
-// for a 4096^2 micrograph).
+// for a 4096^2 micrograph).  Wider panels help the rows and cost the columns:
+// 32 x 4096^2 spectra took 8152 us with widths 2 and 4, 7972 with 4 and 4, 8086
+// with 4 and 8, 8088 with 8 and 4, 8240 with 4 and 2.
 constexpr int kPanelIn = 4;      // after the rows' R2C, before the columns
 constexpr int kPanelOut = 4;     // after the columns, before the rows' C2R
 template <int W>
