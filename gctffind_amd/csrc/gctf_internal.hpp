@@ -95,6 +95,55 @@ struct SearchState {
 	int s1_ndf, s1_n, s1_stage;
 };
 
+__host__ __device__ __forceinline__ void step_program(SearchProgram& d, const SearchProgram& s)
+{
+	d.n_ast = s.n_ast; d.n_ang = s.n_ang; d.n_mag = s.n_mag; d.n_angl = s.n_angl;
+	d.n_df = s.n_df; d.iters = s.iters; d.df_minstep = s.df_minstep;
+	d.fine_n = s.fine_n; d.fine_step = s.fine_step;
+}
+
+// The fields of a state that a transition reads or writes, one by one (a
+// struct assignment would keep the copy in memory instead of registers).
+__host__ __device__ __forceinline__ void step_fields(SearchState& d, const SearchState& s)
+{
+	d.df_min = s.df_min; d.df_max = s.df_max; d.ast_ang = s.ast_ang; d.ext_phase = s.ext_phase; d.score = s.score;
+	d.phase_range = s.phase_range;
+	d.dfmean = s.dfmean; d.ast = s.ast; d.ang = s.ang; d.phase = s.phase; d.ccmax = s.ccmax; d.oldcc = s.oldcc;
+#pragma unroll
+	for (int i = 0; i < 2; ++i) {
+		d.dfrange[i] = s.dfrange[i]; d.astrange[i] = s.astrange[i];
+		d.angrange[i] = s.angrange[i]; d.phrange[i] = s.phrange[i];
+	}
+	d.tot_df = s.tot_df; d.tot_ast = s.tot_ast; d.tot_ang = s.tot_ang;
+	d.done = s.done; d.iter = s.iter; d.skip = s.skip;
+	d.st_kind = s.st_kind; d.st_n = s.st_n; d.st_nast = s.st_nast;
+	d.st_a0 = s.st_a0; d.st_astep = s.st_astep; d.st_b0 = s.st_b0; d.st_bstep = s.st_bstep;
+	d.st_lo = s.st_lo; d.st_hi = s.st_hi; d.st_old = s.st_old;
+	step_program(d.pg, s.pg);
+}
+
+// The other fields: a transition only carries them over.
+__host__ __device__ __forceinline__ void step_kept(SearchState& d, const SearchState& s)
+{
+	d.ctf_res = s.ctf_res;
+	d.lowpassed = s.lowpassed;
+	d.fallback = s.fallback; d.conf = s.conf;
+	d.s1_df0 = s.s1_df0; d.s1_dfstep = s.s1_dfstep; d.s1_ph0 = s.s1_ph0; d.s1_phstep = s.s1_phstep;
+	d.s1_ndf = s.s1_ndf; d.s1_n = s.s1_n; d.s1_stage = s.s1_stage;
+}
+
+// The new state s of a transition from `in` into `out` (which may be `in`) by
+// the lanes of one wavefront.  One lane stores every field, once and by its
+// name: lanes have no order among themselves, and neither have stores to one
+// address through different types.
+__host__ __device__ __forceinline__ void step_store(SearchState* out, const SearchState* in, const SearchState& s,
+	int lane)
+{
+	if (lane != 0) return;
+	step_fields(*out, s);
+	if (out != in) step_kept(*out, *in);
+}
+
 // Per-plan 2D-ring tables in structure-of-arrays form (device pointers).
 struct RingTables {
 	int n;                 // ring pixel count

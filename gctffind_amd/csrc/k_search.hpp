@@ -637,44 +637,6 @@ __device__ __forceinline__ void advance_state(SearchState& s, int prev_kind, int
 	}
 }
 
-__device__ __forceinline__ void step_program(SearchProgram& d, const SearchProgram& s)
-{
-	d.n_ast = s.n_ast; d.n_ang = s.n_ang; d.n_mag = s.n_mag; d.n_angl = s.n_angl;
-	d.n_df = s.n_df; d.iters = s.iters; d.df_minstep = s.df_minstep;
-	d.fine_n = s.fine_n; d.fine_step = s.fine_step;
-}
-
-// The fields of a state that a transition reads or writes, one by one (a
-// struct assignment would keep the copy in memory instead of registers).
-__device__ __forceinline__ void step_fields(SearchState& d, const SearchState& s)
-{
-	d.df_min = s.df_min; d.df_max = s.df_max; d.ast_ang = s.ast_ang; d.ext_phase = s.ext_phase; d.score = s.score;
-	d.phase_range = s.phase_range;
-	d.dfmean = s.dfmean; d.ast = s.ast; d.ang = s.ang; d.phase = s.phase; d.ccmax = s.ccmax; d.oldcc = s.oldcc;
-#pragma unroll
-	for (int i = 0; i < 2; ++i) {
-		d.dfrange[i] = s.dfrange[i]; d.astrange[i] = s.astrange[i];
-		d.angrange[i] = s.angrange[i]; d.phrange[i] = s.phrange[i];
-	}
-	d.tot_df = s.tot_df; d.tot_ast = s.tot_ast; d.tot_ang = s.tot_ang;
-	d.done = s.done; d.iter = s.iter; d.skip = s.skip;
-	d.st_kind = s.st_kind; d.st_n = s.st_n; d.st_nast = s.st_nast;
-	d.st_a0 = s.st_a0; d.st_astep = s.st_astep; d.st_b0 = s.st_b0; d.st_bstep = s.st_bstep;
-	d.st_lo = s.st_lo; d.st_hi = s.st_hi; d.st_old = s.st_old;
-	step_program(d.pg, s.pg);
-}
-
-// The new state s of a transition from `in` into `out` by the lanes of one
-// wavefront: the words of `in`, then the transition's fields over them.
-__device__ __forceinline__ void step_store(SearchState* out, const SearchState* in, const SearchState& s, int lane)
-{
-	static_assert(sizeof(SearchState) % 4 == 0, "copied by words");
-	if (out != in)
-		for (int i = lane; i < (int)(sizeof(SearchState) / 4); i += 64)
-			reinterpret_cast<int*>(out)[i] = reinterpret_cast<const int*>(in)[i];
-	if (lane == 0) step_fields(*out, s);
-}
-
 // The transitions that start a 2D search from the 1D result or a proposal.
 __device__ __forceinline__ void step_begin(SearchState& s, int next, const RefineArgs* refine, const SearchProgram& prog)
 {
@@ -934,7 +896,8 @@ __global__ __launch_bounds__(256) void k_s2d_step(StepArgs sa)
 	SearchState s;
 	step_fields(s, sa.st_in[img]);
 	if (s.skip) {
-		if (tid < 64) step_store(sa.st_out + img, sa.st_in + img, s, tid);
+		// unchanged: nothing to store in place, where other waves may still read
+		if (tid < 64 && sa.st_out != sa.st_in) step_store(sa.st_out + img, sa.st_in + img, s, tid);
 		return;
 	}
 	const bool ran = !s.done && s.st_kind != ST_NONE && s.st_n > 0;
