@@ -938,8 +938,9 @@ __global__ __launch_bounds__(256) void k_bg_rows(const float* __restrict__ raw, 
 }
 
 // Column sums, the subtraction, the r < 0.04 zeroing (evaluated in float as
-// the reference does) and per-workgroup moment partials for the gate (an
-// FP32 tree within the workgroup; k_gate adds the partials in FP64).
+// the reference does) and per-workgroup moment partials for the gate, in FP64
+// as in k_gate: FP32 sums decide the gate wrongly where the variance is within
+// 1e-7 of its threshold.
 // kBgCols columns x 8 kBgRun rows per workgroup, grid (bg_col_groups, images).
 constexpr int kBgCols = 32;
 template <int T>
@@ -952,7 +953,7 @@ __global__ __launch_bounds__(256) void k_bg_cols(const float* __restrict__ raw,
 	constexpr int CX = T / 2 + 1, HB = bg_half<T>(), CG = (CX + kBgCols - 1) / kBgCols;
 	constexpr int RY = 8 * kBgRun, N = RY + 2 * HB;
 	__shared__ float p[N * kBgCols];
-	__shared__ float r1[256], r2[256];
+	__shared__ double red[2][4];
 	const int x0 = blockIdx.x % CG * kBgCols, y0 = blockIdx.x / CG * RY;
 	const float* in = raw + (long long)blockIdx.y * T * CX;
 	const float* h = hsum + (long long)blockIdx.y * T * CX;
@@ -961,7 +962,7 @@ __global__ __launch_bounds__(256) void k_bg_cols(const float* __restrict__ raw,
 	for (int r = threadIdx.x / kBgCols; r < N; r += 256 / kBgCols)
 		p[r * kBgCols + c] = h[((y0 + r - HB + T) & (T - 1)) * CX + min(x, CX - 1)];
 	__syncthreads();
-	float m1 = 0.0f, m2 = 0.0f;
+	double m1 = 0.0, m2 = 0.0;
 	if (x < CX) {
 		const int l0 = threadIdx.x / kBgCols * kBgRun;
 		float s[kBgRun];
@@ -976,19 +977,16 @@ __global__ __launch_bounds__(256) void k_bg_cols(const float* __restrict__ raw,
 			if (!log_spect) acc *= acc;
 			const float o = (double)fr < 0.04 ? 0.f : in[y * CX + x] - acc;
 			spect[(long long)blockIdx.y * T * CX + y * CX + x] = o;
-			m1 += o;
-			m2 += o * o;
+			m1 += (double)o;
+			m2 += (double)o * o;
 		}
 	}
-	r1[threadIdx.x] = m1; r2[threadIdx.x] = m2;
+	for (int s = 32; s > 0; s >>= 1) { m1 += __shfl_xor(m1, s); m2 += __shfl_xor(m2, s); }
+	if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x >> 6] = m1; red[1][threadIdx.x >> 6] = m2; }
 	__syncthreads();
-	for (int s = 128; s > 0; s >>= 1) {
-		if (threadIdx.x < s) { r1[threadIdx.x] += r1[threadIdx.x + s]; r2[threadIdx.x] += r2[threadIdx.x + s]; }
-		__syncthreads();
-	}
-	if (threadIdx.x == 0) {
-		double* m = mom + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * 2;
-		m[0] = r1[0]; m[1] = r2[0];
+	if (threadIdx.x < 2) {
+		const double* r = red[threadIdx.x];
+		mom[((long long)blockIdx.y * gridDim.x + blockIdx.x) * 2 + threadIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
 	}
 }
 
