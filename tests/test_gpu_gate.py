@@ -4,6 +4,8 @@ removed spectrum o is at least 1 in single precision (CFindCtfBase.cpp:
 import numpy as np
 import pytest
 
+import oracle as O
+
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
@@ -86,3 +88,16 @@ def test_gate_at_its_threshold(tile):
         assert want == (not np.array_equal(half, o)), (k, np.var(o.astype(np.float64)) - 1.0)
         decided.append(want)
     assert any(decided) and not all(decided)
+
+
+@pytest.mark.parametrize("tile", [256, 512, 1024])
+@pytest.mark.parametrize("log_spect", [False, True])
+def test_background_without_lowpass(tile, log_spect):
+    """All three tile sizes on the side of the gate where nothing is filtered."""
+    ctx = _context(tile, log_spect)
+    raw, half = _spectra(ctx, 1e-3 * _image(tile, 3 * tile + log_spect))
+    ref = O.rm_background(raw.astype(np.float64), log_spect=int(log_spect))
+    assert O.gate(ref) == 0
+    # FP32 sums of up to 69 x 69 values: below 69 x 6e-8 of the background,
+    # a part of the raw spectrum
+    assert np.linalg.norm(half - ref) <= 5e-6 * np.linalg.norm(raw)
