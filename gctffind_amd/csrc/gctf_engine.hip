@@ -351,6 +351,7 @@ struct gctf_ctx {
 	DevBuf rjobs, rtab, list_plans, qnext;   // its rescale jobs, class tables, plans, work-queue counters
 	DevBuf raw, hsum, spect, mom, q, radial, ring_spec, ring_ss, states, part2d, refine, states2, fullsp,
 		moments1, plans, shell_bins;
+	DevBuf search_map, states_part;   // a search pass on part of a batch
 	int kstride = 0;  // ring pixels reserved per image in ring_spec
 	DevBuf g_bt, g_fn, g_gt, g_cc, g_part, g_top, g_rs, g_rescored;
 	// learned path: proposal-network parameters, activations, outputs
@@ -1168,6 +1169,7 @@ struct Search2DView {
 	const int *boff, *bcnt, *bidx;
 	int nbins;
 	int T, cx, kstride;
+	const int* map = nullptr;   // spectrum numbers of a pass on part of a batch (null: all)
 };
 
 Search2DView view_2d(gctf_ctx* c, int T, int i0)
@@ -1205,7 +1207,7 @@ int run_2d_program(gctf_ctx* c, const Search2DView& v, int m, int begin, const S
 {
 	hipStream_t s = c->stream;
 	PROF(c, "k_ring_gather", k_ring_gather<<<dim3(kRingParts, m), 256, 0, s>>>(v.spect, v.T * v.cx, v.plans, v.kstride,
-		v.ring_spec, v.ring_ss));
+		v.map, v.ring_spec, v.ring_ss));
 	// Transitions go from one copy of the states to the other, stages from one
 	// half of the sums to the other.
 	SearchState* cur = v.st;
@@ -1280,7 +1282,7 @@ int run_2d_program(gctf_ctx* c, const Search2DView& v, int m, int begin, const S
 #undef GCTF_TR
 	alt = v.st;                              // the last transition ends in the caller's states
 	step(next, next2);
-	PROF(c, "k_shell_bins", k_shell_bins<<<dim3(v.nbins, m), 64, 0, s>>>(v.plans, v.spect, v.cx, v.T, v.boff,
+	PROF(c, "k_shell_bins", k_shell_bins<<<dim3(v.nbins, m), 64, 0, s>>>(v.plans, v.spect, v.map, v.cx, v.T, v.boff,
 		v.bcnt, v.bidx, v.nbins, v.st, v.bins));
 	PROF(c, "k_ctf_res", k_ctf_res<<<m, 256, 0, s>>>(v.bins, v.nbins, v.cx, v.T, 10, v.plans, v.st));
 	HIPCHK(c, hipGetLastError());
@@ -1291,6 +1293,23 @@ int run_2d_program(gctf_ctx* c, const Search2DView& v, int m, int begin, const S
 int launch_2d(gctf_ctx* c, int T, int i0, int m, int begin, float phase_range)
 {
 	return run_2d_program(c, view_2d(c, T, i0), m, begin, plain_program(), phase_range);
+}
+
+// CFindDefocus2D::DoIt (plain program) for the micrographs that map names
+// (device, n entries, -1: none) of a batch with one search plan, the 1D search
+// done.  Launches for all of the batch, with the others leaving at once, cost
+// more than the search itself where few take part: a learned batch of 256
+// with 14 fallbacks took 17.1 ms and one with 59 25.1 ms, 8.3 and 11.3 so.
+int launch_2d_some(gctf_ctx* c, int T, const int* map, int n, float phase_range)
+{
+	Search2DView v = view_2d(c, T, 0);
+	v.st = c->states_part.as<SearchState>();
+	v.map = map;
+	PROF(c, "k_states_take", k_states_take<<<(n + 63) / 64, 64, 0, c->stream>>>(c->states.as<SearchState>(), map, n, v.st));
+	CHK(run_2d_program(c, v, n, NX_BEGIN_DO2D, plain_program(), phase_range));
+	PROF(c, "k_states_put", k_states_put<<<(n + 63) / 64, 64, 0, c->stream>>>(v.st, map, n, c->states.as<SearchState>()));
+	HIPCHK(c, hipGetLastError());
+	return GCTF_OK;
 }
 
 // ---- learned path --------------------------------------------------------
@@ -2410,20 +2429,27 @@ int gctf_estimate_batch_learned(gctf_ctx* ctx, const void* dev_imgs, int dtype, 
 		CHK(get_tile_tables(ctx, ctx->prm.tile_size, &tt));
 		const float range = std::max(ctx->prm.ext_phase_range_deg, 0.0f);
 		SearchState* st = ctx->states.as<SearchState>();
-		// one graph for every fallback pattern: which micrographs sit out is data
+		// one graph for every fallback pattern of at most n, n / 2, n / 4, ...
+		// micrographs: which ones they are is data
 		TuneScope tune(ctx, nx, ny, dtype, pix);
-		// few micrographs take part: smaller candidate blocks put more
-		// workgroups on the chip (the results do not depend on the blocking)
-		if (4 * nfb <= n) ctx->cpb = 2;
-		else if (2 * nfb <= n) ctx->cpb = std::min(ctx->cpb, 4);
+		int some = n;
+		while (some / 2 >= nfb) some /= 2;
+		std::vector<int> map;
+		for (int i = 0; i < n; ++i)
+			if (fb[i]) map.push_back(i);
+		map.resize((size_t)some, -1);
+		CHK(ensure_buf(ctx, ctx->search_map, sizeof(int) * (size_t)n));
+		CHK(ensure_buf(ctx, ctx->states_part, sizeof(SearchState) * (size_t)n));
+		HIPCHK(ctx, hipMemcpyAsync(ctx->search_map.p, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice,
+			ctx->stream));
 		char fkey[160];
-		snprintf(fkey, sizeof fkey, "fallback/%d/%d/%a/%a/%a/%d", n, ctx->prm.tile_size, sp->pix, range,
-			ctx->prm.ext_phase_deg, ctx->cpb);
+		snprintf(fkey, sizeof fkey, "fallback/%d/%d/%a/%a/%a/%d/%d", n, ctx->prm.tile_size, sp->pix, range,
+			ctx->prm.ext_phase_deg, ctx->cpb, some);
 		CHK(run_graph(ctx, fkey, [&]() -> int {
 			k_fallback_prepare<<<(n + 63) / 64, 64, 0, ctx->stream>>>(st, n, ctx->prm.ext_phase_deg, range);
 			CHK(fill_plans(ctx, 0, n, *sp));
 			CHK(launch_1d(ctx, *tt, 0, n, 0, 0.f, 0.f, range > 0.0f));
-			CHK(launch_2d(ctx, ctx->prm.tile_size, 0, n, NX_BEGIN_DO2D, range));
+			CHK(launch_2d_some(ctx, ctx->prm.tile_size, ctx->search_map.as<int>(), some, range));
 			k_clear_skip<<<(n + 63) / 64, 64, 0, ctx->stream>>>(st, n);
 			HIPCHK(ctx, hipGetLastError());
 			return GCTF_OK;
@@ -2600,6 +2626,7 @@ int gctf_estimate_series(gctf_ctx* ctx, const void* dev_imgs, int dtype, int n, 
 		CHK(ensure_buf(ctx, ctx->padc, sizeof(float) * (size_t)rp.pitch * rp.nny * C));
 	}
 	CHK(ensure_buf(ctx, ctx->series, sizeof(SeriesCtl) + sizeof(int) * (size_t)n));
+	CHK(ensure_buf(ctx, ctx->states_part, sizeof(SearchState)));
 	// CLoadImages.cpp:71-91: the zero-tilt package first, the others in order
 	const int z = tomo ? zero_tilt(tilts_deg, n) : 0;
 	const float p0 = ctx->prm.ext_phase_deg, range = std::max(ctx->prm.ext_phase_range_deg, 0.0f);
@@ -2632,7 +2659,7 @@ int gctf_estimate_series(gctf_ctx* ctx, const void* dev_imgs, int dtype, int n, 
 	// the full search of the package whose refine failed (the others sit out)
 	auto record_full = [&]() -> int {
 		CHK(launch_1d(ctx, *tt, 0, n, 0, 0.f, 0.f, ctx->prm.ext_phase_range_deg > 0.0f));
-		CHK(launch_2d(ctx, T, 0, n, NX_BEGIN_DO2D, range));
+		CHK(launch_2d_some(ctx, T, &ctl->full, 1, range));
 		k_series_after_full<<<1, 1, 0, ctx->stream>>>(st, ctl, n);
 		HIPCHK(ctx, hipGetLastError());
 		return GCTF_OK;

@@ -450,13 +450,17 @@ __device__ __forceinline__ double ring_energy(const double* __restrict__ ss)
 	return e;
 }
 
-// Grid (kRingParts, images).
+// Grid (kRingParts, images).  Image i's spectrum is number map[i], -1 for none
+// (map null: i).
 __global__ __launch_bounds__(256) void k_ring_gather(const float* __restrict__ spect, int npix,
-	const ImgPlan* __restrict__ plans, int kstride, float* __restrict__ ring_spec, double* __restrict__ ring_ss)
+	const ImgPlan* __restrict__ plans, int kstride, const int* __restrict__ map, float* __restrict__ ring_spec,
+	double* __restrict__ ring_ss)
 {
 	__shared__ double red[4];
+	const int src = map ? map[blockIdx.y] : (int)blockIdx.y;
+	if (src < 0) return;
 	const RingTables ring = plans[blockIdx.y].ring;
-	ring_gather(spect + (long long)blockIdx.y * npix, ring, ring_spec + (long long)blockIdx.y * kstride,
+	ring_gather(spect + (long long)src * npix, ring, ring_spec + (long long)blockIdx.y * kstride,
 		ring_ss + blockIdx.y * kRingParts, blockIdx.x, red);
 }
 
@@ -467,6 +471,28 @@ __global__ __launch_bounds__(256) void k_ring_gather_uniform(const float* __rest
 	__shared__ double red[4];
 	ring_gather(spect + (long long)blockIdx.y * npix, ring, ring_spec + (long long)blockIdx.y * ring.n,
 		ring_ss + blockIdx.y * kRingParts, blockIdx.x, red);
+}
+
+// The states of the micrographs that map names (-1: none, sits out) in
+// consecutive slots, for a search pass on part of a batch, and back.
+__global__ void k_states_take(const SearchState* __restrict__ st, const int* __restrict__ map, int n,
+	SearchState* __restrict__ part)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= n) return;
+	if (map[i] >= 0) {
+		part[i] = st[map[i]];
+	} else {
+		part[i] = SearchState{};
+		part[i].skip = 1;
+	}
+}
+
+__global__ void k_states_put(const SearchState* __restrict__ part, const int* __restrict__ map, int n,
+	SearchState* __restrict__ st)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n && map[i] >= 0) st[map[i]] = part[i];
 }
 
 // ---- controller -----------------------------------------------------------
@@ -934,9 +960,10 @@ __global__ __launch_bounds__(256) void k_s2d_step(StepArgs sa)
 // every bin, radii in the kernel's float arithmetic), and each shell adds
 // its bins.  A pixel is in one bin, so its CTF (FP32, the reference formula,
 // GCalcCTF2D.cu:23-37) is formed where it is summed.
-// Grid (nbins, images), one wavefront per bin; bins[image][bin][6].
+// Grid (nbins, images), one wavefront per bin; bins[image][bin][6]; map as in
+// k_ring_gather.
 __global__ __launch_bounds__(64) void k_shell_bins(const ImgPlan* __restrict__ plans, const float* __restrict__ spect,
-	int cmpx, int cmpy, const int* __restrict__ boff, const int* __restrict__ bcnt,
+	const int* __restrict__ map, int cmpx, int cmpy, const int* __restrict__ boff, const int* __restrict__ bcnt,
 	const int* __restrict__ bidx, int nbins, const SearchState* __restrict__ st, double* __restrict__ bins)
 {
 	const int b = blockIdx.x, img = blockIdx.y;
@@ -949,7 +976,7 @@ __global__ __launch_bounds__(64) void k_shell_bins(const ImgPlan* __restrict__ p
 	const float mean = 0.5f * (dmin + dmax), sig = 0.5f * (dmax - dmin);
 	const float add = cc.amp_phase + ph_rad;
 	const float w2 = cc.wl * cc.wl;
-	const float* sp = spect + (long long)img * cmpx * cmpy;
+	const float* sp = spect + (long long)(map ? map[img] : img) * cmpx * cmpy;
 	const int o = boff[b], n = bcnt[b];
 	double a[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll 4
