@@ -315,7 +315,7 @@ struct gctf_ctx {
 	// images per launch of the spectrum stage: 32 x 4096^2 take 8246 us with 1,
 	// 7707 with 4, 7531 with 8, 7459 with 16 (and twice the memory)
 	int chunk = 8, tile_splits = 8, use_graph = 1;
-	int cpb = 8;          // search blocking: most candidates per 2D-evaluator workgroup (2, 4, 8 or 16)
+	int cpb = 8;          // search blocking: most candidates per 2D-evaluator workgroup (2, 4, 8 or 16; run_2d_program)
 	int list_queue = 1;   // tile row pass of a list: 1 persistent workgroups on a work queue, 0 one item each
 	int tune_gen = 0;     // bumped by gctf_autotune (list graphs read the tuned values)
 	float scan_lo = 0, scan_hi = 0, scan_step = 0;  // Do1D scan (gctf_set_search1d; 0: reference)
@@ -1229,10 +1229,15 @@ int run_2d_program(gctf_ctx* c, const Search2DView& v, int m, int begin, const S
 	// the context's search blocking, whose workgroups all run at once.  A
 	// search of 16 spectra takes 1800 us so, and 2050 us with the largest
 	// block that still has 1024 workgroups (a second, mostly empty round); of
-	// one spectrum 585 us with blocks of 1 and 620 us with blocks of 2.
+	// one spectrum 585 us with blocks of 1 and 620 us with blocks of 2.  The
+	// kernels of blocks of 1 and 2 keep 8 pixels in flight, for one round of
+	// workgroups at 8 waves per CU: more workgroups than that take blocks of at
+	// least 4 whatever the search blocking (32 micrographs 8.1 ms in blocks of
+	// 2, 4.1 in blocks of 4).
 	auto block = [&](int maxc) {
+		const int most = std::max(c->cpb, 4);
 		int b = 1;
-		while (b < c->cpb && (long long)((maxc + b - 1) / b) * kPixChunks * m > kSearchWgs) b *= 2;
+		while (b < most && (long long)((maxc + b - 1) / b) * kPixChunks * m > kSearchWgs) b *= 2;
 		return b;
 	};
 #define GCTF_EVAL(CPB, U)                                                                                        \

@@ -206,9 +206,10 @@ GCTF_API int gctf_grid_search_batch(gctf_ctx* ctx, const void* dev_imgs, int dty
 	int* top_out, float* rescored_out);
 
 /* Knobs of the batched path (0 keeps the current value): images per
- * spectrum chunk, tile-column splits, graph use (1 on, -1 off), 2D search
- * blocking (candidates per evaluator workgroup: 2, 4, 8 or 16) and the tile
- * row pass of gctf_estimate_list (1: persistent workgroups on a work queue,
+ * spectrum chunk (default 8), tile-column splits, graph use (1 on, -1 off),
+ * 2D search blocking (the most candidates per evaluator workgroup: 2, 4, 8 or
+ * 16; fewer, down to 1, where the chip holds all workgroups at once, and up
+ * to 4 whatever the value where it does not) and the tile row pass of gctf_estimate_list (1: persistent workgroups on a work queue,
  * -1: one workgroup per item).  None of them changes results except the
  * tile splits (FP32 partial-sum grouping of the tile average). */
 GCTF_API int gctf_tune(gctf_ctx* ctx, int chunk, int tile_splits, int use_graph, int search_block,
@@ -252,7 +253,7 @@ GCTF_API int gctf_estimate_series(gctf_ctx* ctx, const void* dev_imgs, int dtype
 
 /* Time the spectrum stages of this batch for every (images per chunk, tile
  * splits) pair in {1, 2, 4, 8, 16} x {4, 8, 16}, then the plain search of
- * its spectra with 4, 8 and 16 candidates per 2D-evaluator workgroup, and
+ * its spectra with a search blocking of 4, 8 and 16 (gctf_tune), and
  * keep the fastest for this shape (nx, ny, dtype, pix): later batch,
  * series, learned and list calls of that shape use them (results do not
  * depend on the search blocking).  Outputs optional; best_ms is the

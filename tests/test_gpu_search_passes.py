@@ -70,3 +70,21 @@ def test_fallback_pass_on_part_of_a_batch():
             slow.append(report[-1])
     print("fallbacks, us of the pass, us of a plain batch:", report)
     assert not slow, slow
+
+
+def test_small_blocks_on_a_large_batch():
+    """A search blocking of 2 on a batch whose blocks of 2 do not fit the chip:
+    the same results, and no slower than 4 by more than a tenth."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gctffind_amd import gctf, proposal
+    im = _micrographs(proposal, N)
+    ctx = gctf.Context()
+    run = lambda: ctx.estimate_batch(im.data_ptr(), N, SIDE, SIDE, PIX)
+    res, t = {}, {}
+    for block in (4, 2, 8, 16):
+        ctx.tune(search_block=block)
+        res[block], t[block] = run(), _best(run)
+    print("search block: us", {b: round(x * 1e6) for b, x in t.items()})
+    assert res[2] == res[4] == res[8] == res[16]
+    assert t[2] <= 1.1 * t[4], t
