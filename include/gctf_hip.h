@@ -209,9 +209,10 @@ GCTF_API int gctf_grid_search_batch(gctf_ctx* ctx, const void* dev_imgs, int dty
  * spectrum chunk (default 8), tile-column splits, graph use (1 on, -1 off),
  * 2D search blocking (the most candidates per evaluator workgroup: 2, 4, 8 or
  * 16; fewer, down to 1, where the chip holds all workgroups at once, and up
- * to 4 whatever the value where it does not) and the tile row pass of gctf_estimate_list (1: persistent workgroups on a work queue,
- * -1: one workgroup per item).  None of them changes results except the
- * tile splits (FP32 partial-sum grouping of the tile average). */
+ * to 4 whatever the value where it does not) and the tile row pass of
+ * gctf_estimate_list (1: persistent workgroups on a work queue, -1: one
+ * workgroup per item).  None of them changes results except the tile splits
+ * (FP32 partial-sum grouping of the tile average). */
 GCTF_API int gctf_tune(gctf_ctx* ctx, int chunk, int tile_splits, int use_graph, int search_block,
 	int list_queue);
 
