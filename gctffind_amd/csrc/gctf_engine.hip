@@ -804,14 +804,6 @@ TileGrid make_grid(int nx, int ny, int T)
 	return g;
 }
 
-int check_tile(gctf_ctx* c, int T)
-{
-	if (T != 256 && T != 512 && T != 1024)
-		return fail(c, GCTF_ERR_UNSUPPORTED, "tile size " + std::to_string(T)
-			+ " not supported (256, 512 or 1024)");
-	return GCTF_OK;
-}
-
 // Workgroup maxima per image of a 1D brute-force stage: the largest stage
 // is the initial scan (the reference's 501 points, or the configured scan)
 // times 37 phases, or the refine stage (at most 501 x 37).

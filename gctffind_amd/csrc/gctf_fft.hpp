@@ -430,8 +430,8 @@ __device__ __forceinline__ void fft_regs(float2* buf, const TW& twf, int tid, fl
 }
 
 // In-place power-of-two FFT of the N logical elements of buf (padded
-// layout, fft_lds_len(N) entries) by NT threads.  With NT == 64 the threads
-// must form one wavefront and only they synchronise (fft_sync); otherwise
+// layout, fft_lds_len(N) entries) by NT threads.  With NT <= 64 the threads
+// must be in one wavefront and only they synchronise (fft_sync); otherwise
 // every thread of the workgroup must call it.  The data must be in buf and
 // visible (fft_sync<NT> or a barrier) before the call; results are visible
 // to the NT threads after.
@@ -439,13 +439,6 @@ template <int N, int NT, bool INV>
 __device__ __forceinline__ void fft_lds(float2* buf, const float2* __restrict__ tw, int tid)
 {
 	fft_run<N, 1, 0, NT, INV>(buf, TwTable{tw}, tid);
-}
-
-// The same with the twiddles already in registers (fft_tw_load).
-template <int N, int NT, bool INV>
-__device__ __forceinline__ void fft_lds(float2* buf, const TwRegs<N, NT>& w, int tid)
-{
-	fft_run<N, 1, 0, NT, INV>(buf, w, tid);
 }
 
 // ---- compile-time transform with input and output hooks -----------------
@@ -457,11 +450,7 @@ __device__ __forceinline__ void fft_lds(float2* buf, const TwRegs<N, NT>& w, int
 // fft_sync follows.  Loading and pointwise work before and after a transform
 // then cost no LDS round trip and no barrier of their own.
 
-// The plain input and output: buf itself.
-struct LdsIn {
-	const float2* buf;
-	__device__ __forceinline__ float2 operator()(int i) const { return buf[pidx(i)]; }
-};
+// The plain output: buf itself.
 struct LdsOut {
 	float2* buf;
 	__device__ __forceinline__ void operator()(int i, float2 v) const { buf[pidx(i)] = v; }
