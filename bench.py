@@ -49,8 +49,8 @@ VALU_PEAK_TFLOPS = 78.6   # FP32 FMA without packed math: 256 CU x 64 lanes x 2 
 # scaled by the same counters on a 256 MiB device copy (fetch x2.000,
 # write x1.000); the table is profiles/pmc_traffic_plain_batch32_4096sq.md.
 MEASURED_TRAFFIC_PER_IMAGE = {
-    "k_rescale_rows_r2c": 126.55e6, "k_rescale_cols": 103.76e6,
-    "k_rescale_rows_c2r": 93.52e6, "k_tile_rows": 197.63e6, "k_tile_cols": 156.80e6,
+    "k_rescale_rows_r2c": 126.68e6, "k_rescale_cols": 103.77e6,
+    "k_rescale_rows_c2r": 93.51e6, "k_tile_rows": 197.62e6, "k_tile_cols": 156.80e6,
 }
 
 # Wave64 VALU instructions per 4096x4096 micrograph at 1.0 A (rocprofv3 --pmc

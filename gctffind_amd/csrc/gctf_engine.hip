@@ -964,9 +964,9 @@ int launch_rescale(gctf_ctx* c, const RescalePlan& rp, const void* in, int dtype
 // Images per launch of the tile passes: as many as leave the row pass's
 // output (1 MB per tile of 512) in the 256 MB memory-side cache, where the
 // column pass reads it.  Per 4096^2 micrograph (144 tiles, 152 MB) the two
-// passes took 49.2 + 43.5 us four at a time and 54.4 + 34.3 us one at a time,
-// 41 x 3838x3710 5195 and 4735 us in all; with two at a time (304 MB) nothing
-// is gained any more.
+// passes took 47.1 + 44.2 us four at a time and 53.5 + 39.6 us one at a time
+// (32 spectra 7510 and 7465 us), 41 x 3838x3710 5110 and 4556 us in all; with
+// two at a time (304 MB) nothing is gained any more.
 constexpr size_t kTileRtBytes = 192u << 20;
 int tile_images(const TileGrid& g, int T, int n)
 {
@@ -1296,7 +1296,7 @@ int launch_2d(gctf_ctx* c, int T, int i0, int m, int begin, float phase_range)
 // (device, n entries, -1: none) of a batch with one search plan, the 1D search
 // done.  Launches for all of the batch, with the others leaving at once, cost
 // more than the search itself where few take part: a learned batch of 256
-// with 14 fallbacks took 17.1 ms and one with 59 25.1 ms, 8.3 and 11.3 so.
+// with 14 fallbacks took 17.1 ms and one with 59 25.1 ms, 8.4 and 11.5 so.
 int launch_2d_some(gctf_ctx* c, int T, const int* map, int n, float phase_range)
 {
 	Search2DView v = view_2d(c, T, 0);
